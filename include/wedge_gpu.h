@@ -102,9 +102,10 @@ int wg_sync(wg_ctx* ctx);
 #define WG_RELABEL_ON 1
 #define WG_RELABEL_AUTO 2
 #define WG_OPT_PR_BIN_SLICE 2  /* binned PageRank pull (WG_PR_BINNED): window-destination
-                                  sums one pull workgroup adds, 1..2^24 (default
-                                  262144); a bin with more is split over several
-                                  workgroups whose accumulators are then added.
+                                  sums one pull workgroup adds, 1..2^24 (unset: at
+                                  most 262144, fewer on smaller graphs); a bin with
+                                  more is split over several workgroups whose
+                                  accumulators are then added.
                                   Takes effect at the next layout build */
 #define WG_OPT_MS_BINNED 3     /* dense levels of the 64-source BFS (wg_msbfs) on the binned
                                   layout of WG_PR_BINNED (OR of frontier masks per

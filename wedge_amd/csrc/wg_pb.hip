@@ -48,7 +48,8 @@
 //   tile_pbase[t]  pairs before tile t (WG_PB_TILE entries per tile): pair p's
 //                  partial is part[p]
 //   task[k]        push work: {window, first tile, end tile, end of the real
-//                  entries (code index)}, at most WG_PB_TASK_TILES tiles
+//                  entries (code index)}, at most pb_task_tiles() tiles, the
+//                  longest first
 //   blocks         runs of pairs of one (window, bin), numbered in bin order
 //                  (window order within a bin); bin order position o of block
 //                  kb holds pair o - boff[kb] (32-bit wrap-around)
@@ -61,7 +62,7 @@
 //                  most that many blocks needs no dependent load for them
 //   slice[j]       pull work: {bin, first position, end position, accumulator
 //                  slot or WG_PB_NOSLOT when the slice is its bin's only one},
-//                  at most WG_PB_SLICE pairs, a contiguous range of positions
+//                  at most pb_slice_pairs() pairs, a contiguous range of positions
 //   bin_slot[b]    {first slot, slices} of a bin cut into several slices: each
 //                  slice writes its accumulators to its slot, and the last one
 //                  to finish (a per-bin ticket) adds the slots in slice order
@@ -77,13 +78,16 @@
 #define WG_PB_THREADS 1024                      // 16 wavefronts, one workgroup per CU
 #define WG_PB_WAVES (WG_PB_THREADS / WG_WAVE)
 #define WG_PB_TILE 512u                         // code entries per wavefront tile
-#define WG_PB_TASK_TILES 1024u                  // tiles per push workgroup (512K edges)
+#define WG_PB_TASK_TILES 1024u                  // tiles per push workgroup (512K edges), at most
+#define WG_PB_TASK_TILES_MIN 64u                // and at least (32K edges)
 #define WG_PB_STAGE 256u                        // partials a push wavefront stages in LDS
-#define WG_PB_SLICE (256u * 1024u)              // pairs per pull workgroup (default)
+#define WG_PB_SLICE (256u * 1024u)              // pairs per pull workgroup, at most (default)
+#define WG_PB_SLICE_MIN (32u * 1024u)           // and at least
 #define WG_PB_NOSLOT 0xffffffffu
 #define WG_PB_END 0x8000u                       // code: last edge of a pair
 #define WG_PB_SRC 0x3fffu                       // code: source - window start
 #define WG_PB_MAX_WS_LOG 14
+#define WG_PB_MIN_WD_LOG 12
 #define WG_PB_BFLAG 0x8000u                     // pdst: a block starts here
 #define WG_PB_DMASK 0x7fffu                     // pdst: destination - bin start
 #define WG_PB_CHUNK_OFFS 8u                     // block offsets kept with each 64-position chunk
@@ -320,6 +324,48 @@ static int pb_upload(wg_ctx* ctx, T** d, const std::vector<T>& h)
     return WG_OK;
 }
 
+// How a layout is cut into workgroups.  A push or pull workgroup fills a CU's
+// LDS (push) or its 16 wavefronts (pull), so a graph of a few million edges cut
+// into the large pieces that suit rmat-s27 leaves most of the 256 CUs idle.
+// MI355X, PageRank FP64 with 16K-vertex windows, us per iteration:
+//   push, tiles per task      32    64   128   256  1024
+//     rmat-s20 (16M edges)    37    31    30    45   120
+//     rmat-s21 (33M edges)    65    54    51    49   140
+//     rmat-s24 (260M edges)  533   408   342   313   292
+// Every task copies its window (128 KB) first, so a task should not be shorter
+// than what two per CU need.
+static uint64_t pb_task_tiles(const wg_ctx* ctx, uint64_t E)
+{
+    const uint64_t t = E / WG_PB_TILE / (2ull * (uint64_t)ctx->num_cu);
+    return std::min<uint64_t>(std::max<uint64_t>(t, WG_PB_TASK_TILES_MIN), WG_PB_TASK_TILES);
+}
+
+//   pull, vertices per bin           16K          8K          4K
+//     (pairs per slice)        256K  64K   256K  32K   256K  32K
+//     rmat-s20                  112   66     93   42     60   31
+//     rmat-s21                  120   89    107   66    100   39
+//     rmat-s24                  277  614    269  432    272  390
+// Bins of 16K vertices as long as they give four workgroups per CU, else
+// smaller ones (rmat-s23 with two: 179 us, with four: 131): a bin is one
+// workgroup, without the joins (LDS dumps and a ticket) that a bin cut into
+// slices takes.  512-thread workgroups were slower (rmat-s20 41 us): the
+// longest slice, not the number of them, bounds the pull.
+static int pb_bin_log(const wg_ctx* ctx, int wd_log)
+{
+    while (wd_log > WG_PB_MIN_WD_LOG && (ctx->V >> wd_log) < 4ull * (uint64_t)ctx->num_cu)
+        --wd_log;
+    return wd_log;
+}
+
+// A slice holds about what a CU has to add in all, within limits: hub bins are
+// the only ones cut, and the joins of many short slices cost more than the
+// parallelism gives (above, and 128K pairs at rmat-s27: 4.3 ms against 3.6).
+static uint32_t pb_slice_pairs(const wg_ctx* ctx, uint64_t npairs)
+{
+    const uint64_t p = npairs / (uint64_t)ctx->num_cu;
+    return (uint32_t)std::min<uint64_t>(std::max<uint64_t>(p, WG_PB_SLICE_MIN), WG_PB_SLICE);
+}
+
 static int pb_build(wg_ctx* ctx, wg_pb* pb, int ws_log, int wd_log)
 {
     const uint64_t V = ctx->V, E = ctx->E;
@@ -374,12 +420,13 @@ static int pb_build(wg_ctx* ctx, wg_pb* pb, int ws_log, int wd_log)
     std::vector<uint64_t> pq(S + 1, 0);
     std::vector<uint32_t> tile_win;
     std::vector<uint4> task;
+    const uint64_t task_tiles = pb_task_tiles(ctx, E);
     for (uint32_t s = 0; s < S; ++s) {
         const uint64_t cnt = ws[s + 1] - ws[s];
         const uint64_t tiles = (cnt + WG_PB_TILE - 1) / WG_PB_TILE;
         const uint32_t t0 = (uint32_t)(pq[s] / WG_PB_TILE);
-        for (uint64_t k = 0; k < tiles; k += WG_PB_TASK_TILES) {
-            const uint64_t k1 = std::min<uint64_t>(tiles, k + WG_PB_TASK_TILES);
+        for (uint64_t k = 0; k < tiles; k += task_tiles) {
+            const uint64_t k1 = std::min<uint64_t>(tiles, k + task_tiles);
             task.push_back(make_uint4(s, t0 + (uint32_t)k, t0 + (uint32_t)k1, 0u));
         }
         for (uint64_t k = 0; k < tiles; ++k)
@@ -389,6 +436,9 @@ static int pb_build(wg_ctx* ctx, wg_pb* pb, int ws_log, int wd_log)
     const uint64_t nq = pq[S];
     if (nq >= 0xffffffffull) // code indices are 32-bit
         return WG_E_RANGE;
+    // whole tasks first, the windows' remainders after them: the last round of
+    // workgroups is then made of short ones (rmat-s24 push 325 -> 292 us)
+    std::stable_sort(task.begin(), task.end(), [](const uint4& a, const uint4& b) { return a.z - a.y > b.z - b.y; });
     for (auto& tk : task) // end of the window's real entries, as a code index
         tk.w = (uint32_t)(pq[tk.x] + (ws[tk.x + 1] - ws[tk.x]));
     pb->nq = nq;
@@ -510,7 +560,7 @@ static int pb_build(wg_ctx* ctx, wg_pb* pb, int ws_log, int wd_log)
     const uint64_t nchunks = ((uint64_t)npairs + 63u) / 64u;
     std::vector<uint32_t> chunk_block(nchunks + 1 + nchunks * WG_PB_CHUNK_OFFS, (uint32_t)nb);
     std::vector<uint32_t> bin_out(B + 1, 0u); // first position of each bin in part[]
-    const uint32_t slice_max = ctx->pb_slice ? ctx->pb_slice : WG_PB_SLICE;
+    const uint32_t slice_max = ctx->pb_slice ? ctx->pb_slice : pb_slice_pairs(ctx, npairs);
     std::vector<uint4> slice;
     std::vector<uint2> bin_slot(B, make_uint2(0u, 0u));
     uint32_t nslots = 0;
@@ -575,7 +625,8 @@ static int pb_build(wg_ctx* ctx, wg_pb* pb, int ws_log, int wd_log)
 // Window and bin sizes of a binned shape: 16K-vertex windows (at most what the
 // 14-bit source field holds) and 16K-vertex bins, 128 KiB of FP64 accumulators,
 // for one 1024-thread workgroup per CU (blocks_per_cu 1); 8K-vertex windows
-// and bins, 64 KiB each, for two (blocks_per_cu 2).  FP32 windows of 16K
+// and bins, 64 KiB each, for two (blocks_per_cu 2).  Graphs with few bins take
+// smaller ones (pb_bin_log).  FP32 windows of 16K
 // vertices take 64 KiB.
 static void pb_sizes(int bpc, int* ws_log, int* wd_log)
 {
@@ -585,6 +636,7 @@ static void pb_sizes(int bpc, int* ws_log, int* wd_log)
 
 static int pb_prepare_sizes(wg_ctx* ctx, int ws_log, int wd_log)
 {
+    wd_log = pb_bin_log(ctx, wd_log);
     if (ctx->pb && ctx->pb->ws_log == ws_log && ctx->pb->wd_log == wd_log)
         return WG_OK;
     WG_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -1197,7 +1249,18 @@ __global__ __launch_bounds__(WG_PB_THREADS) void k_pb_total(const double* __rest
 
 // ---- host side --------------------------------------------------------------------
 
-template <typename T, int WS, int WD>
+// Calls K(WD) with the layout's bin size.
+#define PB_BY_BIN(pb, K)            \
+    do {                            \
+        if ((pb)->wd_log == 14)     \
+            K(16384);               \
+        else if ((pb)->wd_log == 13) \
+            K(8192);                \
+        else                        \
+            K(4096);                \
+    } while (0)
+
+template <typename T, int WS>
 static int pb_launch(wg_ctx* ctx, int mode, const T* cin, T* cout, double* S_in, double* S_out)
 {
     const wg_pb* pb = ctx->pb;
@@ -1213,16 +1276,21 @@ static int pb_launch(wg_ctx* ctx, int mode, const T* cin, T* cout, double* S_in,
         wg_prof_end(ctx, WG_K_PB_PUSH, slot);
     }
     const int slot = wg_prof_begin(ctx, WG_K_PB_PULL);
-    if (mode == 0)
-        hipLaunchKernelGGL((k_pb_pull<T, 0, WD>), dim3(pb->nslices), dim3(WG_PB_THREADS), 0, ctx->stream,
-                           (const T*)reinterpret_cast<T*>(pb->part),
-                           pb->pdst, pb->chunk_block, pb->boff, pb->nblocks, (uint32_t)pb->npairs, pb->slice, pb->nslices, pb->bin_slot, pb->slot_acc, pb->bin_ticket, pb->bin_part,
-                           cout, nullptr, ctx->od, V, S_in, ctx->damping, N);
-    else
-        hipLaunchKernelGGL((k_pb_pull<T, 1, WD>), dim3(pb->nslices), dim3(WG_PB_THREADS), 0, ctx->stream,
-                           (const T*)reinterpret_cast<T*>(pb->part),
-                           pb->pdst, pb->chunk_block, pb->boff, pb->nblocks, (uint32_t)pb->npairs, pb->slice, pb->nslices, pb->bin_slot, pb->slot_acc, pb->bin_ticket, pb->bin_part,
-                           nullptr, ctx->acc, ctx->od, V, S_in, ctx->damping, N);
+#define PB_PULL(WD)                                                                                                    \
+    do {                                                                                                               \
+        if (mode == 0)                                                                                                 \
+            hipLaunchKernelGGL((k_pb_pull<T, 0, WD>), dim3(pb->nslices), dim3(WG_PB_THREADS), 0, ctx->stream,          \
+                               (const T*)reinterpret_cast<T*>(pb->part), pb->pdst, pb->chunk_block, pb->boff,          \
+                               pb->nblocks, (uint32_t)pb->npairs, pb->slice, pb->nslices, pb->bin_slot, pb->slot_acc,  \
+                               pb->bin_ticket, pb->bin_part, cout, nullptr, ctx->od, V, S_in, ctx->damping, N);        \
+        else                                                                                                           \
+            hipLaunchKernelGGL((k_pb_pull<T, 1, WD>), dim3(pb->nslices), dim3(WG_PB_THREADS), 0, ctx->stream,          \
+                               (const T*)reinterpret_cast<T*>(pb->part), pb->pdst, pb->chunk_block, pb->boff,          \
+                               pb->nblocks, (uint32_t)pb->npairs, pb->slice, pb->nslices, pb->bin_slot, pb->slot_acc,  \
+                               pb->bin_ticket, pb->bin_part, nullptr, ctx->acc, ctx->od, V, S_in, ctx->damping, N);    \
+    } while (0)
+    PB_BY_BIN(pb, PB_PULL);
+#undef PB_PULL
     int rc = wg_check_launch(ctx);
     if (rc)
         return rc;
@@ -1240,10 +1308,10 @@ int wg_pb_iteration(wg_ctx* ctx, int mode, const void* cin, void* cout, double* 
         return rc;
     const bool big = ctx->pr_bpc == 1;
     if (ctx->pr_fp32)
-        return big ? pb_launch<float, 16384, 16384>(ctx, mode, (const float*)cin, (float*)cout, S_in, S_out)
-                   : pb_launch<float, 8192, 8192>(ctx, mode, (const float*)cin, (float*)cout, S_in, S_out);
-    return big ? pb_launch<double, 16384, 16384>(ctx, mode, (const double*)cin, (double*)cout, S_in, S_out)
-               : pb_launch<double, 8192, 8192>(ctx, mode, (const double*)cin, (double*)cout, S_in, S_out);
+        return big ? pb_launch<float, 16384>(ctx, mode, (const float*)cin, (float*)cout, S_in, S_out)
+                   : pb_launch<float, 8192>(ctx, mode, (const float*)cin, (float*)cout, S_in, S_out);
+    return big ? pb_launch<double, 16384>(ctx, mode, (const double*)cin, (double*)cout, S_in, S_out)
+               : pb_launch<double, 8192>(ctx, mode, (const double*)cin, (double*)cout, S_in, S_out);
 }
 
 int wg_pb_stats(const wg_ctx* ctx, uint64_t* pairs, uint64_t* code_entries, uint32_t* tasks, uint32_t* slices)
@@ -1381,18 +1449,22 @@ int wg_pb_msbfs_level(wg_ctx* ctx, const unsigned long long* front_in, unsigned 
                            front_in, live, pb->task, pb->ntasks, pb->tile_pbase, part, V);
     if ((rc = wg_check_launch(ctx)))
         return rc;
-    if (rows)
-        hipLaunchKernelGGL((k_pb_pull_or<16384, true>), dim3(pb->nslices), dim3(WG_PB_THREADS), 0, ctx->stream,
-                           (const unsigned long long*)part, pb->pdst, pb->chunk_block, pb->boff, pb->nblocks,
-                           (uint32_t)pb->npairs, pb->slice, pb->nslices, pb->bin_slot,
-                           reinterpret_cast<unsigned long long*>(pb->slot_acc), pb->bin_ticket, seen, front_out,
-                           depth, ctx->bm_next, ctx->od, live, level, ctx->ctr, V);
-    else
-        hipLaunchKernelGGL((k_pb_pull_or<16384, false>), dim3(pb->nslices), dim3(WG_PB_THREADS), 0, ctx->stream,
-                           (const unsigned long long*)part, pb->pdst, pb->chunk_block, pb->boff, pb->nblocks,
-                           (uint32_t)pb->npairs, pb->slice, pb->nslices, pb->bin_slot,
-                           reinterpret_cast<unsigned long long*>(pb->slot_acc), pb->bin_ticket, seen, front_out,
-                           depth, ctx->bm_next, ctx->od, live, level, ctx->ctr, V);
+#define PB_PULL_OR(WD, ROWS)                                                                                           \
+    hipLaunchKernelGGL((k_pb_pull_or<WD, ROWS>), dim3(pb->nslices), dim3(WG_PB_THREADS), 0, ctx->stream,               \
+                       (const unsigned long long*)part, pb->pdst, pb->chunk_block, pb->boff, pb->nblocks,              \
+                       (uint32_t)pb->npairs, pb->slice, pb->nslices, pb->bin_slot,                                     \
+                       reinterpret_cast<unsigned long long*>(pb->slot_acc), pb->bin_ticket, seen, front_out, depth,    \
+                       ctx->bm_next, ctx->od, live, level, ctx->ctr, V)
+#define PB_PULL_OR_BIN(WD)          \
+    do {                            \
+        if (rows)                   \
+            PB_PULL_OR(WD, true);   \
+        else                        \
+            PB_PULL_OR(WD, false);  \
+    } while (0)
+    PB_BY_BIN(pb, PB_PULL_OR_BIN);
+#undef PB_PULL_OR_BIN
+#undef PB_PULL_OR
     return wg_check_launch(ctx);
 }
 
@@ -1556,22 +1628,27 @@ static int pb_min_launch(wg_ctx* ctx, int gate)
     int rc = wg_check_launch(ctx);
     if (rc)
         return rc;
-    if (ctx->count_work)
-        hipLaunchKernelGGL((k_pb_pull_min<true, P, 16384>), dim3(lg), dim3(WG_PB_THREADS), 0, ctx->stream,
-                           (const T*)part, pb->pdst, pb->chunk_block, pb->boff, pb->nblocks, (uint32_t)pb->npairs,
-                           pb->slice, pb->nslices, pb->bin_slot, reinterpret_cast<T*>(pb->slot_acc), pb->bin_ticket,
-                           prop, ctx->od, ctx->bm_next, V, ctx->ctr, gate);
-    else
-        hipLaunchKernelGGL((k_pb_pull_min<false, P, 16384>), dim3(lg), dim3(WG_PB_THREADS), 0, ctx->stream,
-                           (const T*)part, pb->pdst, pb->chunk_block, pb->boff, pb->nblocks, (uint32_t)pb->npairs,
-                           pb->slice, pb->nslices, pb->bin_slot, reinterpret_cast<T*>(pb->slot_acc), pb->bin_ticket,
-                           prop, ctx->od, ctx->bm_next, V, ctx->ctr, gate);
+#define PB_PULL_MIN(WD, CW)                                                                                            \
+    hipLaunchKernelGGL((k_pb_pull_min<CW, P, WD>), dim3(lg), dim3(WG_PB_THREADS), 0, ctx->stream, (const T*)part,      \
+                       pb->pdst, pb->chunk_block, pb->boff, pb->nblocks, (uint32_t)pb->npairs, pb->slice, pb->nslices, \
+                       pb->bin_slot, reinterpret_cast<T*>(pb->slot_acc), pb->bin_ticket, prop, ctx->od, ctx->bm_next,  \
+                       V, ctx->ctr, gate)
+#define PB_PULL_MIN_BIN(WD)          \
+    do {                             \
+        if (ctx->count_work)         \
+            PB_PULL_MIN(WD, true);   \
+        else                         \
+            PB_PULL_MIN(WD, false);  \
+    } while (0)
+    PB_BY_BIN(pb, PB_PULL_MIN_BIN);
+#undef PB_PULL_MIN_BIN
+#undef PB_PULL_MIN
     return wg_check_launch(ctx);
 }
 
 int wg_pb_min_pull(wg_ctx* ctx, int gate)
 {
-    if (!ctx->pb || ctx->pb->ws_log != 14 || ctx->pb->wd_log != 14)
+    if (!ctx->pb || ctx->pb->ws_log != 14)
         return WG_E_STATE; // wg_pb_min_prepare first
     if (ctx->app == WG_APP_CC)
         return pb_min_launch<PolCC>(ctx, gate);

@@ -332,6 +332,10 @@ extern "C" int wg_pr_autotune(wg_ctx* ctx, uint32_t iterations, wg_batch_shape* 
     // the timed iterations advanced the state: start again from the uniform ranks
     if ((rc = wg_set_pr_shape(ctx, &best_s)) || (rc = wg_init_pr(ctx, damping, fp32)))
         return rc;
+    // the last candidate's layout may be another binned shape's: the first
+    // iteration after the tuning finds its own
+    if (best_s.xcd_split == WG_PR_BINNED && (rc = wg_pb_prepare(ctx)))
+        return rc;
     if (best)
         *best = best_s;
     return WG_OK;
