@@ -53,114 +53,195 @@ __global__ void k_ppr_seeds(const uint32_t* __restrict__ seeds, uint32_t nseeds,
     D[s] = o ? 0.0 : 1.0;
 }
 
-// One iteration over the edge tiles, one wavefront per tile.  Light tile: the
-// two half-waves take alternate destinations, lane s of a half summing seed
-// s.  Heavy tile (part of one destination): the halves take alternate edges,
-// the tile's sum goes to part[t][s].
+// A row of 32 contributions is 8 lanes' float4: lane l of a group of 8 holds
+// seeds 4l..4l+3, so one load instruction gathers 8 rows (one per group) and a
+// wavefront keeps 8 * PPR_FLIGHT rows in flight.  The gathers are bound by the
+// bytes in flight, not by the rate of the memory behind them: with half a
+// wavefront per row and 4 rows per half an iteration on rmat-s20 took 423 us.
+#define PPR_GROUPS 8
+#define PPR_FLIGHT 4
+typedef float ppr_f4 __attribute__((ext_vector_type(4)));
+
+struct ppr_sum {
+    double x[4];
+};
+
+__device__ __forceinline__ void ppr_add(ppr_sum& a, ppr_f4 r)
+{
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        a.x[j] += (double)r[j];
+}
+
+// In-edges p, p + step, ... < e into a, in that order: this lane's four seeds.
+__device__ __forceinline__ void ppr_gather(uint32_t p, uint32_t e, uint32_t step, const uint32_t* __restrict__ src,
+                                           const ppr_f4* __restrict__ C, uint32_t l, ppr_sum& a)
+{
+    for (; p + (PPR_FLIGHT - 1) * step < e; p += PPR_FLIGHT * step) {
+        uint32_t u[PPR_FLIGHT];
+        ppr_f4 r[PPR_FLIGHT];
+#pragma unroll
+        for (int k = 0; k < PPR_FLIGHT; ++k)
+            u[k] = src[p + k * step];
+#pragma unroll
+        for (int k = 0; k < PPR_FLIGHT; ++k)
+            r[k] = C[(uint64_t)u[k] * (PPR_LANES / 4) + l];
+#pragma unroll
+        for (int k = 0; k < PPR_FLIGHT; ++k)
+            ppr_add(a, r[k]);
+    }
+    // the last 0..PPR_FLIGHT-1 edges, their loads together
+    uint32_t u[PPR_FLIGHT - 1];
+    ppr_f4 r[PPR_FLIGHT - 1];
+#pragma unroll
+    for (int k = 0; k < PPR_FLIGHT - 1; ++k)
+        u[k] = p + k * step < e ? src[p + k * step] : 0u;
+#pragma unroll
+    for (int k = 0; k < PPR_FLIGHT - 1; ++k) {
+        r[k] = ppr_f4{0.0f, 0.0f, 0.0f, 0.0f};
+        if (p + k * step < e)
+            r[k] = C[(uint64_t)u[k] * (PPR_LANES / 4) + l];
+    }
+#pragma unroll
+    for (int k = 0; k < PPR_FLIGHT - 1; ++k)
+        if (p + k * step < e)
+            ppr_add(a, r[k]);
+}
+
+// Adds the groups' sums of one seed: every lane gets the total of its seeds.
+__device__ __forceinline__ void ppr_join(ppr_sum& a)
+{
+#pragma unroll
+    for (int o = PPR_GROUPS; o < WG_WAVE; o <<= 1)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            a.x[j] += __shfl_xor(a.x[j], o, WG_WAVE);
+}
+
+// The vertex phase of v for this lane's seeds.
+__device__ __forceinline__ void ppr_vertex(uint32_t v, uint32_t o, const ppr_sum& a, const uint32_t* seed,
+                                           const double* dang, double damping, uint32_t l, ppr_f4* __restrict__ Cn,
+                                           double* __restrict__ R, ppr_sum& dsum)
+{
+    ppr_f4 c;
+    double r[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        r[j] = ppr_rank(a.x[j], v == seed[j], dang[j], damping);
+        c[j] = o ? (float)(r[j] / (double)o) : 0.0f;
+        if (!o)
+            dsum.x[j] += r[j];
+    }
+    Cn[(uint64_t)v * (PPR_LANES / 4) + l] = c;
+    if (R) {
+        double2* row = reinterpret_cast<double2*>(R + (uint64_t)v * PPR_LANES + 4u * l);
+        row[0] = make_double2(r[0], r[1]);
+        row[1] = make_double2(r[2], r[3]);
+    }
+}
+
+// One iteration over the edge tiles, nsub wavefronts per tile.  Light tile: the
+// groups take the destinations in turn, each summing its in-edges in order.
+// Heavy tile (part of one destination): the groups of the first wavefront take
+// every eighth edge, the tile's sum goes to part[t][s].  More than one
+// wavefront per tile on graphs with few tiles: a group's destinations follow
+// each other, each with its own chain of loads (rmat-s12: 71 -> 47 us per
+// iteration).
 __global__ __launch_bounds__(WG_BLOCK) void k_ppr_tile(const uint32_t* __restrict__ off, const uint32_t* __restrict__ src,
                                                         const uint32_t* __restrict__ od, const uint32_t* __restrict__ tile_v,
                                                         const uint32_t* __restrict__ tile_e, uint32_t ntiles,
                                                         const uint32_t* __restrict__ seeds, uint32_t nseeds,
-                                                        const float* __restrict__ C, float* __restrict__ Cn,
+                                                        const ppr_f4* __restrict__ C, ppr_f4* __restrict__ Cn,
                                                         double* __restrict__ R, double* __restrict__ part,
                                                         const double* __restrict__ D, double* __restrict__ wpart,
-                                                        double damping)
+                                                        double damping, uint32_t nsub)
 {
     const int lane = wg_lane();
-    const uint32_t half = (uint32_t)lane >> 5, s = (uint32_t)lane & 31u;
-    const uint32_t seed = s < nseeds ? seeds[s] : 0xffffffffu;
-    const double dang = D[s];
+    const uint32_t grp = (uint32_t)lane / (PPR_LANES / 4), l = (uint32_t)lane % (PPR_LANES / 4);
+    uint32_t seed[4];
+    double dang[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        seed[j] = 4u * l + j < nseeds ? seeds[4u * l + j] : 0xffffffffu;
+        dang[j] = D[4u * l + j];
+    }
     const uint32_t wave = blockIdx.x * WG_WPB + threadIdx.x / WG_WAVE;
-    const uint32_t stride = gridDim.x * WG_WPB;
-    double dsum = 0.0; // mass of this lane's destinations without out-edges
-    for (uint32_t t = wave; t < ntiles; t += stride) {
+    const uint32_t stride = gridDim.x * WG_WPB / nsub; // the host launches a multiple of nsub wavefronts
+    const uint32_t sub = wave % nsub;
+    ppr_sum dsum = {}; // mass of this lane's destinations without out-edges
+    for (uint32_t t = wave / nsub; t < ntiles; t += stride) {
         const uint32_t tv = tile_v[t];
         const uint32_t e0 = tile_e[t], e1 = tile_e[t + 1];
         const uint32_t v0 = tv & ~WG_HEAVY_BIT;
         if (tv & WG_HEAVY_BIT) {
-            double a = 0.0;
-            uint32_t p = e0 + half;
-            for (; p + 6 < e1; p += 8) { // four edges in flight per half
-                const uint32_t u0 = src[p], u1 = src[p + 2], u2 = src[p + 4], u3 = src[p + 6];
-                const float x0 = C[(uint64_t)u0 * PPR_LANES + s], x1 = C[(uint64_t)u1 * PPR_LANES + s];
-                const float x2 = C[(uint64_t)u2 * PPR_LANES + s], x3 = C[(uint64_t)u3 * PPR_LANES + s];
-                a += (double)x0;
-                a += (double)x1;
-                a += (double)x2;
-                a += (double)x3;
-            }
-            for (; p < e1; p += 2)
-                a += (double)C[(uint64_t)src[p] * PPR_LANES + s];
-            const double lo = __shfl(a, (int)s), hi = __shfl(a, (int)s + 32);
-            if (lane < 32)
-                part[(uint64_t)t * PPR_LANES + s] = lo + hi;
+            if (sub)
+                continue;
+            ppr_sum a = {};
+            ppr_gather(e0 + grp, e1, PPR_GROUPS, src, C, l, a);
+            ppr_join(a);
+            if (grp == 0)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    part[(uint64_t)t * PPR_LANES + 4u * l + j] = a.x[j];
             continue;
         }
         const uint32_t nv = (tile_v[t + 1] & ~WG_HEAVY_BIT) - v0;
-        for (uint32_t i = half; i < nv; i += 2) {
+        for (uint32_t i = sub * PPR_GROUPS + grp; i < nv; i += nsub * PPR_GROUPS) {
             const uint32_t v = v0 + i;
-            const uint32_t b = off[v], e = off[v + 1];
-            double a = 0.0;
-            uint32_t p = b;
-            for (; p + 3 < e; p += 4) {
-                const uint32_t u0 = src[p], u1 = src[p + 1], u2 = src[p + 2], u3 = src[p + 3];
-                const float x0 = C[(uint64_t)u0 * PPR_LANES + s], x1 = C[(uint64_t)u1 * PPR_LANES + s];
-                const float x2 = C[(uint64_t)u2 * PPR_LANES + s], x3 = C[(uint64_t)u3 * PPR_LANES + s];
-                a += (double)x0;
-                a += (double)x1;
-                a += (double)x2;
-                a += (double)x3;
-            }
-            for (; p < e; ++p)
-                a += (double)C[(uint64_t)src[p] * PPR_LANES + s];
-            const double r = ppr_rank(a, v == seed, dang, damping);
+            ppr_sum a = {};
             const uint32_t o = od[v];
-            Cn[(uint64_t)v * PPR_LANES + s] = o ? (float)(r / (double)o) : 0.0f;
-            if (R)
-                R[(uint64_t)v * PPR_LANES + s] = r;
-            if (!o)
-                dsum += r;
+            ppr_gather(off[v], off[v + 1], 1u, src, C, l, a);
+            ppr_vertex(v, o, a, seed, dang, damping, l, Cn, R, dsum);
         }
     }
-    const double lo = __shfl(dsum, (int)s), hi = __shfl(dsum, (int)s + 32);
-    if (lane < 32)
-        wpart[(uint64_t)wave * PPR_LANES + s] = lo + hi;
+    ppr_join(dsum);
+    if (grp == 0)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            wpart[(uint64_t)wave * PPR_LANES + 4u * l + j] = dsum.x[j];
 }
 
-// Heavy destinations: the tile partials in tile order, then the rank.
+// Heavy destinations: the tile partials (every eighth one per group), then the
+// rank.
 __global__ __launch_bounds__(WG_BLOCK) void k_ppr_span(const uint32_t* __restrict__ off, const uint32_t* __restrict__ heavy_v,
                                                         const uint32_t* __restrict__ heavy_t, uint32_t nheavy,
                                                         const uint32_t* __restrict__ od, const uint32_t* __restrict__ seeds,
                                                         uint32_t nseeds, const double* __restrict__ part,
-                                                        float* __restrict__ Cn, double* __restrict__ R,
+                                                        ppr_f4* __restrict__ Cn, double* __restrict__ R,
                                                         const double* __restrict__ D, double* __restrict__ spart,
                                                         double damping)
 {
     const int lane = wg_lane();
-    const uint32_t s = (uint32_t)lane & 31u;
-    const uint32_t seed = s < nseeds ? seeds[s] : 0xffffffffu;
-    const double dang = D[s];
+    const uint32_t grp = (uint32_t)lane / (PPR_LANES / 4), l = (uint32_t)lane % (PPR_LANES / 4);
+    uint32_t seed[4];
+    double dang[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        seed[j] = 4u * l + j < nseeds ? seeds[4u * l + j] : 0xffffffffu;
+        dang[j] = D[4u * l + j];
+    }
     const uint32_t wave = blockIdx.x * WG_WPB + threadIdx.x / WG_WAVE;
     const uint32_t stride = gridDim.x * WG_WPB;
-    double dsum = 0.0;
+    ppr_sum dsum = {};
     for (uint32_t h = wave; h < nheavy; h += stride) {
         const uint32_t v = heavy_v[h], t0 = heavy_t[h];
         const uint32_t nch = (off[v + 1] - off[v] + WG_TILE_EDGES - 1) / WG_TILE_EDGES;
-        double a = 0.0;
-        for (uint32_t c = 0; c < nch; ++c)
-            a += part[(uint64_t)(t0 + c) * PPR_LANES + s];
-        const double r = ppr_rank(a, v == seed, dang, damping);
-        const uint32_t o = od[v];
-        if (lane < 32) {
-            Cn[(uint64_t)v * PPR_LANES + s] = o ? (float)(r / (double)o) : 0.0f;
-            if (R)
-                R[(uint64_t)v * PPR_LANES + s] = r;
+        ppr_sum a = {};
+#pragma unroll 4
+        for (uint32_t c = grp; c < nch; c += PPR_GROUPS) {
+            const double* row = part + (uint64_t)(t0 + c) * PPR_LANES + 4u * l;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                a.x[j] += row[j];
         }
-        if (!o)
-            dsum += r;
+        ppr_join(a);
+        if (grp == 0) // the other groups hold the same sums
+            ppr_vertex(v, od[v], a, seed, dang, damping, l, Cn, R, dsum);
     }
-    if (lane < 32)
-        spart[(uint64_t)wave * PPR_LANES + s] = dsum;
+    if (grp == 0)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            spart[(uint64_t)wave * PPR_LANES + 4u * l + j] = dsum.x[j];
 }
 
 // D_next[s] = the per-wave dangling partials in wave order.
@@ -168,8 +249,8 @@ __global__ __launch_bounds__(WG_BLOCK) void k_ppr_span(const uint32_t* __restric
 // span partials) summed per lane in a fixed order.  Block b takes the rows
 // [b n / B, (b + 1) n / B); its thread t sums lane t % 32 over the rows of
 // group t / 32 (every 8th row, four running sums), the 8 group sums are added
-// in group order, and the last block to finish adds the B block sums in block
-// order.
+// in group order, and the last block to finish adds the B block sums the same
+// way (B = PPR_RED_BLOCKS, the launch).
 #define PPR_RED_BLOCKS 64
 __global__ __launch_bounds__(256) void k_ppr_reduce(const double* __restrict__ p, uint32_t n, double* __restrict__ bpart,
                                                     unsigned int* __restrict__ ticket, double* __restrict__ Dn)
@@ -204,10 +285,16 @@ __global__ __launch_bounds__(256) void k_ppr_reduce(const double* __restrict__ p
     __syncthreads();
     if (s_last) {
         __threadfence();
+        double d = 0.0; // every 8th block's sum, then the 8 groups in order
+#pragma unroll
+        for (uint32_t k = 0; k < PPR_RED_BLOCKS / 8; ++k)
+            d += __builtin_nontemporal_load(&bpart[(uint64_t)(k * 8 + grp) * PPR_LANES + lane]);
+        s_grp[grp][lane] = d;
+        __syncthreads();
         if (threadIdx.x < PPR_LANES) {
-            double d = 0.0;
-            for (uint32_t b = 0; b < gridDim.x; ++b)
-                d += __builtin_nontemporal_load(&bpart[(uint64_t)b * PPR_LANES + lane]);
+            d = 0.0;
+            for (int g = 0; g < 8; ++g)
+                d += s_grp[g][lane];
             Dn[lane] = d;
         }
         if (threadIdx.x == 0)
@@ -236,7 +323,15 @@ extern "C" int wg_ppr(wg_ctx* ctx, const uint64_t* seeds, uint32_t nseeds, uint3
     WG_HIP(ctx, hipSetDevice(ctx->device));
     WG_HIP(ctx, hipStreamSynchronize(ctx->stream));
     const uint64_t V = ctx->V;
-    const uint32_t grid = ctx->pr_grid, sgrid = ctx->span_grid;
+    // wavefronts per tile: a power of two up to 8, while there are fewer
+    // wavefronts than the device holds (WG_WPB is a multiple of 4, so 8 per tile
+    // take an even number of workgroups)
+    uint32_t nsub = 1;
+    while (nsub < 8 && 2ull * nsub * ctx->ntiles <= 32ull * (uint64_t)ctx->num_cu)
+        nsub *= 2;
+    uint32_t grid = wg_grid(ctx, (uint64_t)ctx->ntiles * nsub, WG_WPB, 8);
+    grid += grid & 1u;
+    const uint32_t sgrid = ctx->span_grid;
     const uint32_t nw = grid * WG_WPB, ns = sgrid * WG_WPB;
     void *C0 = nullptr, *C1 = nullptr, *R = nullptr, *aux = nullptr;
     // aux: seeds (32 u32) | D[2][32] | tile partials [ntiles][32] | wave partials | span partials |
@@ -291,9 +386,10 @@ extern "C" int wg_ppr(wg_ctx* ctx, const uint64_t* seeds, uint32_t nseeds, uint3
         double* Dnxt = D + ((it + 1u) & 1u) * PPR_LANES;
         double* Rout = (it + 1 == iterations) ? (double*)R : nullptr;
         hipLaunchKernelGGL(k_ppr_tile, dim3(grid), dim3(WG_BLOCK), 0, ctx->stream, ctx->off, ctx->src, ctx->od, ctx->tile_v,
-                           ctx->tile_e, ctx->ntiles, dseeds, nseeds, cur, nxt, Rout, part, Dcur, wpart, damping);
+                           ctx->tile_e, ctx->ntiles, dseeds, nseeds, (const ppr_f4*)cur,
+                           (ppr_f4*)nxt, Rout, part, Dcur, wpart, damping, nsub);
         hipLaunchKernelGGL(k_ppr_span, dim3(sgrid), dim3(WG_BLOCK), 0, ctx->stream, ctx->off, ctx->heavy_v, ctx->heavy_t,
-                           ctx->nheavy, ctx->od, dseeds, nseeds, part, nxt, Rout, Dcur, spart, damping);
+                           ctx->nheavy, ctx->od, dseeds, nseeds, part, (ppr_f4*)nxt, Rout, Dcur, spart, damping);
         hipLaunchKernelGGL(k_ppr_reduce, dim3(PPR_RED_BLOCKS), dim3(256), 0, ctx->stream, wpart, nw + ns, rpart, ticket,
                            Dnxt);
         if ((rc = wg_check_launch(ctx)))
