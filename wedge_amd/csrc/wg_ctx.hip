@@ -361,31 +361,49 @@ int wg_to_device_ids(wg_ctx* ctx, const uint64_t* orig, uint32_t n, uint32_t* ou
     return WG_OK;
 }
 
+// Results are put into the caller's numbering in one device array that the
+// context keeps until its graph goes (an allocation and a release per read cost
+// as much as copying a megabyte).
+int wg_stage(wg_ctx* ctx, size_t bytes, void** out)
+{
+    if (ctx->stage_bytes < bytes) {
+        WG_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        if (ctx->stage)
+            (void)hipFree(ctx->stage);
+        ctx->stage = nullptr;
+        ctx->stage_bytes = 0;
+        WG_HIP(ctx, hipMalloc(&ctx->stage, bytes));
+        ctx->stage_bytes = bytes;
+    }
+    *out = ctx->stage;
+    return WG_OK;
+}
+
+int wg_copy_out(wg_ctx* ctx, const void* dev, void* host, size_t bytes)
+{
+    WG_HIP(ctx, hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, ctx->stream));
+    WG_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    return WG_OK;
+}
+
 int wg_read_vertex_array(wg_ctx* ctx, const void* dev, void* host, size_t esz)
 {
-    if (!ctx->inv) {
-        WG_HIP(ctx, hipMemcpyAsync(host, dev, ctx->V * esz, hipMemcpyDeviceToHost, ctx->stream));
-        WG_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        return WG_OK;
-    }
-    void* tmp = nullptr;
-    WG_HIP(ctx, hipMalloc(&tmp, ctx->V * esz));
+    if (!ctx->inv)
+        return wg_copy_out(ctx, dev, host, ctx->V * esz);
+    void* stage = nullptr;
+    int rc = wg_stage(ctx, ctx->V * esz, &stage);
+    if (rc)
+        return rc;
     const uint32_t grid = wg_grid(ctx, ctx->V, 1024, 8);
     if (esz == 8)
         hipLaunchKernelGGL(k_to_original<uint64_t>, dim3(grid), dim3(256), 0, ctx->stream, (const uint64_t*)dev, ctx->inv,
-                           ctx->V, (uint64_t*)tmp);
+                           ctx->V, (uint64_t*)stage);
     else
         hipLaunchKernelGGL(k_to_original<uint32_t>, dim3(grid), dim3(256), 0, ctx->stream, (const uint32_t*)dev, ctx->inv,
-                           ctx->V, (uint32_t*)tmp);
-    hipError_t e1 = hipGetLastError();
-    hipError_t e2 = hipMemcpyAsync(host, tmp, ctx->V * esz, hipMemcpyDeviceToHost, ctx->stream);
-    hipError_t e3 = hipStreamSynchronize(ctx->stream);
-    (void)hipFree(tmp);
-    if (e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess) {
-        ctx->last_hip_error = (int)(e1 != hipSuccess ? e1 : e2 != hipSuccess ? e2 : e3);
-        return WG_E_HIP;
-    }
-    return WG_OK;
+                           ctx->V, (uint32_t*)stage);
+    if ((rc = wg_check_launch(ctx)))
+        return rc;
+    return wg_copy_out(ctx, stage, host, ctx->V * esz);
 }
 
 // ---- context ----------------------------------------------------------------------
@@ -521,6 +539,8 @@ static void free_graph(wg_ctx* ctx)
     free_dev((void**)&ctx->csr_dst);
     free_dev((void**)&ctx->perm);
     free_dev((void**)&ctx->inv);
+    free_dev(&ctx->stage);
+    ctx->stage_bytes = 0;
     ctx->V = ctx->E = 0;
     ctx->ntiles = ctx->nheavy = ctx->nbfs_heavy = 0;
 }
@@ -676,39 +696,42 @@ void wg_tile_split_points(const std::vector<uint32_t>& te, uint64_t E, uint32_t 
                                          te.begin());
 }
 
-// Tilings with 4, 16 and 2 edges per lane for the PageRank shapes, from the
-// device offsets (in device order).
-int wg_build_pr_tilings(wg_ctx* ctx)
+// Tiling number i (WG_ALT_IPT4 / 16 / 2: 4, 16 or 2 edges per lane) for the
+// PageRank shapes, the dense SSSP pulls and the 64-source SSSP, from the device
+// offsets (in device order); built on first use.
+int wg_build_pr_tiling(wg_ctx* ctx, int i)
 {
-    if (ctx->pr_alt_built)
+    if ((ctx->pr_alt_built >> i) & 1)
         return WG_OK;
+    static const uint32_t ipts[3] = {4, 16, 2};
     std::vector<uint32_t> hoff(ctx->V + 1);
     WG_HIP(ctx, hipMemcpy(hoff.data(), ctx->off, (ctx->V + 1) * sizeof(uint32_t), hipMemcpyDeviceToHost));
-    uint32_t max_tiles = ctx->ntiles;
-    const uint32_t ipts[3] = {4, 16, 2};
-    for (int i = 0; i < 3; ++i) {
-        std::vector<uint32_t> tv, te, hv, ht;
-        wg_build_tiles(hoff.data(), ctx->V, WG_WAVE * ipts[i], tv, te, hv, ht);
-        wg_tiling& t = ctx->pr_alt[i];
-        t.ntiles = (uint32_t)(tv.size() - 1);
-        t.nheavy = (uint32_t)hv.size();
-        wg_tile_split_points(te, ctx->E, t.split);
-        max_tiles = std::max(max_tiles, t.ntiles);
-        int rc;
-        if ((rc = upload(ctx, &t.tile_v, tv.data(), tv.size())) || (rc = upload(ctx, &t.tile_e, te.data(), te.size())) ||
-            (rc = upload(ctx, &t.heavy_v, hv.data(), hv.size())) || (rc = upload(ctx, &t.heavy_t, ht.data(), ht.size())))
+    std::vector<uint32_t> tv, te, hv, ht;
+    wg_build_tiles(hoff.data(), ctx->V, WG_WAVE * ipts[i], tv, te, hv, ht);
+    wg_tiling& t = ctx->pr_alt[i];
+    t.ntiles = (uint32_t)(tv.size() - 1);
+    t.nheavy = (uint32_t)hv.size();
+    wg_tile_split_points(te, ctx->E, t.split);
+    free_dev((void**)&t.tile_v); // left by a build that ran out of memory
+    free_dev((void**)&t.tile_e);
+    free_dev((void**)&t.heavy_v);
+    free_dev((void**)&t.heavy_t);
+    int rc;
+    if ((rc = upload(ctx, &t.tile_v, tv.data(), tv.size())) || (rc = upload(ctx, &t.tile_e, te.data(), te.size())) ||
+        (rc = upload(ctx, &t.heavy_v, hv.data(), hv.size())) || (rc = upload(ctx, &t.heavy_t, ht.data(), ht.size())))
+        return rc;
+    if (t.ntiles > ctx->tile_part_tiles) { // heavy-tile partials for the finest tiling built
+        double* part = nullptr;
+        if ((rc = upload<double>(ctx, &part, nullptr, (uint64_t)t.ntiles + 1)))
             return rc;
-    }
-    if (max_tiles > ctx->ntiles) { // heavy-tile partials for the finest tiling
+        WG_HIP(ctx, hipStreamSynchronize(ctx->stream));
         free_dev((void**)&ctx->tile_part);
-        int rc = upload<double>(ctx, &ctx->tile_part, nullptr, (uint64_t)max_tiles + 1);
-        if (rc)
-            return rc;
+        ctx->tile_part = part;
+        ctx->tile_part_tiles = t.ntiles;
     }
-    ctx->pr_alt_built = 1;
+    ctx->pr_alt_built |= 1 << i;
     return WG_OK;
 }
-
 
 // Relabelling pays off when a few vertices hold many edges (their values are
 // gathered over and over and end up in one place); on near-regular graphs such
@@ -960,6 +983,7 @@ extern "C" int wg_load_csc(wg_ctx* ctx, uint64_t V, uint64_t E, const uint32_t* 
     wg_tile_split_points(te, E, ctx->pr_split8);
     ctx->heavy_cap = (uint32_t)(E / 32 + E / 4096 + 16); // bound on deferred out-edge chunks per build
     ctx->span_grid = wg_grid(ctx, ctx->nheavy, 4, 4);
+    ctx->tile_part_tiles = ctx->ntiles;
     if ((rc = upload<uint64_t>(ctx, &ctx->bm_cur, nullptr, ctx->bm_words)) ||
         (rc = upload<uint64_t>(ctx, &ctx->bm_next, nullptr, ctx->bm_words)) ||
         (rc = upload<uint64_t>(ctx, &ctx->bm_visited, nullptr, ctx->bm_words)) ||

@@ -199,20 +199,23 @@ struct wg_ctx {
     size_t ms_aux_bytes;      // personalised PageRank: size of ms[2] (its reduction partials)
     void* idmap;              // wg_to_device_ids: original ids in, device ids out (grown as needed)
     size_t idmap_bytes;
+    void* stage;              // wg_stage: results in the caller's numbering, on their way to the host
+    size_t stage_bytes;
     int pr_cur;               // PR: index of the current contribution buffer
     int pr_parity;            // PR: index of S[] holding the current iteration's sum
     int pr_fp32;
     double damping;
     double* acc;              // PR accumulators (stand-alone edge phase)
     double* tile_part;        // PR: per-tile partial sums of heavy destinations
+    uint32_t tile_part_tiles; // tiles tile_part has room for
     double* blk_part;         // PR: per-block partial sums for S
     uint32_t pr_grid;         // blocks of the tile kernel
     uint32_t span_grid;       // blocks of the span kernel
     // PageRank tile shape (wg_set_pr_shape / wg_pr_autotune): edges per lane
     // 4, 8 (the tiles above) or 16, workgroups per CU, XCD split
     int pr_ipt, pr_bpc, pr_xcd;
-    wg_tiling pr_alt[3];      // tilings with 4, 16 and 2 edges per lane (built on first use)
-    int pr_alt_built;
+    wg_tiling pr_alt[3];      // tilings with 4, 16 and 2 edges per lane (each built on first use)
+    int pr_alt_built;         // bit i: pr_alt[i] is built
     uint32_t pr_split8[9];    // XCD split of the default tiles
     struct wg_pb* pb;         // layout of the binned PageRank pull (wg_pb.hip), built on first use
     uint32_t pb_slice;        // option: pairs per pull workgroup of that layout (0 = default)
@@ -354,6 +357,10 @@ int wg_to_device_id(wg_ctx* ctx, uint64_t orig, uint32_t* out);
 int wg_to_device_ids(wg_ctx* ctx, const uint64_t* orig, uint32_t n, uint32_t* out);
 // copies V values stored in device order to host memory in original order
 int wg_read_vertex_array(wg_ctx* ctx, const void* dev, void* host, size_t elem_size);
+// a kept device array of at least `bytes` for results on their way to the host
+int wg_stage(wg_ctx* ctx, size_t bytes, void** out);
+// device to host, waited for
+int wg_copy_out(wg_ctx* ctx, const void* dev, void* host, size_t bytes);
 // edge tiles of at most tile_edges edges (and WG_TILE_VERTS destinations)
 void wg_build_tiles(const uint32_t* off, uint64_t V, uint32_t tile_edges, std::vector<uint32_t>& tv,
                     std::vector<uint32_t>& te, std::vector<uint32_t>& hv, std::vector<uint32_t>& ht);
@@ -363,8 +370,11 @@ void wg_free_members(wg_ctx* ctx);
 void wg_drop_graph(wg_ctx* ctx);
 // XCD split points of a tiling (first tile at or after x/8 of the edges)
 void wg_tile_split_points(const std::vector<uint32_t>& te, uint64_t E, uint32_t start[9]);
-// builds the 4- and 16-edges-per-lane PageRank tilings once per graph
-int wg_build_pr_tilings(wg_ctx* ctx);
+// builds tiling pr_alt[i] (4, 16 or 2 edges per lane) once per graph
+#define WG_ALT_IPT4 0
+#define WG_ALT_IPT16 1
+#define WG_ALT_IPT2 2
+int wg_build_pr_tiling(wg_ctx* ctx, int i);
 // binned PageRank pull (wg_pb.hip): one iteration (mode 0 fused, 1 edge phase
 // only), building the layout for the current precision and shape first if needed
 int wg_pb_iteration(wg_ctx* ctx, int mode, const void* cin, void* cout, double* S_in, double* S_out);

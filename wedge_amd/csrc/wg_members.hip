@@ -203,14 +203,15 @@ template <typename T>
 __global__ __launch_bounds__(WG_BLOCK) void k_bm_ranks(const uint32_t* __restrict__ od, const T* __restrict__ c,
                                                        double* __restrict__ r, const uint32_t* __restrict__ chunk_v,
                                                        const uint32_t* __restrict__ chunk_m,
-                                                       const uint32_t* __restrict__ first, uint32_t nchunks)
+                                                       const uint32_t* __restrict__ first, uint32_t nchunks,
+                                                       const uint32_t* __restrict__ perm)
 {
     for (uint32_t ch = blockIdx.x; ch < nchunks; ch += gridDim.x) {
         const uint32_t g = chunk_m[ch];
         const double N = (double)(first[g + 1] - first[g]);
         for (uint32_t v = chunk_v[ch] + threadIdx.x; v < chunk_v[ch + 1]; v += WG_BLOCK) {
             const uint32_t o = od[v];
-            r[v] = (double)c[v] * (o ? (double)o : N);
+            r[perm ? perm[v] : v] = (double)c[v] * (o ? (double)o : N);
         }
     }
 }
@@ -567,18 +568,20 @@ extern "C" int wg_read_batch_ranks(wg_ctx* ctx, double* host_ranks)
     if (!m || m->cur < 0)
         return WG_E_STATE;
     WG_HIP(ctx, hipSetDevice(ctx->device));
-    double* r = nullptr;
-    WG_HIP(ctx, hipMalloc((void**)&r, (ctx->V ? ctx->V : 1) * sizeof(double)));
+    void* r = nullptr;
+    int rc = wg_stage(ctx, ctx->V * sizeof(double), &r);
+    if (rc)
+        return rc;
     const uint32_t cgrid = wg_grid(ctx, m->nchunks, 1, 16);
     if (m->c_fp32)
         hipLaunchKernelGGL(k_bm_ranks<float>, dim3(cgrid), dim3(WG_BLOCK), 0, ctx->stream, ctx->od,
-                           (const float*)m->c[m->cur], r, m->chunk_v, m->chunk_m, m->d_first, m->nchunks);
+                           (const float*)m->c[m->cur], (double*)r, m->chunk_v, m->chunk_m, m->d_first, m->nchunks,
+                           ctx->perm);
     else
         hipLaunchKernelGGL(k_bm_ranks<double>, dim3(cgrid), dim3(WG_BLOCK), 0, ctx->stream, ctx->od,
-                           (const double*)m->c[m->cur], r, m->chunk_v, m->chunk_m, m->d_first, m->nchunks);
-    int rc = wg_check_launch(ctx);
-    if (rc == WG_OK)
-        rc = wg_read_vertex_array(ctx, r, host_ranks, sizeof(double));
-    (void)hipFree(r);
-    return rc;
+                           (const double*)m->c[m->cur], (double*)r, m->chunk_v, m->chunk_m, m->d_first, m->nchunks,
+                           ctx->perm);
+    if ((rc = wg_check_launch(ctx)))
+        return rc;
+    return wg_copy_out(ctx, r, host_ranks, ctx->V * sizeof(double));
 }

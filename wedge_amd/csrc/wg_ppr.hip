@@ -302,10 +302,12 @@ __global__ __launch_bounds__(256) void k_ppr_reduce(const double* __restrict__ p
     }
 }
 
-__global__ void k_ppr_column(const double* __restrict__ R, uint32_t s, uint64_t V, double* __restrict__ out)
+// Column s of R, in the caller's numbering.
+__global__ void k_ppr_column(const double* __restrict__ R, uint32_t s, const uint32_t* __restrict__ inv, uint64_t V,
+                             double* __restrict__ out)
 {
     for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < V; v += (uint64_t)gridDim.x * blockDim.x)
-        out[v] = R[v * PPR_LANES + s];
+        out[v] = R[(uint64_t)(inv ? inv[v] : v) * PPR_LANES + s];
 }
 
 extern "C" int wg_ppr(wg_ctx* ctx, const uint64_t* seeds, uint32_t nseeds, uint32_t iterations, double damping)
@@ -410,13 +412,13 @@ extern "C" int wg_read_ppr(wg_ctx* ctx, uint32_t seed, double* host_ranks)
         return WG_E_STATE;
     if (seed >= ctx->ms_n)
         return WG_E_RANGE;
-    double* tmp = nullptr;
-    WG_HIP(ctx, hipMalloc((void**)&tmp, ctx->V * sizeof(double)));
+    void* stage = nullptr;
+    int rc = wg_stage(ctx, ctx->V * sizeof(double), &stage);
+    if (rc)
+        return rc;
     hipLaunchKernelGGL(k_ppr_column, dim3(wg_grid(ctx, ctx->V, 1024, 8)), dim3(256), 0, ctx->stream,
-                       (const double*)ctx->prop[0], seed, ctx->V, tmp);
-    int rc = wg_check_launch(ctx);
-    if (!rc)
-        rc = wg_read_vertex_array(ctx, tmp, host_ranks, sizeof(double));
-    (void)hipFree(tmp);
-    return rc;
+                       (const double*)ctx->prop[0], seed, ctx->inv, ctx->V, (double*)stage);
+    if ((rc = wg_check_launch(ctx)))
+        return rc;
+    return wg_copy_out(ctx, stage, host_ranks, ctx->V * sizeof(double));
 }

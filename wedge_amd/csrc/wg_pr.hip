@@ -77,13 +77,15 @@ __global__ void k_pr_init(const uint32_t* __restrict__ od, T* __restrict__ c, ui
     }
 }
 
+// Ranks in the caller's numbering.
 template <typename T>
-__global__ void k_pr_ranks(const uint32_t* __restrict__ od, const T* __restrict__ c, double* __restrict__ r, uint64_t V,
-                           double N)
+__global__ void k_pr_ranks(const uint32_t* __restrict__ od, const uint32_t* __restrict__ inv, const T* __restrict__ c,
+                           double* __restrict__ r, uint64_t V, double N)
 {
-    for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < V; v += (uint64_t)gridDim.x * blockDim.x) {
+    for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < V; i += (uint64_t)gridDim.x * blockDim.x) {
+        const uint64_t v = inv ? inv[i] : i;
         const uint32_t o = od[v];
-        r[v] = (double)c[v] * (o ? (double)o : N);
+        r[i] = (double)c[v] * (o ? (double)o : N);
     }
 }
 
@@ -243,7 +245,7 @@ extern "C" int wg_set_pr_shape(wg_ctx* ctx, const wg_batch_shape* shape)
     if (ipt != WG_IPT) {
         WG_HIP(ctx, hipSetDevice(ctx->device));
         WG_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        int rc = wg_build_pr_tilings(ctx);
+        int rc = wg_build_pr_tiling(ctx, ipt == 4 ? WG_ALT_IPT4 : ipt == 16 ? WG_ALT_IPT16 : WG_ALT_IPT2);
         if (rc)
             return rc;
     }
@@ -417,19 +419,19 @@ extern "C" int wg_read_ranks(wg_ctx* ctx, double* host_ranks)
 {
     if (!ctx || ctx->app != WG_APP_PR || !host_ranks)
         return WG_E_STATE;
-    double* tmp = nullptr;
-    WG_HIP(ctx, hipMalloc((void**)&tmp, ctx->V * sizeof(double)));
+    void* stage = nullptr;
+    int rc = wg_stage(ctx, ctx->V * sizeof(double), &stage);
+    if (rc)
+        return rc;
     const double N = (double)ctx->V;
     const uint32_t grid = wg_grid(ctx, ctx->V, 1024, 8);
     if (ctx->pr_fp32)
-        hipLaunchKernelGGL(k_pr_ranks<float>, dim3(grid), dim3(256), 0, ctx->stream, ctx->od,
-                           (const float*)ctx->prop[ctx->pr_cur], tmp, ctx->V, N);
+        hipLaunchKernelGGL(k_pr_ranks<float>, dim3(grid), dim3(256), 0, ctx->stream, ctx->od, ctx->inv,
+                           (const float*)ctx->prop[ctx->pr_cur], (double*)stage, ctx->V, N);
     else
-        hipLaunchKernelGGL(k_pr_ranks<double>, dim3(grid), dim3(256), 0, ctx->stream, ctx->od,
-                           (const double*)ctx->prop[ctx->pr_cur], tmp, ctx->V, N);
-    int rc = wg_check_launch(ctx);
-    if (rc == WG_OK)
-        rc = wg_read_vertex_array(ctx, tmp, host_ranks, sizeof(double));
-    (void)hipFree(tmp);
-    return rc;
+        hipLaunchKernelGGL(k_pr_ranks<double>, dim3(grid), dim3(256), 0, ctx->stream, ctx->od, ctx->inv,
+                           (const double*)ctx->prop[ctx->pr_cur], (double*)stage, ctx->V, N);
+    if ((rc = wg_check_launch(ctx)))
+        return rc;
+    return wg_copy_out(ctx, stage, host_ranks, ctx->V * sizeof(double));
 }

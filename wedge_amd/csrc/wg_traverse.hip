@@ -1753,8 +1753,9 @@ static int init_common(wg_ctx* ctx, int app)
     ctx->app = app;
     ctx->iter = 0;
     ctx->roots_frontier = 0;
-    // the 256-edge tiles of the dense SSSP pulls (built once per graph)
-    if (app == WG_APP_SSSP && (rc = wg_build_pr_tilings(ctx)))
+    // the 256-edge tiles of the dense SSSP pulls, unless those run on the
+    // binned layout (built once per graph)
+    if (app == WG_APP_SSSP && !wg_pb_min_on(ctx) && (rc = wg_build_pr_tiling(ctx, WG_ALT_IPT4)))
         return rc;
     // the smallest in-neighbours the dense BFS levels test first (once per graph)
     if (app == WG_APP_BFS && !ctx->first_src) {
@@ -2083,8 +2084,8 @@ struct min_tiling {
 template <class P>
 static min_tiling dense_min_tiling(const wg_ctx* ctx)
 {
-    if (P::DENSE_IPT == 4 && ctx->pr_alt_built) {
-        const wg_tiling& t = ctx->pr_alt[0];
+    if (P::DENSE_IPT == 4 && ((ctx->pr_alt_built >> WG_ALT_IPT4) & 1)) {
+        const wg_tiling& t = ctx->pr_alt[WG_ALT_IPT4];
         return min_tiling{t.tile_v, t.tile_e, t.ntiles, 4};
     }
     return min_tiling{ctx->tile_v, ctx->tile_e, ctx->ntiles, WG_IPT};
