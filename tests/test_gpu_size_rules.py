@@ -1,0 +1,100 @@
+"""The branches that a graph's size selects, each at a size that takes it:
+pull bins of 4K, 8K and 16K vertices of the binned layout, the 128- and
+512-edge tiles of the 64-source SSSP with and without marked destinations
+(hub lists cut into chunks), and one to eight wavefronts per tile of the
+personalised PageRank.  Against the oracle: exact for BFS, CC and SSSP, 1e-10
+L1 for FP64 PageRank (sums of FP64 values in another order), 2e-7 L1 for
+FP32-stored contributions (one rounding of 6e-8 per contribution)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle
+import wedge_amd as W
+
+pytestmark = pytest.mark.gpu
+
+
+def _sparse(V, n, seed, symmetric=False, weights=None):
+    """n random edges over V vertices, some into and out of a hub, some among
+    the last vertices (the last window and bin)."""
+    rng = np.random.default_rng(seed)
+    src = np.concatenate([rng.integers(0, V, n), rng.integers(0, V, 3000), np.full(3000, 7),
+                          rng.integers(V - 50, V, 300)])
+    dst = np.concatenate([rng.integers(0, V, n), np.full(3000, 7), rng.integers(0, V, 3000),
+                          rng.integers(V - 50, V, 300)])
+    if symmetric:
+        src, dst = np.concatenate([src, dst]), np.concatenate([dst, src])
+    w = None
+    if weights == "f64":
+        w = rng.random(src.size) + 1e-3
+    elif weights == "int":
+        w = rng.integers(1, 1000, src.size).astype(np.uint32)
+    return W.from_edges(V, src, dst, w, dedup=True)
+
+
+# 1024 bins of 4K, 8K and 16K vertices are the smallest counts that select them
+@pytest.mark.parametrize("V", [(1 << 22) - 1, 1 << 23, (1 << 24) + 5])
+def test_binned_bin_sizes(V):
+    g = _sparse(V, 40000, 3)
+    gs = _sparse(V, 20000, 4, symmetric=True)
+    c = W.Context(0, relabel=False)
+    try:
+        c.load(g)
+        ref, _ = oracle.Oracle.of(g, 8).pr(4, 0.85)
+        for fp32 in (False, True):
+            c.set_pr_shape((8, 1, W.PR_BINNED))
+            ranks, _ = c.run_pr(iterations=4, damping=0.85, contrib_fp32=int(fp32))
+            assert float(np.abs(ranks - ref).sum()) <= (2e-7 if fp32 else 1e-10), fp32
+        c.set_option(W.OPT_MS_BINNED, 1)
+        roots = np.array([7, V - 3, 7], np.uint64)
+        c.msbfs(roots, schedule="dense")
+        for i, r in enumerate(roots):
+            assert np.array_equal(c.read_msbfs(i), oracle.Oracle.of(g, 8).bfs(int(r))[1]), i
+        c.set_option(W.OPT_MIN_BINNED, 1)
+        c.load(gs)
+        labels, _ = c.run_cc(schedule="dense")
+        assert np.array_equal(labels.astype(np.float64), oracle.Oracle.of(gs, 8).cc()[0])
+    finally:
+        c.close()
+
+
+@pytest.mark.parametrize("weights", ["f64", "int"])
+@pytest.mark.parametrize("relabel", [False, True])
+def test_mssssp_hub_lists(weights, relabel):
+    """A hub with 3000 out-edges (three chunks of the marking) and 3000 in-edges
+    (several heavy tiles), every schedule."""
+    g = _sparse(5003, 30000, 5, weights=weights)
+    orc = oracle.Oracle.of(g, 8)
+    roots = np.concatenate([[7, 5002], np.arange(11)]).astype(np.uint64)
+    want = [orc.sssp(int(r))[0] for r in roots]
+    c = W.Context(0, relabel=relabel)
+    try:
+        c.load(g)
+        for schedule in ("plain", "dense", "frontier"):
+            c.mssssp(roots, schedule=schedule)
+            for i in range(len(roots)):
+                got = c.read_mssssp(i)
+                if weights == "int":  # the oracle's unreached is UINT64_MAX
+                    got = np.where(got == np.uint32(0xFFFFFFFF), np.uint64(2**64 - 1), got.astype(np.uint64))
+                assert np.array_equal(got, want[i]), (schedule, i)
+    finally:
+        c.close()
+
+
+# tiles of at most 256 destinations: 4, 79, 1563 and 7813 of them give 8, 8, 4
+# and 1 wavefronts per tile on 256 CUs
+@pytest.mark.parametrize("V", [1000, 20000, 400001, 2000000])
+def test_ppr_wavefronts_per_tile(V):
+    g = _sparse(V, 2 * V, 6)
+    seeds = np.array([7, V - 2, 0, 3], np.uint64)
+    want = oracle.Oracle.of(g, 8).ppr(seeds, 5, 0.85)
+    c = W.Context(0)
+    try:
+        c.load(g)
+        c.ppr(seeds, 5, 0.85)
+        for i in range(len(seeds)):
+            assert float(np.abs(c.read_ppr(i) - want[i]).sum()) <= 2e-7, i
+    finally:
+        c.close()

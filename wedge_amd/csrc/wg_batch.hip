@@ -350,10 +350,12 @@ __global__ void k_ms_reached(const unsigned long long* __restrict__ seen, const 
 }
 
 __global__ void k_ms_column(const uint16_t* __restrict__ depth, const unsigned long long* __restrict__ seen, uint32_t s,
-                            uint32_t V, uint32_t* __restrict__ out)
+                            const uint32_t* __restrict__ inv, uint32_t V, uint32_t* __restrict__ out)
 {
-    for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < V; v += (uint64_t)gridDim.x * blockDim.x)
-        out[v] = ((seen[v] >> s) & 1ull) ? (uint32_t)depth[v * WG_MS_MAX_SOURCES + s] : 0xffffffffu;
+    for (uint64_t o = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; o < V; o += (uint64_t)gridDim.x * blockDim.x) {
+        const uint64_t v = inv ? inv[o] : o;
+        out[o] = ((seen[v] >> s) & 1ull) ? (uint32_t)depth[v * WG_MS_MAX_SOURCES + s] : 0xffffffffu;
+    }
 }
 
 // ---- host side ----------------------------------------------------------------------
@@ -531,16 +533,16 @@ extern "C" int wg_read_msbfs(wg_ctx* ctx, uint32_t source, uint32_t* host_depths
         return WG_E_STATE;
     if (source >= ctx->ms_n)
         return WG_E_RANGE;
-    uint32_t* tmp = nullptr;
-    WG_HIP(ctx, hipMalloc((void**)&tmp, ctx->V * sizeof(uint32_t)));
+    void* stage = nullptr;
+    int rc = wg_stage(ctx, ctx->V * sizeof(uint32_t), &stage);
+    if (rc)
+        return rc;
     hipLaunchKernelGGL(k_ms_column, dim3(wg_grid(ctx, ctx->V, 1024, 8)), dim3(256), 0, ctx->stream,
-                       (const uint16_t*)ctx->prop[0], (const unsigned long long*)ctx->ms[0], source, (uint32_t)ctx->V,
-                       tmp);
-    int rc = wg_check_launch(ctx);
-    if (!rc)
-        rc = wg_read_vertex_array(ctx, tmp, host_depths, sizeof(uint32_t));
-    (void)hipFree(tmp);
-    return rc;
+                       (const uint16_t*)ctx->prop[0], (const unsigned long long*)ctx->ms[0], source, ctx->inv,
+                       (uint32_t)ctx->V, (uint32_t*)stage);
+    if ((rc = wg_check_launch(ctx)))
+        return rc;
+    return wg_copy_out(ctx, stage, host_depths, ctx->V * sizeof(uint32_t));
 }
 
 // ---- SSSP from up to 64 sources ---------------------------------------------------------
@@ -548,28 +550,29 @@ extern "C" int wg_read_msbfs(wg_ctx* ctx, uint32_t source, uint32_t* host_depths
 //   dist[v][64]  distance from source s (lane s): FP64 bit patterns (non-negative
 //                doubles order like their bits) or uint32, INF if unreached
 //   chg[v]       sources whose distance to v improved in the last iteration
-// An iteration relaxes destinations, one wavefront per destination, lane s
-// taking min over in-edges u->v of dist[u][s] + w; the row of u is read only
-// when some source improved u.  Dense iterations relax every destination;
-// sparse ones first mark the out-neighbours of the improved vertices and
-// relax only those.  Minimum is order-independent, so the result is each
+// An iteration relaxes the edges whose source improved in the last one: their
+// destinations take min over dist[u][s] + w, lane s for source s, and the row
+// of u is read only for the sources that improved u.  With few improved
+// vertices their out-neighbours are marked first, and tiles without a marked
+// destination are skipped.  Minimum is order-independent, so the result is each
 // source's single-source SSSP fixpoint (source/phase_edge_pull_sssp.c:57-169).
 
 struct MsF64 {
     typedef unsigned long long T;
     static constexpr unsigned long long INF = 0x7FF0000000000000ull;
-    __device__ static T add(T d, const void* __restrict__ w, uint32_t p, unsigned int* __restrict__)
+    // distance d over an edge of weight w (its bits)
+    __device__ static T add(T d, T w, unsigned int* __restrict__)
     {
-        return (T)__double_as_longlong(__longlong_as_double((long long)d) + ((const double*)w)[p]);
+        return (T)__double_as_longlong(__longlong_as_double((long long)d) + __longlong_as_double((long long)w));
     }
 };
 
 struct MsU32 {
     typedef uint32_t T;
     static constexpr uint32_t INF = 0xffffffffu;
-    __device__ static T add(T d, const void* __restrict__ w, uint32_t p, unsigned int* __restrict__ ovf)
+    __device__ static T add(T d, T w, unsigned int* __restrict__ ovf)
     {
-        const uint32_t s = d + ((const uint32_t*)w)[p];
+        const uint32_t s = d + w;
         if (s < d || s == INF) {
             *ovf = 1u;
             return INF;
@@ -602,154 +605,235 @@ __global__ void k_mss_roots(const uint32_t* __restrict__ roots, uint32_t n, type
 }
 
 // Marks the out-neighbours of the vertices set in `active` in `touched`.
-// Lanes take vertices with few out-edges; longer lists are walked by the
-// whole wavefront.
+// Lanes take vertices with few out-edges; longer lists are left to
+// k_mss_touch_heavy as chunks of WG_MSS_CHUNK out-edges, so that a hub's list
+// is spread over many wavefronts (one wavefront walking it alone took 420 us
+// of a 1.0 ms round on rmat-s18).  At most E/32 + E/WG_MSS_CHUNK chunks are
+// listed, which heavy_list holds; heavy_cap bounds the writes regardless.
+#define WG_MSS_CHUNK 1024u
 __global__ __launch_bounds__(WG_BLOCK) void k_mss_touch(const uint64_t* __restrict__ active, uint64_t nwords,
                                                          const uint32_t* __restrict__ csri_off,
                                                          const uint32_t* __restrict__ csri_pos,
                                                          const uint32_t* __restrict__ dst,
-                                                         unsigned long long* __restrict__ touched)
+                                                         unsigned long long* __restrict__ touched,
+                                                         uint32_t* __restrict__ heavy, uint32_t heavy_cap,
+                                                         wg_dev_counters* __restrict__ ctr)
 {
     const int lane = wg_lane();
     const uint64_t nwaves = (uint64_t)gridDim.x * WG_WPB;
     for (uint64_t w = (uint64_t)blockIdx.x * WG_WPB + threadIdx.x / WG_WAVE; w < nwords; w += nwaves) {
         const uint64_t bits = active[w];
-        if (!bits)
+        if (!((bits >> lane) & 1ull))
             continue;
         const uint32_t u = (uint32_t)(w * 64 + (uint64_t)lane);
-        uint32_t s = 0, e = 0;
-        if ((bits >> lane) & 1ull) {
-            s = csri_off[u];
-            e = csri_off[u + 1];
+        const uint32_t s = csri_off[u], e = csri_off[u + 1];
+        if (e - s > WG_WEDGE_LANE_MAX) {
+            const uint32_t nch = (e - s + WG_MSS_CHUNK - 1) / WG_MSS_CHUNK;
+            const uint32_t base = atomicAdd(&ctr->heavy_len, nch);
+            for (uint32_t c = 0; c < nch && base + c < heavy_cap; ++c) {
+                heavy[2 * (base + c)] = u;
+                heavy[2 * (base + c) + 1] = s + c * WG_MSS_CHUNK;
+            }
+            continue;
         }
-        const bool big = e - s > WG_WEDGE_LANE_MAX;
-        if (!big)
-            for (uint32_t p = s; p < e; ++p) {
-                const uint32_t v = dst[csri_pos[p]];
-                atomicOr(&touched[v >> 6], 1ull << (v & 63));
-            }
-        unsigned long long many = wg_ballot(big);
-        while (many) {
-            const int l = __ffsll((long long)many) - 1;
-            many &= many - 1ull;
-            const uint32_t ls = __shfl(s, l), le = __shfl(e, l);
-            for (uint32_t p = ls + (uint32_t)lane; p < le; p += WG_WAVE) {
-                const uint32_t v = dst[csri_pos[p]];
-                atomicOr(&touched[v >> 6], 1ull << (v & 63));
-            }
+        for (uint32_t p = s; p < e; ++p) {
+            const uint32_t v = dst[csri_pos[p]];
+            atomicOr(&touched[v >> 6], 1ull << (v & 63));
         }
     }
 }
 
-// Minimum over in-edges [b, e) of dist[u][lane] + w for the sources improved
-// at u (lane = source), four edges in flight.
-template <class P>
-__device__ __forceinline__ typename P::T mss_min(uint32_t b, uint32_t e, const uint32_t* __restrict__ src,
-                                                 const void* __restrict__ w, const typename P::T* __restrict__ dist,
-                                                 const unsigned long long* __restrict__ chg, int lane,
-                                                 unsigned int* __restrict__ ovf)
+// The listed chunks, one wavefront each.
+__global__ __launch_bounds__(WG_BLOCK) void k_mss_touch_heavy(const uint32_t* __restrict__ heavy, uint32_t heavy_cap,
+                                                               const uint32_t* __restrict__ csri_off,
+                                                               const uint32_t* __restrict__ csri_pos,
+                                                               const uint32_t* __restrict__ dst,
+                                                               unsigned long long* __restrict__ touched,
+                                                               const wg_dev_counters* __restrict__ ctr)
 {
-    typedef typename P::T T;
-    T m = P::INF;
-    for (uint32_t p = b; p < e; p += 4) {
-        uint32_t u[4];
-        unsigned long long c[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            u[k] = p + k < e ? src[p + k] : 0u;
-            c[k] = p + k < e ? chg[u[k]] : 0ull;
+    const uint32_t n = ctr->heavy_len < heavy_cap ? ctr->heavy_len : heavy_cap;
+    const uint32_t nwaves = gridDim.x * WG_WPB;
+    for (uint32_t i = blockIdx.x * WG_WPB + threadIdx.x / WG_WAVE; i < n; i += nwaves) {
+        const uint32_t u = heavy[2 * i], s = heavy[2 * i + 1];
+        const uint32_t end = csri_off[u + 1];
+        const uint32_t e = (s + WG_MSS_CHUNK < end) ? s + WG_MSS_CHUNK : end;
+#pragma unroll 4
+        for (uint32_t p = s + (uint32_t)wg_lane(); p < e; p += WG_WAVE) {
+            const uint32_t v = dst[csri_pos[p]];
+            const unsigned long long m = 1ull << (v & 63);
+            if (!(touched[v >> 6] & m))
+                atomicOr(&touched[v >> 6], m);
         }
-        T x[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-            x[k] = ((c[k] >> lane) & 1ull) ? dist[(uint64_t)u[k] * WG_MS_MAX_SOURCES + lane] : P::INF;
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-            if (x[k] != P::INF) {
-                const T cand = P::add(x[k], w, p + k, ovf);
-                m = cand < m ? cand : m;
-            }
     }
-    return m;
 }
 
-// Relaxation over the edge tiles, one wavefront per tile, lane = source.  A
-// light tile relaxes its destinations one after the other and owns them; a
-// heavy tile (part of one destination's in-edges) folds its minimum in with
-// per-lane atomics.  With `sel`, only the destinations set in it are relaxed.
-// Improved sources go to chg_next[v], improved vertices to the bitmask bm.
+// The value lane l (uniform) of the wavefront holds.
+__device__ __forceinline__ uint32_t lane_value(uint32_t x, int l)
+{
+    return (uint32_t)__builtin_amdgcn_readlane((int)x, l);
+}
+__device__ __forceinline__ unsigned long long lane_value(unsigned long long x, int l)
+{
+    return ((unsigned long long)lane_value((uint32_t)(x >> 32), l) << 32) | lane_value((uint32_t)x, l);
+}
+
+// End of a destination of a light tile, which its wavefront owns: the improved
+// sources (lanes) are stored, set in chg_next[v], and v in bm.
 template <class P>
-__global__ __launch_bounds__(WG_BLOCK) void k_mss_relax(const uint32_t* __restrict__ off, const uint32_t* __restrict__ src,
+__device__ __forceinline__ void mss_settle(uint32_t v, typename P::T m, typename P::T old,
+                                           typename P::T* __restrict__ dist, unsigned long long* __restrict__ chg_next,
+                                           unsigned long long* __restrict__ bm, const uint32_t* __restrict__ od, int lane,
+                                           act_tally& t)
+{
+    const bool better = m < old;
+    if (better)
+        dist[(uint64_t)v * WG_MS_MAX_SOURCES + lane] = m;
+    const unsigned long long nm = wg_ballot(better);
+    if (nm) {
+        const unsigned long long fresh = wg_ballot(better && old == P::INF);
+        if (lane == 0) {
+            chg_next[v] = nm;
+            t.edges += od[v];
+            t.verts += 1ull;
+            t.fresh += (unsigned long long)__popcll(fresh);
+            atomicOr(&bm[v >> 6], 1ull << (v & 63));
+        }
+    }
+}
+
+// Relaxation over the edge tiles, one wavefront per tile.  Only an edge whose
+// source improved in the last round (a bit of `active`) can lower anything, so
+// the wavefront first tests 64 edges at a time, an edge per lane, and then
+// walks the ones left with lane = source: WG_MSS_FLIGHT edges at a time, their
+// source rows and the rows of the destinations they start all loading
+// together.  (Walking destination by destination, each with its own chain of
+// offset, source, mask and row loads, took 620 us per round on rmat-s18, whose
+// rows fit the Infinity Cache; this way 190 us, and 64 sources 27 -> 5 ms.)  A light tile owns its
+// destinations; a heavy tile (part of one destination's in-edges) folds its
+// minimum in with per-lane atomics.  `sel`, if given, holds every destination
+// of an active source: tiles without one are skipped before their edges are
+// read.  Improved sources go to chg_next[v], improved vertices to the bitmask
+// bm.
+#define WG_MSS_FLIGHT 8
+#define MSS_MARK_LOG2 11 // destinations are marked up to E / 2048 active out-edges
+template <class P>
+__global__ __launch_bounds__(WG_BLOCK) void k_mss_relax(const uint32_t* __restrict__ src, const uint32_t* __restrict__ dst,
                                                          const void* __restrict__ w, const uint32_t* __restrict__ od,
                                                          const uint32_t* __restrict__ tile_v,
                                                          const uint32_t* __restrict__ tile_e, uint32_t ntiles,
                                                          typename P::T* __restrict__ dist,
                                                          const unsigned long long* __restrict__ chg,
                                                          unsigned long long* __restrict__ chg_next,
+                                                         const uint64_t* __restrict__ active,
                                                          const uint64_t* __restrict__ sel, unsigned long long* __restrict__ bm,
                                                          unsigned int* __restrict__ ovf, wg_dev_counters* __restrict__ ctr)
 {
     typedef typename P::T T;
+    constexpr int K = WG_MSS_FLIGHT;
     const int lane = wg_lane();
     const uint32_t stride = gridDim.x * WG_WPB;
     act_tally t = { 0ull, 0ull, 0ull };
     for (uint32_t ti = blockIdx.x * WG_WPB + threadIdx.x / WG_WAVE; ti < ntiles; ti += stride) {
-        const uint32_t tv = tile_v[ti];
+        const uint32_t tv = __builtin_amdgcn_readfirstlane(tile_v[ti]);
         const uint32_t v0 = tv & ~WG_HEAVY_BIT;
-        if (tv & WG_HEAVY_BIT) {
-            if (sel && !((sel[v0 >> 6] >> (v0 & 63)) & 1ull))
-                continue;
-            const T m = mss_min<P>(tile_e[ti], tile_e[ti + 1], src, w, dist, chg, lane, ovf);
-            const uint64_t slot = (uint64_t)v0 * WG_MS_MAX_SOURCES + lane;
-            bool better = false;
-            if (m < dist[slot]) {
-                const T old = atomic_min_t<T>(&dist[slot], m);
-                better = m < old;
-                if (better && old == P::INF)
-                    t.fresh += 1ull; // counted once: only the atomic that replaced INF sees it
+        const bool heavy = (tv & WG_HEAVY_BIT) != 0u;
+        if (sel) { // none of the tile's destinations (at most 256) is selected: skip its edges
+            const uint32_t v1 = heavy ? v0 + 1u : tile_v[ti + 1] & ~WG_HEAVY_BIT;
+            const uint32_t wd = (v0 >> 6) + (uint32_t)lane;
+            bool any = false;
+            if (wd <= (v1 - 1u) >> 6) {
+                uint64_t bits = sel[wd];
+                if (wd == v0 >> 6)
+                    bits &= ~0ull << (v0 & 63u);
+                if (wd == (v1 - 1u) >> 6)
+                    bits &= ~0ull >> (63u - ((v1 - 1u) & 63u));
+                any = bits != 0ull;
             }
-            const unsigned long long nm = wg_ballot(better);
-            if (lane == 0 && nm) {
-                const unsigned long long was = atomicOr(&chg_next[v0], nm);
-                if (!was) { // first improvement of v0 this iteration
-                    t.edges += od[v0];
-                    t.verts += 1ull;
-                    atomicOr(&bm[v0 >> 6], 1ull << (v0 & 63));
+            if (!wg_ballot(any))
+                continue;
+        }
+        const uint32_t e0 = tile_e[ti], e1 = tile_e[ti + 1];
+        uint32_t cur = 0xffffffffu; // destination being summed up (uniform), none yet
+        T m = P::INF, old = P::INF;
+        for (uint32_t p = e0; p < e1; p += WG_WAVE) {
+            const uint32_t q = p + (uint32_t)lane;
+            const uint32_t u = q < e1 ? src[q] : 0u;
+            const bool a = q < e1 && test_bit64(active, u);
+            const uint32_t v = (a && !heavy) ? dst[q] : v0;
+            unsigned long long left = wg_ballot(a);
+            if (!left)
+                continue;
+            const unsigned long long c = a ? chg[u] : 0ull;
+            const T we = a ? ((const T*)w)[q] : T(0); // the weight's bits
+            while (left) {
+                const int n = __popcll(left) < K ? __popcll(left) : K;
+                uint32_t vk[K];
+                T wk[K], x[K], o[K];
+#pragma unroll
+                for (int k = 0; k < K; ++k) {
+                    // past the last edge: that edge again, its loads left out
+                    const int l = k < n ? __ffsll((long long)left) - 1 : 0;
+                    left &= left - 1ull;
+                    const uint32_t uk = lane_value(u, l);
+                    const unsigned long long ck = lane_value(c, l);
+                    vk[k] = lane_value(v, l);
+                    wk[k] = lane_value(we, l);
+                    x[k] = (k < n && ((ck >> lane) & 1ull)) ? dist[(uint64_t)uk * WG_MS_MAX_SOURCES + lane] : P::INF;
+                    o[k] = P::INF;
+                    if (k < n && !heavy && vk[k] != (k ? vk[k - 1] : cur))
+                        o[k] = dist[(uint64_t)vk[k] * WG_MS_MAX_SOURCES + lane];
+                }
+#pragma unroll
+                for (int k = 0; k < K; ++k) {
+                    if (k >= n)
+                        break;
+                    if (!heavy && vk[k] != cur) {
+                        if (cur != 0xffffffffu)
+                            mss_settle<P>(cur, m, old, dist, chg_next, bm, od, lane, t);
+                        cur = vk[k];
+                        m = P::INF;
+                        old = o[k];
+                    }
+                    if (x[k] != P::INF) {
+                        const T cand = P::add(x[k], wk[k], ovf);
+                        m = cand < m ? cand : m;
+                    }
                 }
             }
+        }
+        if (!heavy) {
+            if (cur != 0xffffffffu)
+                mss_settle<P>(cur, m, old, dist, chg_next, bm, od, lane, t);
             continue;
         }
-        const uint32_t v1 = tile_v[ti + 1] & ~WG_HEAVY_BIT;
-        for (uint32_t v = v0; v < v1; ++v) {
-            if (sel && !((sel[v >> 6] >> (v & 63)) & 1ull))
-                continue;
-            const T m = mss_min<P>(off[v], off[v + 1], src, w, dist, chg, lane, ovf);
-            const uint64_t slot = (uint64_t)v * WG_MS_MAX_SOURCES + lane;
-            const T old = dist[slot];
-            const bool better = m < old;
-            if (better)
-                dist[slot] = m;
-            const unsigned long long nm = wg_ballot(better);
-            if (nm) {
-                const unsigned long long fresh = wg_ballot(better && old == P::INF);
-                if (lane == 0) {
-                    chg_next[v] = nm;
-                    t.edges += od[v];
-                    t.verts += 1ull;
-                    t.fresh += (unsigned long long)__popcll(fresh);
-                    atomicOr(&bm[v >> 6], 1ull << (v & 63));
-                }
+        const uint64_t slot = (uint64_t)v0 * WG_MS_MAX_SOURCES + lane;
+        bool better = false;
+        if (m < dist[slot]) {
+            const T was = atomic_min_t<T>(&dist[slot], m);
+            better = m < was;
+            if (better && was == P::INF)
+                t.fresh += 1ull; // counted once: only the atomic that replaced INF sees it
+        }
+        const unsigned long long nm = wg_ballot(better);
+        if (lane == 0 && nm) {
+            const unsigned long long was = atomicOr(&chg_next[v0], nm);
+            if (!was) { // first improvement of v0 this iteration
+                t.edges += od[v0];
+                t.verts += 1ull;
+                atomicOr(&bm[v0 >> 6], 1ull << (v0 & 63));
             }
         }
     }
     add_tally(t, ctr); // counts sit in lane 0; the wave sum adds the zeros of the others
 }
 
+// Source s's distances in the caller's numbering.
 template <class P>
-__global__ void k_mss_column(const typename P::T* __restrict__ dist, uint32_t s, uint64_t V, typename P::T* __restrict__ out)
+__global__ void k_mss_column(const typename P::T* __restrict__ dist, uint32_t s, const uint32_t* __restrict__ inv,
+                             uint64_t V, typename P::T* __restrict__ out)
 {
     for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < V; v += (uint64_t)gridDim.x * blockDim.x)
-        out[v] = dist[v * WG_MS_MAX_SOURCES + s];
+        out[v] = dist[(uint64_t)(inv ? inv[v] : v) * WG_MS_MAX_SOURCES + s];
 }
 
 template <class P>
@@ -778,41 +862,60 @@ static int mssssp_run(wg_ctx* ctx, const std::vector<uint32_t>& roots, const wg_
     unsigned long long* touched = (unsigned long long*)aux;
     uint32_t* droots = (uint32_t*)((char*)aux + nw * 8);
     unsigned long long *chg = (unsigned long long*)c0, *chg_next = (unsigned long long*)c1;
+    uint64_t *active = ctx->bm_cur, *improved = ctx->bm_next; // vertices improved last round / this round
     unsigned int* ovf = &ctx->ctr->overflow;
     WG_HIP(ctx, hipMemcpyAsync(droots, roots.data(), (size_t)n * 4, hipMemcpyHostToDevice, ctx->stream));
     hipLaunchKernelGGL(k_mss_init<P>, dim3(wg_grid(ctx, (uint64_t)V * WG_MS_MAX_SOURCES, 1024, 8)), dim3(256), 0,
                        ctx->stream, (T*)dist, (uint64_t)V * WG_MS_MAX_SOURCES);
     if ((rc = wg_check_launch(ctx)) || (rc = wg_clear_u64(ctx, (uint64_t*)chg, V)) ||
-        (rc = wg_clear_u64(ctx, (uint64_t*)chg_next, V)) || (rc = wg_clear_u64(ctx, (uint64_t*)touched, nw)) ||
-        (rc = wg_clear_u64(ctx, ctx->bm_next, nw)) || (rc = wg_reset_counters(ctx, RST_ACTIVITY | RST_OVERFLOW)))
+        (rc = wg_clear_u64(ctx, (uint64_t*)touched, nw)) || (rc = wg_clear_u64(ctx, active, nw)) ||
+        (rc = wg_reset_counters(ctx, RST_ACTIVITY | RST_OVERFLOW)))
         return rc;
     hipLaunchKernelGGL(k_mss_roots<P>, dim3((n + 63) / 64), dim3(64), 0, ctx->stream, droots, n, (T*)dist, chg,
-                       (unsigned long long*)ctx->bm_next, ctx->od, ctx->ctr);
-    if ((rc = wg_check_launch(ctx)) || (rc = wg_read_counters(ctx)))
+                       (unsigned long long*)active, ctx->od, ctx->ctr);
+    if ((rc = wg_check_launch(ctx)) || (rc = wg_take_activity(ctx)))
         return rc;
     unsigned long long act = ctx->hctr->activity;
     const unsigned long long threshold = (ctx->E * (unsigned long long)params->threshold_pct) / 100ull;
     const uint64_t cap = 64ull * V + 64ull;
+    // 128-edge tiles until there are 512-edge ones enough for every wavefront
+    // slot eight times over: a wavefront walks its tile's rows one after the
+    // other (128 / 256 / 512 edges: rmat-s14 1.3 / 1.7 / 2.4 ms, rmat-s18 5.0 /
+    // 5.5 / 6.2, rmat-s20 15.7 / 15.9 / 16.7, rmat-s23 139 / 136 / 134)
+    const bool fine = ctx->ntiles < 8u * 32u * (uint32_t)ctx->num_cu;
+    if (fine && (rc = wg_build_pr_tiling(ctx, WG_ALT_IPT2)))
+        return rc;
+    const uint32_t* tile_v = fine ? ctx->pr_alt[WG_ALT_IPT2].tile_v : ctx->tile_v;
+    const uint32_t* tile_e = fine ? ctx->pr_alt[WG_ALT_IPT2].tile_e : ctx->tile_e;
+    const uint32_t ntiles = fine ? ctx->pr_alt[WG_ALT_IPT2].ntiles : ctx->ntiles;
+    const uint32_t grid = wg_grid(ctx, ntiles, WG_WPB, 64);
     uint64_t it = 0;
     for (;;) {
-        const bool dense = params->schedule == 2 || (params->schedule != 3 && act > threshold);
-        if ((rc = wg_reset_counters(ctx, RST_ACTIVITY)))
-            return rc;
-        if (!dense) {
-            hipLaunchKernelGGL(k_mss_touch, dim3(wg_wedge_build_grid(ctx)), dim3(WG_BLOCK), 0, ctx->stream,
-                               ctx->bm_next, nw, ctx->csri_off, ctx->csri_pos, ctx->dst, touched);
+        // Marking the destinations costs three random accesses per out-edge of
+        // the improved vertices and pays by the tiles it leaves out; a round
+        // without it reads every edge's source and tests its bit.
+        const bool sparse = params->schedule == 3 ||
+                            (params->schedule != 2 && act <= threshold && act <= ctx->E >> MSS_MARK_LOG2);
+        if (sparse) {
+            if ((rc = wg_reset_counters(ctx, RST_HEAVY)))
+                return rc;
+            hipLaunchKernelGGL(k_mss_touch, dim3(wg_wedge_build_grid(ctx)), dim3(WG_BLOCK), 0, ctx->stream, active, nw,
+                               ctx->csri_off, ctx->csri_pos, ctx->dst, touched, ctx->heavy_list, ctx->heavy_cap,
+                               ctx->ctr);
+            hipLaunchKernelGGL(k_mss_touch_heavy, dim3(ctx->num_cu * 4), dim3(WG_BLOCK), 0, ctx->stream,
+                               ctx->heavy_list, ctx->heavy_cap, ctx->csri_off, ctx->csri_pos, ctx->dst, touched,
+                               ctx->ctr);
             if ((rc = wg_check_launch(ctx)))
                 return rc;
         }
-        // the improved-vertex bitmask is rebuilt by the relaxation
-        if ((rc = wg_clear_u64(ctx, ctx->bm_next, nw)))
+        if ((rc = wg_clear_u64(ctx, improved, nw)) || (rc = wg_clear_u64(ctx, (uint64_t*)chg_next, V)))
             return rc;
-        hipLaunchKernelGGL(k_mss_relax<P>, dim3(ctx->pr_grid), dim3(WG_BLOCK), 0, ctx->stream, ctx->off, ctx->src, ctx->w,
-                           ctx->od, ctx->tile_v, ctx->tile_e, ctx->ntiles, (T*)dist, chg, chg_next,
-                           dense ? (const uint64_t*)nullptr : (const uint64_t*)touched,
-                           (unsigned long long*)ctx->bm_next, ovf, ctx->ctr);
-        if ((rc = wg_check_launch(ctx)) || (!dense && (rc = wg_clear_u64(ctx, (uint64_t*)touched, nw))) ||
-            (rc = wg_read_counters(ctx)))
+        hipLaunchKernelGGL(k_mss_relax<P>, dim3(grid), dim3(WG_BLOCK), 0, ctx->stream, ctx->src, ctx->dst, ctx->w,
+                           ctx->od, tile_v, tile_e, ntiles, (T*)dist, chg, chg_next, active,
+                           sparse ? (const uint64_t*)touched : (const uint64_t*)nullptr,
+                           (unsigned long long*)improved, ovf, ctx->ctr);
+        if ((rc = wg_check_launch(ctx)) || (sparse && (rc = wg_clear_u64(ctx, (uint64_t*)touched, nw))) ||
+            (rc = wg_take_activity(ctx))) // the counters start the next round at 0
             return rc;
         ++it;
         if (ctx->hctr->activated == 0)
@@ -820,15 +923,13 @@ static int mssssp_run(wg_ctx* ctx, const std::vector<uint32_t>& roots, const wg_
         if (it > cap || (params->max_iterations && it >= params->max_iterations))
             break;
         act = ctx->hctr->activity;
-        // the improved masks become the next iteration's input; the old ones are cleared for reuse
-        unsigned long long* tmp = chg;
-        chg = chg_next;
-        chg_next = tmp;
-        if ((rc = wg_clear_u64(ctx, (uint64_t*)chg_next, V)))
-            return rc;
+        std::swap(chg, chg_next); // the improved masks and vertices are the next round's input
+        std::swap(active, improved);
     }
     if (iters)
         *iters = it;
+    if ((rc = wg_read_counters(ctx)))
+        return rc;
     return ctx->hctr->overflow ? WG_E_OVERFLOW : WG_OK;
 }
 
@@ -864,18 +965,19 @@ extern "C" int wg_read_mssssp(wg_ctx* ctx, uint32_t source, void* host_dist)
     if (source >= ctx->ms_n)
         return WG_E_RANGE;
     const size_t esz = ctx->wkind == WG_WEIGHT_F64 ? 8 : 4;
-    void* tmp = nullptr;
-    WG_HIP(ctx, hipMalloc(&tmp, ctx->V * esz));
+    void* stage = nullptr;
+    int rc = wg_stage(ctx, ctx->V * esz, &stage);
+    if (rc)
+        return rc;
     const uint32_t grid = wg_grid(ctx, ctx->V, 1024, 8);
     if (esz == 8)
         hipLaunchKernelGGL(k_mss_column<MsF64>, dim3(grid), dim3(256), 0, ctx->stream,
-                           (const unsigned long long*)ctx->prop[0], source, ctx->V, (unsigned long long*)tmp);
+                           (const unsigned long long*)ctx->prop[0], source, ctx->inv, ctx->V,
+                           (unsigned long long*)stage);
     else
         hipLaunchKernelGGL(k_mss_column<MsU32>, dim3(grid), dim3(256), 0, ctx->stream, (const uint32_t*)ctx->prop[0],
-                           source, ctx->V, (uint32_t*)tmp);
-    int rc = wg_check_launch(ctx);
-    if (!rc)
-        rc = wg_read_vertex_array(ctx, tmp, host_dist, esz);
-    (void)hipFree(tmp);
-    return rc;
+                           source, ctx->inv, ctx->V, (uint32_t*)stage);
+    if ((rc = wg_check_launch(ctx)))
+        return rc;
+    return wg_copy_out(ctx, stage, host_dist, ctx->V * esz);
 }
