@@ -2,7 +2,7 @@
 pull bins of 4K, 8K and 16K vertices of the binned layout, the 128- and
 512-edge tiles of the 64-source SSSP with and without marked destinations
 (hub lists cut into chunks), and one to eight wavefronts per tile of the
-personalised PageRank.  Against the oracle: exact for BFS, CC and SSSP, 1e-10
+personalised PageRank, BFS levels in one workgroup.  Against the oracle: exact for BFS, CC and SSSP, 1e-10
 L1 for FP64 PageRank (sums of FP64 values in another order), 2e-7 L1 for
 FP32-stored contributions (one rounding of 6e-8 per contribution)."""
 from __future__ import annotations
@@ -96,5 +96,75 @@ def test_ppr_wavefronts_per_tile(V):
         c.ppr(seeds, 5, 0.85)
         for i in range(len(seeds)):
             assert float(np.abs(c.read_ppr(i) - want[i]).sum()) <= 2e-7, i
+    finally:
+        c.close()
+
+
+def _levels_graph(name):
+    """Road-like graphs (at most 4 out-edges per vertex) whose levels take each
+    road through the one-workgroup levels."""
+    if name == "grid":  # levels stay small
+        return W.grid(37, 53, seed=4, p_keep=0.9)
+    if name == "wide":  # levels outgrow one workgroup (2048 vertices) and shrink again
+        return _broom(5000)
+    return _broom(300)
+
+
+def _broom(width):
+    """A path, a fan of `width` vertices (more destinations than a record
+    holds) each with a chain of 5, all chains meeting in one vertex, and a path."""
+    n = 0
+    src, dst = [], []
+
+    def chain(a, length):
+        nonlocal n
+        for _ in range(length):
+            src.append(a)
+            dst.append(n)
+            a = n
+            n += 1
+        return a
+
+    n = 1
+    hub = chain(0, 20)
+    ends = [chain(hub, 6) for _ in range(width)]
+    meet = n
+    n += 1
+    for e in ends:
+        src.append(e)
+        dst.append(meet)
+    chain(meet, 30)
+    return W.from_edges(n, src, dst)
+
+
+@pytest.mark.parametrize("relabel", [False, True])
+@pytest.mark.parametrize("name", ["grid", "wide", "fan"])
+def test_bfs_levels_in_one_workgroup(name, relabel):
+    g = _levels_graph(name)
+    root = 0 if name != "grid" else g.max_outdegree_vertex()
+    _, depth, _ = oracle.Oracle.of(g, 4).bfs(root)
+    W.mlp_load()
+    c = W.Context(0, relabel=relabel)
+    try:
+        c.load(g)
+        c.set_schedule_model(W.mlp_get())
+        for schedule, cap in ((W.SCHED_FRONTIER, 0), (W.SCHED_PLAIN, 0), (W.SCHED_LEARNED, 0), (W.SCHED_FRONTIER, 9)):
+            got = []
+            for wgs in (0, 32, 1):
+                c.set_fused_levels(wgs)
+                c.init_bfs(root)
+                it = c.converge(schedule, max_iterations=cap)
+                got.append((c.read_bfs(), it))
+                if schedule == W.SCHED_FRONTIER and wgs == 32:
+                    assert c.fused_level_count() > 0
+                if cap:  # what follows finds visited, frontier and depths as after any level
+                    c.edge_pull(W.APP_BFS, W.MODE_DENSE)
+                    got[-1] += (c.read_bfs(),)
+            for other in got[1:]:
+                assert other[1] == got[0][1], (schedule, cap)
+                for a, b in zip(got[0][::2], other[::2]):
+                    assert np.array_equal(a, b), (schedule, cap)
+            if not cap:
+                assert np.array_equal(W.bfs_depth(got[0][0]), depth), schedule
     finally:
         c.close()

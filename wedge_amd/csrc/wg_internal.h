@@ -183,6 +183,8 @@ struct wg_ctx {
                               // none or more than WG_BFS_HEAVY (built by the first BFS init)
     uint32_t* csr_dst;        // BFS: destination of out-edge position p, dst[csri_pos[p]] (E entries,
                               // built by the first BFS init)
+    uint4* solo_rec;          // BFS: out-degree and first destinations of each vertex, on graphs with few
+                              // out-edges per vertex (built by the first BFS init)
     uint32_t* bfs_heavy_v;
     uint32_t* bfs_heavy_e;    // chunk start edge (chunk end = min(start + WG_BFS_HEAVY, off[v+1]))
     uint32_t n_out_pos;       // vertices with out-degree > 0

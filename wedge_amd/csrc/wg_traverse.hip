@@ -1174,6 +1174,29 @@ __global__ __launch_bounds__(WG_BLOCK) void k_level_advance(uint64_t* __restrict
 // error.
 #define WG_RUN_SPIN (1u << 19)
 
+// Levels of one workgroup (bfs_solo, below).
+#define SOLO_T 1024u
+#define SOLO_WAVES (SOLO_T / WG_WAVE)
+#define SOLO_NACT 2048u
+#define SOLO_PER (SOLO_NACT / SOLO_T)
+#define SOLO_ACT 12288u
+#define SOLO_Q SOLO_ACT    // queue entries: a level appends at most one per out-edge
+#define SOLO_MEAN_DEGREE 4u // records and such levels up to this many out-edges per vertex
+#define SOLO_REC 7u        // destinations in a vertex's record
+#define SOLO_NBIG (SOLO_ACT / (SOLO_REC + 1u))
+
+// x as a value the compiler knows nothing about, in its register now.  For
+// several loads or atomics in flight, each in a branch of its own: their
+// results start from such a value (from a constant, what is done with a result
+// is folded into its branch, and the wavefront waits for one before it issues
+// the next), and an operand that comes from a load is waited for ahead of them
+// (else every branch waits for all that is outstanding).
+__device__ __forceinline__ unsigned long long opaque(unsigned long long x)
+{
+    asm volatile("" : "+v"(x));
+    return x;
+}
+
 __device__ bool run_barrier(wg_run_ctl* __restrict__ rc, unsigned int G, wg_dev_counters* __restrict__ ctr)
 {
     __shared__ int s_ok;
@@ -1416,7 +1439,7 @@ __device__ void run_entry(const uint64_t* __restrict__ act, uint64_t nwords, con
 __device__ __forceinline__ bool run_level_end(wg_run_ctl* __restrict__ rc, wg_dev_counters* __restrict__ ctr,
                                               unsigned int r, unsigned long long act, unsigned long long nact,
                                               unsigned long long fresh, run_state& st, const float* s_mlp, bool learned,
-                                              bool* ok)
+                                              bool solo, bool* ok)
 {
     const unsigned int rn = (r + 1u) % 3u, rz = (r + 2u) % 3u;
     __shared__ int s_dec[2];
@@ -1464,9 +1487,13 @@ __device__ __forceinline__ bool run_level_end(wg_run_ctl* __restrict__ rc, wg_de
     const int mode = stop ? 0 : s_dec[0];
     const int blog2 = stop ? st.g.plain_blog2 : s_dec[1];
     __syncthreads();
+    // a level that one workgroup does faster goes back to the decision kernel
+    // (if that takes levels; half of what it takes, so that a level near the line
+    // does not come straight back)
+    const bool small = solo && N <= SOLO_NACT / 2u && A <= SOLO_ACT / 2u;
     const bool cont =
         !stop && mode == WG_MODE_FRONTIER && A <= WG_RUN_ACT_PER_WG * gridDim.x &&
-        N <= WG_RUN_NACT_PER_WG * gridDim.x && T <= WG_RUN_QCAP;
+        N <= WG_RUN_NACT_PER_WG * gridDim.x && T <= WG_RUN_QCAP && !small;
     if (!cont && blockIdx.x == 0 && threadIdx.x == 0) {
         ctr->iters = st.iters;
         ctr->fiters = st.fiters;
@@ -1499,7 +1526,7 @@ __global__ __launch_bounds__(WG_BLOCK) void k_bfs_run(const uint32_t* __restrict
                                                        uint64_t nwords, const uint32_t* __restrict__ perm,
                                                        uint4* __restrict__ qa, uint4* __restrict__ qb,
                                                        wg_run_ctl* __restrict__ rc, wg_dev_counters* __restrict__ ctr,
-                                                       const float* __restrict__ mlp)
+                                                       const float* __restrict__ mlp, bool solo)
 {
     run_state st;
     if (!run_gate(ctr, st))
@@ -1536,17 +1563,23 @@ __global__ __launch_bounds__(WG_BLOCK) void k_bfs_run(const uint32_t* __restrict
                     atomicAnd((unsigned long long*)&next[u >> 6], ~m);
                 }
                 const uint32_t pid = perm ? perm[u] : u;
-                const unsigned long long val = (newdepth << 32) | (unsigned long long)pid;
+                const unsigned long long val = opaque((newdepth << 32) | (unsigned long long)pid);
                 work.edges += en.z - en.y; // each out-edge and its destination's state
                 work.dests += en.z - en.y;
 #pragma unroll
                 for (int j = 0; j < (int)WG_RUN_CH; ++j)
                     if (en.y + (uint32_t)j < en.z)
                         vv[j] = csr_dst[en.y + (uint32_t)j];
+                unsigned long long old[WG_RUN_CH];
+#pragma unroll
+                for (int j = 0; j < (int)WG_RUN_CH; ++j) {
+                    old[j] = opaque(0ull);
+                    if (en.y + (uint32_t)j < en.z)
+                        old[j] = atomicMin((unsigned long long*)&packed[vv[j]], val);
+                }
 #pragma unroll
                 for (int j = 0; j < (int)WG_RUN_CH; ++j)
-                    if (en.y + (uint32_t)j < en.z)
-                        nw[j] = atomicMin((unsigned long long*)&packed[vv[j]], val) == ~0ull;
+                    nw[j] = old[j] == ~0ull;
 #pragma unroll
                 for (int j = 0; j < (int)WG_RUN_CH; ++j)
                     if (nw[j]) {
@@ -1568,7 +1601,7 @@ __global__ __launch_bounds__(WG_BLOCK) void k_bfs_run(const uint32_t* __restrict
         add_work(work, ctr);
         work = work_tally<CW>();
         // a BFS activation is always a first visit
-        if (!run_level_end(rc, ctr, r, act, nact, nact, st, s_mlp, learned, &ok))
+        if (!run_level_end(rc, ctr, r, act, nact, nact, st, s_mlp, learned, solo, &ok))
             return;
         uint4* t = qc;
         qc = qn;
@@ -1666,7 +1699,7 @@ __global__ __launch_bounds__(WG_BLOCK) void k_min_run(const uint32_t* __restrict
         bool ok = true;
         add_work(work, ctr);
         work = work_tally<CW>();
-        if (!run_level_end(rc, ctr, r, act, nact, fresh, st, s_mlp, learned, &ok)) {
+        if (!run_level_end(rc, ctr, r, act, nact, fresh, st, s_mlp, learned, false, &ok)) {
             if (ok && (r & 1u) == 0u) // the last activations are in spare
                 for (uint64_t wd = (uint64_t)blockIdx.x * WG_BLOCK + threadIdx.x; wd < nwords;
                      wd += (uint64_t)gridDim.x * WG_BLOCK) {
@@ -1682,6 +1715,330 @@ __global__ __launch_bounds__(WG_BLOCK) void k_min_run(const uint32_t* __restrict
         qc = qn;
         qn = t;
     }
+}
+
+// ---- levels in one workgroup --------------------------------------------------------
+//
+// A level of up to about a thousand vertices is bound by its chain of dependent
+// memory round trips, and in a fused run half of that chain is traffic between
+// workgroups: the queue's entries and tail, the counts, the barrier (9-11 us per
+// level with 32 workgroups).  On graphs with few out-edges per vertex the
+// decision kernel, which is one workgroup anyway, therefore goes on with such
+// levels itself, 1024 threads strong, its queues in LDS.  What remains per level
+// is the vertices' records (out-degree and first destinations in 32 bytes), the
+// destinations' visited bits, the atomicMin of those not visited, and an LDS
+// append: 2.6 us on a 60x80 road grid, 2.9 on 300x401, 6.6 on 1000x1501 (whose
+// lines come from beyond the L2, at the rate one CU takes them).  It stops when a
+// level outgrows it (SOLO_NACT vertices or SOLO_ACT out-edges, where 32
+// workgroups are faster: 15 us a level against 11 with 4096 vertices on the
+// 4096x6144 grid), and the loop goes on from there: a fused run if the level
+// suits one, else a level per launch sequence.
+
+// Sum over the wavefront by DPP adds; every lane gets it.
+__device__ __forceinline__ uint32_t wave_sum_dpp(uint32_t x)
+{
+    int v = (int)x;
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true); // row_shr:1, 2, 4, 8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false); // row_bcast:15 into rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false); // row_bcast:31 into rows 2 and 3
+    return (uint32_t)__builtin_amdgcn_readlane(v, WG_WAVE - 1);
+}
+
+// A word that this kernel's atomics change: read past the L1, where an old one
+// would stay.
+__device__ __forceinline__ unsigned long long solo_load(const uint64_t* p)
+{
+    return __hip_atomic_load((const unsigned long long*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Appends the vertices v[j] with put[j] set to the LDS queue: one LDS atomic
+// per wavefront.  Called by the lanes of a wavefront that are active together;
+// entries past the queue's end are not written (the caller sees the tail).
+template <int N>
+__device__ __forceinline__ void solo_append(uint32_t* q, uint32_t* tail, uint32_t cap, const uint32_t* v, const bool* put)
+{
+    uint32_t pre[N], tot = 0;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        const unsigned long long m = wg_ballot(put[j]);
+        pre[j] = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, tot));
+        tot += (uint32_t)__popcll(m);
+    }
+    if (!tot) // uniform
+        return;
+    uint32_t base = 0;
+    const unsigned long long here = wg_ballot(true);
+    const int leader = __ffsll((long long)here) - 1;
+    if (wg_lane() == leader)
+        base = atomicAdd(tail, tot);
+    base = (uint32_t)__builtin_amdgcn_readlane((int)base, leader);
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+        if (put[j] && base + pre[j] < cap)
+            q[base + pre[j]] = v[j];
+}
+
+struct solo_lds {
+    uint32_t q[2][SOLO_Q];
+    uint32_t tail[2];
+    uint32_t nbig, big[SOLO_NBIG]; // vertices of the level with more out-edges than a record holds
+    uint32_t act[2];               // out-edges of the level's vertices
+    int dec[2];
+    float mlp[WG_MLP_OFF_END];     // the schedule model, under the learned schedule
+};
+
+// rec[v]: v's out-degree and its first SOLO_REC destinations, two 16-byte words.
+__global__ void k_solo_rec(const uint32_t* __restrict__ csri_off, const uint32_t* __restrict__ csr_dst, uint64_t V,
+                           uint4* __restrict__ rec)
+{
+    for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < V; v += (uint64_t)gridDim.x * blockDim.x) {
+        const uint32_t s = csri_off[v], d = csri_off[v + 1] - s;
+        uint32_t x[SOLO_REC];
+#pragma unroll
+        for (uint32_t j = 0; j < SOLO_REC; ++j)
+            x[j] = j < d ? csr_dst[s + j] : 0u;
+        rec[2 * v] = make_uint4(d, x[0], x[1], x[2]);
+        rec[2 * v + 1] = make_uint4(x[3], x[4], x[5], x[6]);
+    }
+}
+
+// BFS levels of one workgroup (all its SOLO_T threads), in the state that
+// decide_wave left; as k_bfs_run, which see for the rules.
+template <bool CW>
+__device__ void bfs_solo(solo_lds& L, const uint32_t* __restrict__ csri_off, const uint32_t* __restrict__ csr_dst,
+                         const uint4* __restrict__ rec, uint64_t* __restrict__ next, uint64_t* __restrict__ visited,
+                         uint64_t* __restrict__ packed, uint64_t nwords, const uint32_t* __restrict__ perm,
+                         wg_dev_counters* __restrict__ ctr, const float* __restrict__ mlp)
+{
+    if (ctr->done || ctr->mode != WG_MODE_FRONTIER || ctr->last_activity > SOLO_ACT || ctr->last_activated > SOLO_NACT)
+        return;
+    run_state st;
+    st.g = read_cfg(ctr);
+    st.max_iters = ctr->max_iters;
+    st.level0 = ctr->level;
+    st.iters = ctr->iters;
+    st.fiters = ctr->fiters;
+    st.unvisited = ctr->unvisited;
+    const uint32_t tid = threadIdx.x;
+    const int lane = wg_lane();
+    if (tid < 2) {
+        L.tail[tid] = 0u;
+        L.act[tid] = 0u;
+    }
+    if (tid == 0)
+        L.nbig = 0u;
+    if (st.g.sched != LOOP_SCHED_LEARNED)
+        mlp = nullptr;
+    if (mlp)
+        for (uint32_t i = tid; i < WG_MLP_OFF_END; i += SOLO_T)
+            L.mlp[i] = mlp[i];
+    __syncthreads();
+    // the activated set leaves next for the queue (at most SOLO_NACT vertices)
+    for (uint64_t w0 = tid; w0 < nwords; w0 += (uint64_t)WG_RUN_SCAN_BATCH * SOLO_T) {
+        uint64_t x[WG_RUN_SCAN_BATCH];
+#pragma unroll
+        for (int j = 0; j < WG_RUN_SCAN_BATCH; ++j) {
+            const uint64_t w = w0 + (uint64_t)j * SOLO_T;
+            x[j] = (w < nwords) ? next[w] : 0ull;
+        }
+#pragma unroll
+        for (int j = 0; j < WG_RUN_SCAN_BATCH; ++j)
+            if (x[j]) {
+                const uint64_t w = w0 + (uint64_t)j * SOLO_T;
+                next[w] = 0ull;
+                for (uint64_t b = x[j]; b; b &= b - 1ull) {
+                    const uint32_t i = atomicAdd(&L.tail[0], 1u);
+                    if (i < SOLO_Q)
+                        L.q[0][i] = (uint32_t)(w * 64u + (uint64_t)(__ffsll((long long)b) - 1));
+                }
+            }
+    }
+    __syncthreads();
+    uint32_t cur = 0;
+    uint32_t u[SOLO_PER], deg[SOLO_PER], nb[SOLO_PER][SOLO_REC]; // this thread's vertices of the level
+    auto load_level = [&](uint32_t n) {
+#pragma unroll
+        for (uint32_t k = 0; k < SOLO_PER; ++k) {
+            const uint32_t i = tid + k * SOLO_T;
+            u[k] = i < n ? L.q[cur][i] : 0u;
+            uint4 a = make_uint4(0u, 0u, 0u, 0u), b = a;
+            if (i < n) {
+                a = rec[2ull * u[k]];
+                b = rec[2ull * u[k] + 1ull];
+            }
+            deg[k] = a.x;
+            nb[k][0] = a.y;
+            nb[k][1] = a.z;
+            nb[k][2] = a.w;
+            nb[k][3] = b.x;
+            nb[k][4] = b.y;
+            nb[k][5] = b.z;
+            nb[k][6] = b.w;
+        }
+    };
+    uint32_t n = L.tail[0];
+    n = n < SOLO_NACT ? n : SOLO_NACT; // last_activated of them
+    load_level(n);
+    work_tally<CW> work;
+    for (unsigned int r = 0;; ++r) {
+        const unsigned long long depth = (unsigned long long)(st.level0 + 2u + r) << 32;
+        uint32_t* qn = L.q[cur ^ 1u];
+        uint32_t* tn = &L.tail[cur ^ 1u];
+#pragma unroll
+        for (uint32_t k = 0; k < SOLO_PER; ++k) {
+            if (k * SOLO_T >= n) // the whole workgroup
+                break;
+            unsigned long long val = depth | (unsigned long long)u[k];
+            if (tid + k * SOLO_T < n) {
+                work.edges += deg[k]; // each out-edge and its destination's state
+                work.dests += deg[k];
+                if (perm)
+                    val = depth | (unsigned long long)perm[u[k]];
+                if (deg[k] > SOLO_REC) { // left to a wavefront
+                    const uint32_t b = atomicAdd(&L.nbig, 1u);
+                    if (b < SOLO_NBIG)
+                        L.big[b] = u[k];
+                    deg[k] = 0u;
+                }
+            }
+            val = opaque(val);
+            // most destinations were visited before, and their bits lie closer
+            // together than their packed words: only the others take an atomic
+            bool nw[SOLO_REC];
+            unsigned long long old[SOLO_REC];
+#pragma unroll
+            for (uint32_t j = 0; j < SOLO_REC; ++j) {
+                old[j] = opaque(~0ull);
+                if (j < deg[k])
+                    old[j] = solo_load(&visited[nb[k][j] >> 6]);
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < SOLO_REC; ++j)
+                nw[j] = !((old[j] >> (nb[k][j] & 63u)) & 1ull);
+#pragma unroll
+            for (uint32_t j = 0; j < SOLO_REC; ++j) {
+                old[j] = opaque(0ull);
+                if (nw[j])
+                    old[j] = atomicMin((unsigned long long*)&packed[nb[k][j]], val);
+            }
+            // (behind the atomics: a wait for them would wait for it too)
+            if (tid + k * SOLO_T < n)
+                atomicOr((unsigned long long*)&visited[u[k] >> 6], 1ull << (u[k] & 63u));
+#pragma unroll
+            for (uint32_t j = 0; j < SOLO_REC; ++j)
+                nw[j] = old[j] == ~0ull;
+            solo_append<SOLO_REC>(qn, tn, SOLO_Q, nb[k], nw);
+        }
+        __syncthreads();
+        if (const uint32_t nbig = L.nbig < SOLO_NBIG ? L.nbig : SOLO_NBIG) { // the same in the whole workgroup
+            for (uint32_t b = tid / WG_WAVE; b < nbig; b += SOLO_WAVES) {
+                const uint32_t x = L.big[b], e = csri_off[x + 1];
+                const unsigned long long val = depth | (unsigned long long)(perm ? perm[x] : x);
+                for (uint32_t c = csri_off[x]; c < e; c += WG_WAVE) {
+                    uint32_t v[1] = {0u};
+                    bool nw[1] = {false};
+                    if (c + (uint32_t)lane < e) {
+                        v[0] = csr_dst[c + (uint32_t)lane];
+                        nw[0] = !((solo_load(&visited[v[0] >> 6]) >> (v[0] & 63u)) & 1ull) &&
+                                atomicMin((unsigned long long*)&packed[v[0]], val) == ~0ull;
+                    }
+                    solo_append<1>(qn, tn, SOLO_Q, v, nw);
+                }
+            }
+            __syncthreads();
+        }
+        // the level's end: its counts, then the decision decide_wave takes
+        cur ^= 1u;
+        n = L.tail[cur]; // at most SOLO_ACT <= SOLO_Q: one per out-edge of the level
+        if (tid == 0) {
+            L.tail[cur ^ 1u] = 0u;
+            L.nbig = 0u;
+            L.act[cur ^ 1u] = 0u; // of the next level's end
+        }
+        uint32_t a = 0;
+        if (n <= SOLO_NACT) {
+            load_level(n);
+#pragma unroll
+            for (uint32_t k = 0; k < SOLO_PER; ++k)
+                a += deg[k];
+        } else
+            for (uint32_t i = tid; i < n; i += SOLO_T)
+                a += rec[2ull * L.q[cur][i]].x;
+        a = wave_sum_dpp(a);
+        if (lane == 0 && a)
+            atomicAdd(&L.act[cur], a);
+        __syncthreads();
+        const unsigned long long A = L.act[cur];
+        st.iters += 1u;
+        st.fiters += 1u;
+        st.unvisited = st.unvisited >= n ? st.unvisited - n : 0ull;
+        const bool stop = A == 0ull || (st.max_iters && st.iters >= st.max_iters);
+        int mode = 0, blog2 = st.g.plain_blog2;
+        if (!mlp) { // every wavefront decides for itself
+            if (!stop)
+                loop_choose_wave(st.g, nullptr, A, n, st.iters, st.unvisited, &mode, &blog2);
+        } else {
+            if (!stop && tid < WG_WAVE) {
+                loop_choose_wave(st.g, L.mlp, A, n, st.iters, st.unvisited, &mode, &blog2);
+                if (tid == 0) {
+                    L.dec[0] = mode;
+                    L.dec[1] = blog2;
+                }
+            }
+            __syncthreads();
+            if (!stop) {
+                mode = L.dec[0];
+                blog2 = L.dec[1];
+            }
+        }
+        if (!stop && mode == WG_MODE_FRONTIER && A <= SOLO_ACT && n <= SOLO_NACT)
+            continue;
+        for (uint32_t i = tid; i < n; i += SOLO_T) // back to next
+            atomicOr((unsigned long long*)&next[L.q[cur][i] >> 6], 1ull << (L.q[cur][i] & 63u));
+        if (tid == 0) {
+            ctr->iters = st.iters;
+            ctr->fiters = st.fiters;
+            ctr->last_activity = A;
+            ctr->last_activated = n;
+            ctr->unvisited = st.unvisited;
+            ctr->level = st.level0 + r + 1u;
+            ctr->run_levels += r + 1u;
+            if (stop) {
+                ctr->done = 1u;
+            } else {
+                ctr->mode = (unsigned int)mode;
+                ctr->blog2 = blog2;
+            }
+        }
+        add_work(work, ctr);
+        return;
+    }
+}
+
+// The decision of a BFS loop with fused levels on a graph with records, and the
+// levels that follow it in this workgroup.
+template <bool CW>
+__global__ __launch_bounds__(SOLO_T) void k_decide_bfs(wg_dev_counters* __restrict__ c, const float* __restrict__ mlp,
+                                                       wg_run_ctl* __restrict__ rc, const uint32_t* __restrict__ csri_off,
+                                                       const uint32_t* __restrict__ csr_dst,
+                                                       const uint4* __restrict__ rec, uint64_t* __restrict__ next,
+                                                       uint64_t* __restrict__ visited, uint64_t* __restrict__ packed,
+                                                       uint64_t nwords, const uint32_t* __restrict__ perm)
+{
+    __shared__ solo_lds L;
+    if (threadIdx.x < WG_WAVE)
+        decide_wave(c, mlp);
+    if (threadIdx.x < 3) {
+        rc->tail[threadIdx.x].v = 0ull;
+        rc->act[threadIdx.x].v = 0ull;
+        rc->nact[threadIdx.x].v = 0ull;
+        rc->fresh[threadIdx.x].v = 0ull;
+    }
+    __syncthreads(); // the control block as the first wavefront left it
+    bfs_solo<CW>(L, csri_off, csr_dst, rec, next, visited, packed, nwords, perm, c, mlp);
 }
 
 // ---- host side ----------------------------------------------------------------------
@@ -1772,6 +2129,15 @@ static int init_common(wg_ctx* ctx, int app)
         if (ctx->E)
             hipLaunchKernelGGL(k_csr_dst, dim3(wg_grid(ctx, ctx->E, 1024, 8)), dim3(256), 0, ctx->stream, ctx->csri_pos,
                                ctx->dst, ctx->E, ctx->csr_dst);
+        if ((rc = wg_check_launch(ctx)))
+            return rc;
+    }
+    // vertex records for the levels of one workgroup, on graphs with few
+    // out-edges per vertex (once per graph; 32 bytes per vertex)
+    if (app == WG_APP_BFS && !ctx->solo_rec && ctx->E <= ctx->V * SOLO_MEAN_DEGREE) {
+        WG_HIP(ctx, hipMalloc((void**)&ctx->solo_rec, ctx->V * 2 * sizeof(uint4)));
+        hipLaunchKernelGGL(k_solo_rec, dim3(wg_grid(ctx, ctx->V, 256, 8)), dim3(256), 0, ctx->stream, ctx->csri_off,
+                           ctx->csr_dst, ctx->V, ctx->solo_rec);
         if ((rc = wg_check_launch(ctx)))
             return rc;
     }
@@ -2301,14 +2667,19 @@ static int enqueue_iteration(wg_ctx* ctx)
     }
     const uint32_t run_wgs = ctx->run_wgs[ctx->app & 7];
     const bool run = run_wgs && ctx->run_q && (ctx->app == WG_APP_BFS || ctx->run_spare);
-    hipLaunchKernelGGL(k_decide, dim3(1), dim3(WG_WAVE), 0, ctx->stream, ctx->ctr, mlp, run ? ctx->run_ctl : nullptr);
+    if (run && ctx->app == WG_APP_BFS && ctx->solo_rec && run_wgs * WG_RUN_NACT_PER_WG >= SOLO_NACT) {
+        hipLaunchKernelGGL(WG_CW(ctx, k_decide_bfs), dim3(1), dim3(SOLO_T), 0, ctx->stream, ctx->ctr, mlp, ctx->run_ctl,
+                           ctx->csri_off, ctx->csr_dst, ctx->solo_rec, ctx->bm_next, ctx->bm_visited, packed,
+                           ctx->bm_words, ctx->perm);
+    } else
+        hipLaunchKernelGGL(k_decide, dim3(1), dim3(WG_WAVE), 0, ctx->stream, ctx->ctr, mlp, run ? ctx->run_ctl : nullptr);
     if (run) {
         const dim3 rg(run_wgs), rb(WG_BLOCK);
         uint4* qb = ctx->run_q + WG_RUN_QCAP;
         if (ctx->app == WG_APP_BFS) {
             hipLaunchKernelGGL(WG_CW(ctx, k_bfs_run), rg, rb, 0, ctx->stream, ctx->csri_off, ctx->csr_dst, ctx->bm_next,
                                ctx->bm_visited, packed, ctx->bm_words, ctx->perm, ctx->run_q, qb, ctx->run_ctl, ctx->ctr,
-                               mlp);
+                               mlp, ctx->solo_rec && run_wgs * WG_RUN_NACT_PER_WG >= SOLO_NACT);
         } else {
 #define WG_MIN_RUN(P, T)                                                                                               \
     hipLaunchKernelGGL(WG_CW(ctx, k_min_run, P), rg, rb, 0, ctx->stream, ctx->csri_off, ctx->csri_pos, ctx->dst, ctx->w,            \
