@@ -267,7 +267,12 @@ int wg_dense_pull_binned(const wg_ctx* ctx, int* on);
  * iteration counts and schedule decisions are unchanged; CC labels and SSSP
  * distances are unchanged, their iteration counts may differ (a
  * frontier-filtered pull reads whole edge blocks, which can settle values in
- * fewer iterations).  Default: BFS with 32 workgroups, CC and SSSP off. */
+ * fewer iterations).  Default: BFS with 32 workgroups, CC and SSSP off.
+ * On graphs with at most 4 edges per vertex, levels that suit one workgroup run
+ * inside the decision kernel: BFS levels of up to 2048 vertices (counted as
+ * fused; with workgroups >= 2), and, unless SSSP is in apps, SSSP rounds that
+ * take the activated vertices nearest first (distances unchanged, each round an
+ * iteration and a frontier iteration). */
 int wg_set_fused_levels(wg_ctx* ctx, uint32_t workgroups, uint32_t apps);
 /* Iterations of the last wg_converge that ran fused (included in its
  * iteration counts). */

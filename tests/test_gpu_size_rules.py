@@ -168,3 +168,52 @@ def test_bfs_levels_in_one_workgroup(name, relabel):
                 assert np.array_equal(W.bfs_depth(got[0][0]), depth), schedule
     finally:
         c.close()
+
+
+def _weighted(g, kind, seed):
+    """g with weights: random, all equal (ties everywhere), or many zeros."""
+    rng = np.random.default_rng(seed)
+    E = g.num_edges
+    w = {"random": rng.integers(1, 1000, E), "equal": np.full(E, 7), "zeros": rng.integers(0, 3, E)}[kind]
+    return w.astype(np.uint32), w.astype(np.float64) * 0.37
+
+
+# at most 4 out-edges per vertex: a grid; a fan of 300 and one of 20000 (more
+# than the near queue holds); random edges (more vertices waiting than one
+# workgroup keeps)
+@pytest.mark.parametrize("kind", ["random", "equal", "zeros"])
+@pytest.mark.parametrize("graph", ["grid", "fan", "wide", "random"])
+def test_sssp_rounds_in_one_workgroup(graph, kind):
+    g = {"grid": lambda: W.grid(61, 83, seed=4), "fan": lambda: _broom(300), "wide": lambda: _broom(20000),
+         "random": lambda: _sparse(200000, 500000, 8)}[graph]()
+    root = 7 if graph == "random" else 0
+    if graph == "grid":
+        root = g.max_outdegree_vertex()
+    for w in _weighted(g, kind, 5):
+        gw = W.Graph(g.offsets, g.sources, w)
+        want = oracle.Oracle.of(gw, 8).sssp(root)[0]
+        c = W.Context(0)
+        try:
+            c.load(gw)
+            for schedule in (W.SCHED_FRONTIER, W.SCHED_PLAIN):
+                c.init_sssp(root)
+                it, _ = c.converge(schedule)
+                got = c.read_sssp()
+                if w.dtype == np.uint32:
+                    got = np.where(got == np.uint32(0xFFFFFFFF), np.uint64(2**64 - 1), got.astype(np.uint64))
+                assert np.array_equal(got, want), (w.dtype, schedule)
+                assert c.validate() == 0 or kind == "zeros"
+                c.init_sssp(root)  # stopped early
+                assert c.converge(schedule, max_iterations=3)[0] == 3
+                c.set_fused_levels(0, (W.APP_SSSP,))  # the same without these rounds
+                c.init_sssp(root)
+                c.converge(schedule)
+                again = c.read_sssp()
+                if w.dtype == np.uint32:
+                    again = np.where(again == np.uint32(0xFFFFFFFF), np.uint64(2**64 - 1), again.astype(np.uint64))
+                assert np.array_equal(again, want), (w.dtype, schedule)
+                c.close()
+                c = W.Context(0)
+                c.load(gw)
+        finally:
+            c.close()

@@ -538,6 +538,8 @@ static void free_graph(wg_ctx* ctx)
     free_dev((void**)&ctx->first_src);
     free_dev((void**)&ctx->csr_dst);
     free_dev((void**)&ctx->solo_rec);
+    free_dev((void**)&ctx->solo_wrec);
+    free_dev((void**)&ctx->solo_far);
     free_dev((void**)&ctx->perm);
     free_dev((void**)&ctx->inv);
     free_dev(&ctx->stage);

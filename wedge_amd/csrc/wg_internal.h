@@ -185,6 +185,9 @@ struct wg_ctx {
                               // built by the first BFS init)
     uint4* solo_rec;          // BFS: out-degree and first destinations of each vertex, on graphs with few
                               // out-edges per vertex (built by the first BFS init)
+    uint4* solo_wrec;         // SSSP: the same with weights (built by the first SSSP init)
+    uint32_t* solo_far;       // SSSP: far lists of the rounds of one workgroup
+    double solo_delta;        // and their first step between cutoffs
     uint32_t* bfs_heavy_v;
     uint32_t* bfs_heavy_e;    // chunk start edge (chunk end = min(start + WG_BFS_HEAVY, off[v+1]))
     uint32_t n_out_pos;       // vertices with out-degree > 0
@@ -249,6 +252,7 @@ struct wg_ctx {
     struct wg_members* members;      // batch of member graphs (wg_set_members), NULL if none
     // fused small-frontier levels of the device loop (k_bfs_run)
     uint32_t run_wgs[8];      // workgroups of a run, by WG_APP_*, 0 = off
+    uint32_t run_set;         // bit per application: wg_set_fused_levels was called for it
     struct wg_run_ctl* run_ctl;
     uint4* run_q;             // two queues of WG_RUN_QCAP entries
     uint64_t* run_spare;      // CC / SSSP runs: second activation mask (bm_words), zero between runs

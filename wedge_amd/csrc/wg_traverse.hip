@@ -1754,7 +1754,19 @@ __device__ __forceinline__ unsigned long long solo_load(const uint64_t* p)
     return __hip_atomic_load((const unsigned long long*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Appends the vertices v[j] with put[j] set to the LDS queue: one LDS atomic
+template <typename T>
+__device__ __forceinline__ T solo_load_t(const T* p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ T opaque_t(T x)
+{
+    asm volatile("" : "+v"(x));
+    return x;
+}
+
+// Appends the vertices v[j] with put[j] set to the queue q: one LDS atomic
 // per wavefront.  Called by the lanes of a wavefront that are active together;
 // entries past the queue's end are not written (the caller sees the tail).
 template <int N>
@@ -2041,6 +2053,432 @@ __global__ __launch_bounds__(SOLO_T) void k_decide_bfs(wg_dev_counters* __restri
     bfs_solo<CW>(L, csri_off, csr_dst, rec, next, visited, packed, nwords, perm, c, mlp);
 }
 
+// ---- SSSP in one workgroup ----------------------------------------------------------
+//
+// On road-like graphs a frontier-filtered pull of SSSP relaxes in no order of
+// distance: vertices are lowered again and again (4096x6144 grid: each edge read
+// 64 times), by a few wavefronts that own the marked words.  Here the
+// decision kernel's workgroup goes on as for BFS, nearest vertices first: the
+// near queue (LDS) holds activated vertices within the cutoff distance, the far
+// list (global) the others; a round relaxes the near queue's out-edges, and when
+// no near vertex is left the cutoff moves past the nearest far one.  A vertex
+// whose distance falls is put on one of the two every time, so the fixpoint is
+// that of the pulls.  The step between cutoffs follows the size of the rounds
+// (about a vertex per thread: wide enough to fill the workgroup, no wider, since
+// vertices relaxed too early are relaxed again).  SOLO_PENDING waiting vertices
+// are work for the whole device: the loop's pulls go on from there.
+#define SOLO_NEAR 16384u     // near queue entries
+#define SOLO_PENDING 32768u  // far list entries (about) at which the workgroup hands back
+#define SOLO_FAR (1u << 20)  // capacity of each of the two far lists
+#define SOLO_SBIG 2048u
+#define SOLO_SNACT 16384u    // entered with at most so many activated vertices
+#define SOLO_SACT 65536u     // and out-edges
+#define SOLO_ROUNDS 16384u   // rounds per launch
+
+// A vertex's record: 64 bytes, its out-degree, first REC destinations, weights.
+template <class P>
+struct solo_pol;
+template <>
+struct solo_pol<PolSU> {
+    typedef uint32_t W;
+    static constexpr uint32_t REC = 7, WAT = 9; // word of the first weight
+    __device__ static uint32_t add(uint32_t d, uint32_t w, unsigned int* ovf)
+    {
+        const uint32_t s = d + w;
+        if (s < d || s == PolSU::INF) {
+            *ovf = 1u;
+            return PolSU::INF;
+        }
+        return s;
+    }
+    __device__ static uint32_t step(uint32_t d, double delta)
+    {
+        const double x = (double)d + delta;
+        return x < 4294967294.0 ? (uint32_t)x : PolSU::INF - 1u;
+    }
+};
+template <>
+struct solo_pol<PolSF> {
+    typedef unsigned long long W; // the weight's bits
+    static constexpr uint32_t REC = 5, WAT = 6;
+    __device__ static unsigned long long add(unsigned long long d, unsigned long long w, unsigned int*)
+    {
+        return (unsigned long long)__double_as_longlong(__longlong_as_double((long long)d) +
+                                                        __longlong_as_double((long long)w));
+    }
+    __device__ static unsigned long long step(unsigned long long d, double delta)
+    {
+        return (unsigned long long)__double_as_longlong(__longlong_as_double((long long)d) + delta);
+    }
+};
+
+template <class P>
+__global__ void k_solo_wrec(const uint32_t* __restrict__ csri_off, const uint32_t* __restrict__ csri_pos,
+                            const uint32_t* __restrict__ dst, const typename solo_pol<P>::W* __restrict__ w, uint64_t V,
+                            uint4* __restrict__ rec)
+{
+    typedef solo_pol<P> S;
+    for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < V; v += (uint64_t)gridDim.x * blockDim.x) {
+        const uint32_t s = csri_off[v], d = csri_off[v + 1] - s;
+        union {
+            uint4 q[4];
+            uint32_t x[16];
+        } r = {};
+        r.x[0] = d;
+        for (uint32_t j = 0; j < S::REC && j < d; ++j) {
+            const uint32_t p = csri_pos[s + j];
+            const unsigned long long b = (unsigned long long)w[p];
+            r.x[1 + j] = dst[p];
+            if (sizeof(typename S::W) == 8) {
+                r.x[S::WAT + 2 * j] = (uint32_t)b;
+                r.x[S::WAT + 2 * j + 1] = (uint32_t)(b >> 32);
+            } else
+                r.x[S::WAT + j] = (uint32_t)b;
+        }
+        for (int k = 0; k < 4; ++k)
+            rec[4 * v + k] = r.q[k];
+    }
+}
+
+// Mean weight (FP64, any order: it only sets the first step between cutoffs).
+template <typename W>
+__global__ __launch_bounds__(WG_BLOCK) void k_weight_sum(const W* __restrict__ w, uint64_t E, double* __restrict__ sum)
+{
+    double a = 0.0;
+    for (uint64_t e = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; e < E; e += (uint64_t)gridDim.x * blockDim.x)
+        a += (double)w[e];
+    a = wg_wave_sum(a);
+    if (wg_lane() == 0)
+        atomicAdd(sum, a);
+}
+
+template <typename T>
+struct sssp_lds {
+    uint32_t q[2][SOLO_NEAR];
+    uint32_t tail[2], ftail[2];
+    uint32_t nbig, big[SOLO_SBIG];
+    unsigned long long act, fresh; // at the end: out-edges of the waiting vertices, vertices first reached
+    T least;                       // smallest distance left on the far list
+};
+
+// Puts the improved destinations v[j] (new value m[j]) on the near queue or the
+// far list; one that finds no room goes back to next.
+template <int N, typename T>
+__device__ __forceinline__ void sssp_put(sssp_lds<T>& L, uint32_t nxt, uint32_t* __restrict__ far, uint32_t fi,
+                                         const uint32_t* v, const T* m, const bool* up, T cutoff,
+                                         uint64_t* __restrict__ next)
+{
+    bool near[N], away[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        near[j] = up[j] && m[j] <= cutoff;
+        away[j] = up[j] && m[j] > cutoff;
+    }
+    solo_append<N>(L.q[nxt], &L.tail[nxt], SOLO_NEAR, v, near);
+    solo_append<N>(far, &L.ftail[fi], SOLO_FAR, v, away);
+    // past the end of either (the tails say so): all of these, rather than sort out which
+    if (L.tail[nxt] > SOLO_NEAR || L.ftail[fi] > SOLO_FAR) {
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+            if (up[j])
+                atomicOr((unsigned long long*)&next[v[j] >> 6], 1ull << (v[j] & 63u));
+    }
+}
+
+template <bool CW, class P>
+__device__ void sssp_solo(sssp_lds<typename P::T>& L, const uint32_t* __restrict__ csri_off,
+                          const uint32_t* __restrict__ csri_pos, const uint32_t* __restrict__ dst,
+                          const typename solo_pol<P>::W* __restrict__ w, const uint4* __restrict__ rec,
+                          typename P::T* __restrict__ prop, uint64_t* __restrict__ next, uint64_t nwords,
+                          uint32_t* __restrict__ far0, double delta, wg_dev_counters* __restrict__ ctr,
+                          unsigned int* __restrict__ ovf, const float* __restrict__ mlp)
+{
+    typedef typename P::T T;
+    typedef solo_pol<P> S;
+    if (ctr->done || ctr->mode != WG_MODE_FRONTIER || ctr->last_activity > SOLO_SACT || ctr->last_activated > SOLO_SNACT)
+        return;
+    run_state st;
+    st.g = read_cfg(ctr);
+    st.max_iters = ctr->max_iters;
+    st.iters = ctr->iters;
+    st.fiters = ctr->fiters;
+    st.unvisited = ctr->unvisited;
+    const uint32_t tid = threadIdx.x;
+    const int lane = wg_lane();
+    uint32_t* far[2] = {far0, far0 + SOLO_FAR};
+    if (tid < 2) {
+        L.tail[tid] = 0u;
+        L.ftail[tid] = 0u;
+    }
+    if (tid == 0) {
+        L.nbig = 0u;
+        L.act = 0ull;
+        L.fresh = 0ull;
+        L.least = P::INF;
+    }
+    __syncthreads();
+    // the activated set leaves next for the far list (at most SOLO_SNACT)
+    for (uint64_t w0 = tid; w0 < nwords; w0 += (uint64_t)WG_RUN_SCAN_BATCH * SOLO_T) {
+        uint64_t x[WG_RUN_SCAN_BATCH];
+#pragma unroll
+        for (int j = 0; j < WG_RUN_SCAN_BATCH; ++j) {
+            const uint64_t wd = w0 + (uint64_t)j * SOLO_T;
+            x[j] = (wd < nwords) ? next[wd] : 0ull;
+        }
+#pragma unroll
+        for (int j = 0; j < WG_RUN_SCAN_BATCH; ++j)
+            if (x[j]) {
+                const uint64_t wd = w0 + (uint64_t)j * SOLO_T;
+                next[wd] = 0ull;
+                for (uint64_t b = x[j]; b; b &= b - 1ull) {
+                    const uint32_t i = atomicAdd(&L.ftail[0], 1u);
+                    if (i < SOLO_FAR)
+                        far[0][i] = (uint32_t)(wd * 64u + (uint64_t)(__ffsll((long long)b) - 1));
+                }
+            }
+    }
+    __syncthreads();
+    uint32_t cur = 0, fi = 0; // near queue being relaxed, far list being filled
+    bool started = false;
+    T cutoff = T(0);
+    uint32_t n = 0, rounds = 0, phase_rounds = 0, phase_n = 0;
+    unsigned long long fresh = 0ull;
+    work_tally<CW> work;
+    bool stop = false, full = false; // full: vertices went back to next for want of room
+    const uint32_t aim = st.g.nv / 64u < SOLO_T ? (uint32_t)(st.g.nv / 64u) + 1u : SOLO_T;
+    for (;;) {
+        if (n == 0u) { // the next cutoff
+            uint32_t nf = L.ftail[fi];
+            nf = nf < SOLO_FAR ? nf : SOLO_FAR;
+            if (nf == 0u) {
+                stop = true;
+                break;
+            }
+            if (phase_rounds) { // a vertex per thread and round, on small graphs fewer
+                if (phase_n < phase_rounds * aim / 2u)
+                    delta *= 1.5;
+                else if (phase_n > phase_rounds * aim / 2u * 3u)
+                    delta *= 0.6;
+            }
+            phase_rounds = phase_n = 0u;
+            // past the last cutoff first; if that finds none, past the nearest
+            T to = started ? S::step(cutoff, delta) : T(0);
+            bool none = false;
+            for (int pass = started ? 0 : 1; pass < 2; ++pass) {
+                if (pass == 1) {
+                    T m = P::INF;
+                    for (uint32_t i = tid; i < nf; i += SOLO_T) {
+                        const T d = solo_load_t(&prop[far[fi][i]]);
+                        if ((!started || d > cutoff) && d < m)
+                            m = d;
+                    }
+                    m = wg_wave_min(m);
+                    if (lane == 0 && m < P::INF)
+                        atomicMin(&L.least, m);
+                    __syncthreads();
+                    none = L.least == P::INF;
+                    to = none ? cutoff : S::step(L.least, delta);
+                    __syncthreads();
+                    if (tid == 0)
+                        L.least = P::INF;
+                }
+                // far entries: those at or below the last cutoff (on the near queue
+                // since they fell there) leave, near ones move, the others stay
+                for (uint32_t i0 = tid & ~63u; i0 < nf; i0 += SOLO_T) {
+                    const uint32_t i = i0 + (uint32_t)lane;
+                    uint32_t v[1] = {0u};
+                    T m[1] = {P::INF};
+                    bool up[1] = {false};
+                    if (i < nf) {
+                        v[0] = far[fi][i];
+                        m[0] = solo_load_t(&prop[v[0]]);
+                        up[0] = !started || m[0] > cutoff;
+                    }
+                    sssp_put<1, T>(L, cur, far[fi ^ 1u], fi ^ 1u, v, m, up, to, next);
+                }
+                __syncthreads();
+                n = L.tail[cur];
+                nf = L.ftail[fi ^ 1u];
+                full = full || n > SOLO_NEAR || nf > SOLO_FAR;
+                n = n < SOLO_NEAR ? n : SOLO_NEAR;
+                nf = nf < SOLO_FAR ? nf : SOLO_FAR;
+                __syncthreads();
+                if (tid == 0)
+                    L.ftail[fi] = 0u;
+                fi ^= 1u;
+                __syncthreads();
+                if (n || nf == 0u)
+                    break;
+            }
+            cutoff = to;
+            started = true;
+            if (full)
+                break;
+            if (n == 0u) { // every entry was settled
+                stop = true;
+                break;
+            }
+        }
+        // one round: the near queue's out-edges
+        const uint32_t nxt = cur ^ 1u;
+        uint32_t edges = 0;
+        for (uint32_t i0 = tid & ~63u; i0 < n; i0 += SOLO_T) { // uniform per wavefront
+            const uint32_t i = i0 + (uint32_t)lane;
+            uint32_t x[16] = {};
+            uint32_t deg = 0;
+            T du = T(0);
+            if (i < n) {
+                const uint32_t u = L.q[cur][i];
+                const uint4* r = rec + 4ull * u;
+                du = solo_load_t(&prop[u]);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const uint4 y = r[k];
+                    x[4 * k] = y.x;
+                    x[4 * k + 1] = y.y;
+                    x[4 * k + 2] = y.z;
+                    x[4 * k + 3] = y.w;
+                }
+                deg = x[0];
+                edges += deg;
+                if (deg > S::REC) { // left to a wavefront
+                    const uint32_t b = atomicAdd(&L.nbig, 1u);
+                    if (b < SOLO_SBIG)
+                        L.big[b] = u;
+                    else // no room: its own thread would be too slow, back to next
+                        atomicOr((unsigned long long*)&next[u >> 6], 1ull << (u & 63u));
+                    deg = 0u;
+                }
+            }
+            T m[S::REC], old[S::REC];
+            uint32_t v[S::REC];
+            bool up[S::REC];
+#pragma unroll
+            for (uint32_t j = 0; j < S::REC; ++j) {
+                v[j] = x[1 + j];
+                unsigned long long b = x[S::WAT + j];
+                if (sizeof(typename S::W) == 8)
+                    b = (unsigned long long)x[S::WAT + 2 * j] | ((unsigned long long)x[S::WAT + 2 * j + 1] << 32);
+                m[j] = j < deg ? S::add(du, (typename S::W)b, ovf) : P::INF;
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < S::REC; ++j) {
+                old[j] = opaque_t(T(0));
+                if (m[j] < P::INF) {
+                    work.dests += 1ull;
+                    old[j] = atomic_min_t<T>(&prop[v[j]], m[j]);
+                }
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < S::REC; ++j) {
+                up[j] = old[j] > m[j];
+                fresh += up[j] && old[j] == P::INF ? 1ull : 0ull;
+            }
+            sssp_put<S::REC, T>(L, nxt, far[fi], fi, v, m, up, cutoff, next);
+        }
+        __syncthreads();
+        if (const uint32_t nb = L.nbig < SOLO_SBIG ? L.nbig : SOLO_SBIG) { // the same in the whole workgroup
+            for (uint32_t b = tid / WG_WAVE; b < nb; b += SOLO_WAVES) {
+                const uint32_t u = L.big[b], e = csri_off[u + 1];
+                const T du = solo_load_t(&prop[u]);
+                for (uint32_t c = csri_off[u]; c < e; c += WG_WAVE) {
+                    uint32_t v[1] = {0u};
+                    T m[1] = {P::INF};
+                    bool up[1] = {false};
+                    if (c + (uint32_t)lane < e) {
+                        const uint32_t p = csri_pos[c + (uint32_t)lane];
+                        v[0] = dst[p];
+                        m[0] = S::add(du, w[p], ovf);
+                        if (m[0] < P::INF) {
+                            work.dests += 1ull;
+                            const T old = atomic_min_t<T>(&prop[v[0]], m[0]);
+                            up[0] = old > m[0];
+                            fresh += up[0] && old == P::INF ? 1ull : 0ull;
+                        }
+                    }
+                    sssp_put<1, T>(L, nxt, far[fi], fi, v, m, up, cutoff, next);
+                }
+            }
+            __syncthreads();
+        }
+        work.edges += edges;
+        phase_rounds += 1u;
+        phase_n += n;
+        rounds += 1u;
+        st.iters += 1u;
+        st.fiters += 1u;
+        full = L.tail[nxt] > SOLO_NEAR || L.ftail[fi] > SOLO_FAR || L.nbig > SOLO_SBIG;
+        n = L.tail[nxt];
+        n = n < SOLO_NEAR ? n : SOLO_NEAR;
+        const uint32_t nf = L.ftail[fi];
+        __syncthreads(); // all have read the tails
+        if (tid == 0) {
+            L.tail[cur] = 0u;
+            L.nbig = 0u;
+        }
+        cur = nxt;
+        __syncthreads();
+        if (full || nf > SOLO_PENDING || rounds >= SOLO_ROUNDS || (st.max_iters && st.iters >= st.max_iters))
+            break;
+    }
+    // what waits goes back to next, counted as the pulls count it (a vertex that
+    // is listed twice counts twice: these counts only choose the next pull)
+    const uint32_t nf = L.ftail[fi] < SOLO_FAR ? L.ftail[fi] : SOLO_FAR;
+    uint32_t a = 0;
+    for (uint32_t i = tid; i < n + nf; i += SOLO_T) {
+        const uint32_t v = i < n ? L.q[cur][i] : far[fi][i - n];
+        atomicOr((unsigned long long*)&next[v >> 6], 1ull << (v & 63u));
+        a += rec[4ull * v].x;
+    }
+    a = wave_sum_dpp(a);
+    const uint32_t f = wave_sum_dpp((uint32_t)fresh);
+    if (lane == 0) {
+        if (a)
+            atomicAdd(&L.act, (unsigned long long)a);
+        if (f)
+            atomicAdd(&L.fresh, (unsigned long long)f);
+    }
+    __syncthreads();
+    const unsigned long long A = L.act, F = L.fresh;
+    st.unvisited = st.unvisited >= F ? st.unvisited - F : 0ull;
+    stop = stop || (A == 0ull && !full) || (st.max_iters && st.iters >= st.max_iters);
+    int mode = 0, blog2 = st.g.plain_blog2;
+    if (!stop && tid < WG_WAVE)
+        loop_choose_wave(st.g, mlp, A, n + nf, st.iters, st.unvisited, &mode, &blog2);
+    if (tid == 0) {
+        ctr->iters = st.iters;
+        ctr->fiters = st.fiters;
+        ctr->last_activity = A;
+        ctr->last_activated = n + nf;
+        ctr->unvisited = st.unvisited;
+        if (stop) {
+            ctr->done = 1u;
+        } else {
+            ctr->mode = (unsigned int)mode;
+            ctr->blog2 = blog2;
+        }
+    }
+    add_work(work, ctr);
+}
+
+template <bool CW, class P>
+__global__ __launch_bounds__(SOLO_T) void k_decide_sssp(wg_dev_counters* __restrict__ c, const float* __restrict__ mlp,
+                                                        const uint32_t* __restrict__ csri_off,
+                                                        const uint32_t* __restrict__ csri_pos,
+                                                        const uint32_t* __restrict__ dst, const void* __restrict__ w,
+                                                        const uint4* __restrict__ rec, typename P::T* __restrict__ prop,
+                                                        uint64_t* __restrict__ next, uint64_t nwords,
+                                                        uint32_t* __restrict__ far, double delta,
+                                                        unsigned int* __restrict__ ovf)
+{
+    __shared__ sssp_lds<typename P::T> L;
+    if (threadIdx.x < WG_WAVE)
+        decide_wave(c, mlp);
+    __syncthreads(); // the control block as the first wavefront left it
+    sssp_solo<CW, P>(L, csri_off, csri_pos, dst, (const typename solo_pol<P>::W*)w, rec, prop, next, nwords, far, delta, c,
+                     ovf, mlp);
+}
+
 // ---- host side ----------------------------------------------------------------------
 
 // The instance of a pull kernel with (CW = true) or without the work counts.
@@ -2095,6 +2533,47 @@ static int clear_wedge_state(wg_ctx* ctx)
     return rc;
 }
 
+// Vertex records, far lists and the mean weight for the SSSP rounds of one
+// workgroup (once per graph; 64 bytes per vertex and 8 MiB).
+static int build_solo_sssp(wg_ctx* ctx)
+{
+    double *sum = nullptr, total = 0.0;
+    WG_HIP(ctx, hipMalloc((void**)&sum, sizeof(double)));
+    uint4* rec = nullptr;
+    if (!ctx->solo_far && hipMalloc((void**)&ctx->solo_far, 2ull * SOLO_FAR * sizeof(uint32_t)) != hipSuccess)
+        ctx->solo_far = nullptr;
+    hipError_t e = ctx->solo_far ? hipMalloc((void**)&rec, ctx->V * 4 * sizeof(uint4)) : hipErrorOutOfMemory;
+    if (e == hipSuccess) {
+        const dim3 gv(wg_grid(ctx, ctx->V, 256, 8)), ge(wg_grid(ctx, ctx->E, 4096, 4)), blk(WG_BLOCK);
+        const uint64_t one = 0;
+        (void)hipMemcpyAsync(sum, &one, sizeof(double), hipMemcpyHostToDevice, ctx->stream);
+        if (ctx->wkind == WG_WEIGHT_F64) {
+            hipLaunchKernelGGL(k_solo_wrec<PolSF>, gv, blk, 0, ctx->stream, ctx->csri_off, ctx->csri_pos, ctx->dst,
+                               (const unsigned long long*)ctx->w, ctx->V, rec);
+            hipLaunchKernelGGL(k_weight_sum<double>, ge, blk, 0, ctx->stream, (const double*)ctx->w, ctx->E, sum);
+        } else {
+            hipLaunchKernelGGL(k_solo_wrec<PolSU>, gv, blk, 0, ctx->stream, ctx->csri_off, ctx->csri_pos, ctx->dst,
+                               (const uint32_t*)ctx->w, ctx->V, rec);
+            hipLaunchKernelGGL(k_weight_sum<uint32_t>, ge, blk, 0, ctx->stream, (const uint32_t*)ctx->w, ctx->E, sum);
+        }
+        e = hipGetLastError();
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(&total, sum, sizeof(double), hipMemcpyDeviceToHost, ctx->stream);
+        const hipError_t e2 = hipStreamSynchronize(ctx->stream);
+        e = e == hipSuccess ? e2 : e;
+    }
+    (void)hipFree(sum);
+    if (e != hipSuccess) {
+        (void)hipFree(rec);
+        ctx->last_hip_error = (int)e;
+        return WG_E_HIP;
+    }
+    ctx->solo_wrec = rec;
+    const double mean = total / (double)ctx->E;
+    ctx->solo_delta = mean > 0.0 && mean < 1e300 ? 4.0 * mean : 1.0;
+    return WG_OK;
+}
+
 static int init_common(wg_ctx* ctx, int app)
 {
     if (!ctx || !ctx->off)
@@ -2132,6 +2611,9 @@ static int init_common(wg_ctx* ctx, int app)
         if ((rc = wg_check_launch(ctx)))
             return rc;
     }
+    if (app == WG_APP_SSSP && !ctx->solo_wrec && !wg_pb_min_on(ctx) && ctx->E &&
+        ctx->E <= ctx->V * SOLO_MEAN_DEGREE && (rc = build_solo_sssp(ctx)))
+        return rc;
     // vertex records for the levels of one workgroup, on graphs with few
     // out-edges per vertex (once per graph; 32 bytes per vertex)
     if (app == WG_APP_BFS && !ctx->solo_rec && ctx->E <= ctx->V * SOLO_MEAN_DEGREE) {
@@ -2671,6 +3153,16 @@ static int enqueue_iteration(wg_ctx* ctx)
         hipLaunchKernelGGL(WG_CW(ctx, k_decide_bfs), dim3(1), dim3(SOLO_T), 0, ctx->stream, ctx->ctr, mlp, ctx->run_ctl,
                            ctx->csri_off, ctx->csr_dst, ctx->solo_rec, ctx->bm_next, ctx->bm_visited, packed,
                            ctx->bm_words, ctx->perm);
+    } else if (ctx->app == WG_APP_SSSP && ctx->solo_wrec && !((ctx->run_set >> WG_APP_SSSP) & 1u) && !wg_pb_min_on(ctx)) {
+#define WG_DECIDE_SSSP(P, T)                                                                                           \
+    hipLaunchKernelGGL(WG_CW(ctx, k_decide_sssp, P), dim3(1), dim3(SOLO_T), 0, ctx->stream, ctx->ctr, mlp,             \
+                       ctx->csri_off, ctx->csri_pos, ctx->dst, ctx->w, ctx->solo_wrec, (T*)ctx->prop[0], ctx->bm_next, \
+                       ctx->bm_words, ctx->solo_far, ctx->solo_delta, &ctx->ctr->overflow)
+        if (ctx->wkind == WG_WEIGHT_F64)
+            WG_DECIDE_SSSP(PolSF, unsigned long long);
+        else
+            WG_DECIDE_SSSP(PolSU, uint32_t);
+#undef WG_DECIDE_SSSP
     } else
         hipLaunchKernelGGL(k_decide, dim3(1), dim3(WG_WAVE), 0, ctx->stream, ctx->ctr, mlp, run ? ctx->run_ctl : nullptr);
     if (run) {
@@ -2714,6 +3206,7 @@ extern "C" int wg_set_fused_levels(wg_ctx* ctx, uint32_t workgroups, uint32_t ap
     for (int a = 0; a < 8; ++a)
         if ((apps >> a) & 1u)
             ctx->run_wgs[a] = workgroups;
+    ctx->run_set |= apps;
     return WG_OK;
 }
 
