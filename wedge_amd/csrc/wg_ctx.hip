@@ -494,7 +494,22 @@ int wg_free_app_state(wg_ctx* ctx)
     free_dev((void**)&ctx->roots);
     free_dev((void**)&ctx->root_off);
     ctx->nroots = 0;
+    ctx->roots_cap = 0;
+    ctx->prop_bytes = 0;
     ctx->app = WG_APP_NONE;
+    return WG_OK;
+}
+
+int wg_app_state(wg_ctx* ctx, int app, size_t bytes, int both)
+{
+    if (ctx->app == app && ctx->prop_bytes == bytes && ctx->prop[0] && (!both || ctx->prop[1]))
+        return WG_OK;
+    WG_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    wg_free_app_state(ctx);
+    WG_HIP(ctx, hipMalloc(&ctx->prop[0], bytes));
+    if (both)
+        WG_HIP(ctx, hipMalloc(&ctx->prop[1], bytes));
+    ctx->prop_bytes = bytes;
     return WG_OK;
 }
 

@@ -151,6 +151,7 @@ __device__ inline void fold_counts(wg_dev_counters* c, unsigned long long* tot =
 #define RST_OVERFLOW 8u
 #define RST_HEAVY 16u
 #define RST_WORK 32u
+#define RST_REACHED 64u
 
 // Lane -> (marked block, edge) mapping shared by the frontier pulls.
 struct block_walk {

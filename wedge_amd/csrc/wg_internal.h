@@ -198,6 +198,7 @@ struct wg_ctx {
     // application state
     int app;
     void* prop[2];            // PR contributions (double buffer) / BFS packed / CC labels / SSSP dist
+    size_t prop_bytes;        // bytes of prop[0] (and prop[1]) as wg_app_state allocated them
     void* ms[4];              // batched sources: per-vertex masks or rows (freed with the app state)
     uint32_t ms_n;            // batched sources: number of roots / seeds
     bool ms_nl_clean;         // 64-source BFS: nl is all zero (the last run completed)
@@ -241,12 +242,11 @@ struct wg_ctx {
     wg_dev_counters* ctr;     // device
     wg_dev_counters* hctr;    // pinned host mirror
     wg_dev_counters* hctr_dev; // the mirror's device address (null if it has none)
-    uint32_t root_dev;        // BFS / SSSP root in device numbering (the first root)
     uint32_t* roots;          // BFS / SSSP roots in device numbering, distinct
-    uint32_t* root_off;       // BFS, at most WG_PUSH_ROOTS_MAX roots: exclusive prefix of the roots'
-                              // out-degrees (nroots + 1 entries), for the first level's push
+    uint32_t* root_off;       // exclusive prefix of the roots' out-degrees (nroots + 1 entries): for the first
+                              // level's push, and the activity a traversal starts with
     uint32_t nroots;
-    unsigned long long root_activity; // summed out-degree of the roots
+    uint32_t roots_cap;       // roots the two arrays have room for
     int roots_frontier;       // the BFS frontier is still the roots (no pull or advance since the init)
     uint32_t push_roots;      // roots the running wg_converge pushes on its first level (0: none)
     struct wg_members* members;      // batch of member graphs (wg_set_members), NULL if none
@@ -353,6 +353,9 @@ uint32_t wg_wedge_build_grid(const wg_ctx* ctx);
 uint32_t wg_advance_grid(const wg_ctx* ctx);
 int wg_pr_reset(wg_ctx* ctx);
 int wg_free_app_state(wg_ctx* ctx);
+// prop[0] (and prop[1] if `both`) of `bytes` for the application, kept if it is
+// the one whose state the context holds; else everything is released first
+int wg_app_state(wg_ctx* ctx, int app, size_t bytes, int both);
 int wg_alloc_bitmasks(wg_ctx* ctx);
 int wg_clear_u64(wg_ctx* ctx, uint64_t* p, uint64_t words);
 int wg_fill_u32(wg_ctx* ctx, uint32_t* p, uint64_t n, uint32_t value);

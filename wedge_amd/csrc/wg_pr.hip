@@ -69,8 +69,13 @@ __global__ __launch_bounds__(WG_BLOCK) void k_pr_vertex(const double* __restrict
 }
 
 template <typename T>
-__global__ void k_pr_init(const uint32_t* __restrict__ od, T* __restrict__ c, uint64_t V, double N)
+__global__ void k_pr_init(const uint32_t* __restrict__ od, T* __restrict__ c, uint64_t V, double N, double s1,
+                          wg_dev_counters* __restrict__ ctr)
 {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        ctr->S[0] = s1;
+        ctr->ticket = 0u;
+    }
     for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < V; v += (uint64_t)gridDim.x * blockDim.x) {
         const uint32_t o = od[v];
         c[v] = (T)((1.0 / N) / (o ? (double)o : N));
@@ -98,11 +103,10 @@ extern "C" int wg_init_pr(wg_ctx* ctx, double damping, int contrib_fp32)
     if (!(damping >= 0.0 && damping <= 1.0))
         return WG_E_INVAL;
     WG_HIP(ctx, hipSetDevice(ctx->device));
-    WG_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    wg_free_app_state(ctx);
     const size_t esz = contrib_fp32 ? sizeof(float) : sizeof(double);
-    WG_HIP(ctx, hipMalloc(&ctx->prop[0], ctx->V * esz));
-    WG_HIP(ctx, hipMalloc(&ctx->prop[1], ctx->V * esz));
+    int rc = wg_app_state(ctx, WG_APP_PR, ctx->V * esz, 1);
+    if (rc)
+        return rc;
     ctx->app = WG_APP_PR;
     ctx->pr_fp32 = contrib_fp32 ? 1 : 0;
     ctx->damping = damping;
@@ -111,19 +115,15 @@ extern "C" int wg_init_pr(wg_ctx* ctx, double damping, int contrib_fp32)
     ctx->iter = 0;
     const double N = (double)ctx->V;
     const uint32_t grid = wg_grid(ctx, ctx->V, 1024, 8);
-    if (ctx->pr_fp32)
-        hipLaunchKernelGGL(k_pr_init<float>, dim3(grid), dim3(256), 0, ctx->stream, ctx->od, (float*)ctx->prop[0], ctx->V, N);
-    else
-        hipLaunchKernelGGL(k_pr_init<double>, dim3(grid), dim3(256), 0, ctx->stream, ctx->od, (double*)ctx->prop[0], ctx->V, N);
-    int rc = wg_check_launch(ctx);
-    if (rc)
-        return rc;
     // sum over vertices with out-degree > 0 of the initial rank 1/N
     const double s1 = (double)ctx->n_out_pos * (1.0 / N);
-    WG_HIP(ctx, hipMemcpyAsync(&ctx->ctr->S[0], &s1, sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-    WG_HIP(ctx, hipMemsetAsync(&ctx->ctr->ticket, 0, sizeof(unsigned int), ctx->stream));
-    WG_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    return WG_OK;
+    if (ctx->pr_fp32)
+        hipLaunchKernelGGL(k_pr_init<float>, dim3(grid), dim3(256), 0, ctx->stream, ctx->od, (float*)ctx->prop[0], ctx->V, N,
+                           s1, ctx->ctr);
+    else
+        hipLaunchKernelGGL(k_pr_init<double>, dim3(grid), dim3(256), 0, ctx->stream, ctx->od, (double*)ctx->prop[0], ctx->V,
+                           N, s1, ctx->ctr);
+    return wg_check_launch(ctx);
 }
 
 // The tiling and launch shape of the PageRank edge pull.

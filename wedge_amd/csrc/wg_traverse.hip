@@ -72,6 +72,10 @@ __global__ void k_reset(wg_dev_counters* c, unsigned int flags)
             c->edges_read = 0ull;
             c->dests_examined = 0ull;
         }
+        if (flags & RST_REACHED) {
+            c->reached_verts = 0ull;
+            c->reached_edges = 0ull;
+        }
     }
 }
 
@@ -872,13 +876,6 @@ __global__ void k_or_bit(uint64_t* bm, uint32_t v)
     bm[v >> 6] |= 1ull << (v & 63);
 }
 
-// label[v] = original id of v
-__global__ void k_iota_u32(uint32_t* p, uint64_t n, const uint32_t* __restrict__ perm)
-{
-    for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
-        p[i] = perm ? perm[i] : (uint32_t)i;
-}
-
 // ---- device-resident iteration loop ------------------------------------------------
 
 #define LOOP_SCHED_PLAIN 0u
@@ -951,15 +948,22 @@ __device__ __forceinline__ void loop_choose_wave(const loop_cfg& g, const float*
 }
 
 // One wavefront.  initial_vertices / initial_activity describe the state
-// before the first pull (the root, or every vertex for CC).
+// before the first pull (the root, or every vertex for CC; activity_dev: the
+// activity is there).
 __global__ void k_loop_init(wg_dev_counters* c, const float* __restrict__ mlp, unsigned int sched,
                             unsigned long long threshold, int plain_blog2, unsigned int max_iters,
-                            unsigned long long initial_activity, unsigned long long initial_vertices, int dense_first,
+                            unsigned long long initial_activity, const uint32_t* __restrict__ activity_dev,
+                            wg_run_ctl* __restrict__ rc, unsigned long long initial_vertices, int dense_first,
                             unsigned long long unvisited, unsigned int app, unsigned long long nv, unsigned long long ne,
                             unsigned int binned)
 {
     if (blockIdx.x != 0 || threadIdx.x >= WG_WAVE)
         return;
+    if (rc) // control block of the fused runs
+        for (uint32_t i = threadIdx.x; i < sizeof(wg_run_ctl) / 8; i += WG_WAVE)
+            ((unsigned long long*)rc)[i] = 0ull;
+    if (activity_dev)
+        initial_activity = *activity_dev;
     loop_cfg g;
     g.sched = sched;
     g.app = app;
@@ -1386,6 +1390,7 @@ __device__ __forceinline__ bool run_stage_model(const float* __restrict__ mlp, c
 // Each thread reads 16 words at a time, strided by the grid, so that the
 // loads are coalesced and many are in flight.
 #define WG_RUN_SCAN_BATCH 16
+#define WG_RUN_BIG 512u
 __device__ void run_entry(const uint64_t* __restrict__ act, uint64_t nwords, const uint32_t* __restrict__ csri_off,
                           uint4* __restrict__ q, wg_run_ctl* __restrict__ rc)
 {
@@ -1406,11 +1411,14 @@ __device__ void run_entry(const uint64_t* __restrict__ act, uint64_t nwords, con
                 k += run_entries(csri_off[v + 1] - csri_off[v]);
             }
     }
-    __shared__ uint32_t s_base;
+    __shared__ uint32_t s_base, s_nbig;
+    __shared__ uint2 s_big[WG_RUN_BIG]; // vertices with long lists: {vertex, first entry}
     uint32_t tot;
     const uint32_t pre = block_excl_scan(k, &tot);
-    if (threadIdx.x == 0)
+    if (threadIdx.x == 0) {
         s_base = tot ? atomicAdd((unsigned int*)&rc->tail[0].v, tot) : 0u;
+        s_nbig = 0u;
+    }
     __syncthreads();
     uint32_t idx = s_base + pre;
     if (k)
@@ -1426,9 +1434,28 @@ __device__ void run_entry(const uint64_t* __restrict__ act, uint64_t nwords, con
                 for (uint64_t b = x[j]; b; b &= b - 1ull) {
                     const uint32_t v =
                         (uint32_t)((w0 + (uint64_t)j * stride) * 64u + (uint64_t)(__ffsll((long long)b) - 1));
-                    idx = run_put(q, idx, v, csri_off[v], csri_off[v + 1]);
+                    const uint32_t s = csri_off[v], e = csri_off[v + 1], n = run_entries(e - s);
+                    const uint32_t at = n > WG_RUN_SERIAL ? atomicAdd(&s_nbig, 1u) : WG_RUN_BIG;
+                    if (at < WG_RUN_BIG) {
+                        s_big[at] = make_uint2(v, idx);
+                        idx += n;
+                    } else
+                        idx = run_put(q, idx, v, s, e);
                 }
         }
+    __syncthreads();
+    // the long lists, all threads together: a hub's thousands of entries written
+    // by the thread that met it took 130 us of an rmat-s22 BFS
+    const uint32_t nbig = s_nbig < WG_RUN_BIG ? s_nbig : WG_RUN_BIG;
+    for (uint32_t i = 0; i < nbig; ++i) {
+        const uint32_t v = s_big[i].x, at = s_big[i].y, s = csri_off[v], e = csri_off[v + 1];
+        const uint32_t n = run_entries(e - s);
+        for (uint32_t c = threadIdx.x; c < n; c += WG_BLOCK) {
+            const uint32_t cs = s + c * WG_RUN_CH;
+            if (at + c < WG_RUN_QCAP)
+                q[at + c] = make_uint4(v, cs, e - cs > WG_RUN_CH ? cs + WG_RUN_CH : e, c == 0 ? 1u : 0u);
+        }
+    }
 }
 
 // End of level r: the workgroup's counts into the level's totals, the
@@ -2484,14 +2511,40 @@ __global__ __launch_bounds__(SOLO_T) void k_decide_sssp(wg_dev_counters* __restr
 // The instance of a pull kernel with (CW = true) or without the work counts.
 #define WG_CW(ctx, K, ...) ((ctx)->count_work ? K<true, ##__VA_ARGS__> : K<false, ##__VA_ARGS__>)
 
+// Copies the counters to the host mirror (mapped pinned memory), after folding
+// the slots if `fold` is set (one wavefront).
+__global__ void k_publish(wg_dev_counters* c, wg_dev_counters* host, int fold)
+{
+    if (fold)
+        fold_counts(c);
+    __threadfence();
+    for (uint32_t i = threadIdx.x; i < WG_CTR_HOST_BYTES / 8; i += WG_WAVE)
+        ((unsigned long long*)host)[i] =
+            __hip_atomic_load((unsigned long long*)c + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __threadfence_system();
+}
+static_assert(WG_CTR_HOST_BYTES % 8 == 0, "copied in 8-byte words");
+
+// The counters into the host mirror, waited for.
+static int publish(wg_ctx* ctx, int fold)
+{
+    if (ctx->hctr_dev) {
+        hipLaunchKernelGGL(k_publish, dim3(1), dim3(WG_WAVE), 0, ctx->stream, ctx->ctr, ctx->hctr_dev, fold);
+        WG_HIP(ctx, hipGetLastError());
+    } else {
+        if (fold)
+            hipLaunchKernelGGL(k_fold, dim3(1), dim3(WG_WAVE), 0, ctx->stream, ctx->ctr);
+        WG_HIP(ctx, hipGetLastError());
+        WG_HIP(ctx, hipMemcpyAsync(ctx->hctr, ctx->ctr, WG_CTR_HOST_BYTES, hipMemcpyDeviceToHost, ctx->stream));
+    }
+    WG_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    return WG_OK;
+}
+
 // Folds the counter slots and copies the counters to the host mirror.
 int wg_read_counters(wg_ctx* ctx)
 {
-    hipLaunchKernelGGL(k_fold, dim3(1), dim3(WG_WAVE), 0, ctx->stream, ctx->ctr);
-    WG_HIP(ctx, hipGetLastError());
-    WG_HIP(ctx, hipMemcpyAsync(ctx->hctr, ctx->ctr, WG_CTR_HOST_BYTES, hipMemcpyDeviceToHost, ctx->stream));
-    WG_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    return WG_OK;
+    return publish(ctx, 1);
 }
 
 // Folds the slots and hands the level's activity counts to the host mirror
@@ -2574,18 +2627,104 @@ static int build_solo_sssp(wg_ctx* ctx)
     return WG_OK;
 }
 
-static int init_common(wg_ctx* ctx, int app)
+// Everything an application starts from, in one launch: the bitmasks and the
+// Wedge frontier cleared, the vertex values, the counters.  (A launch per array
+// was a dozen on a traversal that takes a few itself.)
+#define INIT_U64 0
+#define INIT_U32 1
+#define INIT_IDS 2 // label[v] = original id of v
+struct app_init {
+    uint64_t *cur, *next, *visited;
+    uint64_t nwords;
+    uint32_t* wedge;
+    uint64_t nwedge;
+    void* prop;
+    uint64_t V;
+    int kind;
+    uint64_t value;
+    const uint32_t* perm;
+};
+
+__global__ __launch_bounds__(WG_BLOCK) void k_app_init(app_init a, wg_dev_counters* __restrict__ c)
+{
+    const uint64_t t = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x, n = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t i = t; i < a.nwords; i += n) {
+        a.cur[i] = 0ull;
+        a.next[i] = 0ull;
+        a.visited[i] = 0ull;
+    }
+    for (uint64_t i = t; i < a.nwedge; i += n)
+        a.wedge[i] = 0u;
+    if (a.kind == INIT_U64)
+        for (uint64_t i = t; i < a.V; i += n)
+            ((uint64_t*)a.prop)[i] = a.value;
+    else if (a.kind == INIT_U32)
+        for (uint64_t i = t; i < a.V; i += n)
+            ((uint32_t*)a.prop)[i] = (uint32_t)a.value;
+    else
+        for (uint64_t i = t; i < a.V; i += n)
+            ((uint32_t*)a.prop)[i] = a.perm ? a.perm[i] : (uint32_t)i;
+    if (blockIdx.x != 0)
+        return;
+    if (threadIdx.x < WG_CSLOTS)
+        for (int f = 0; f < WG_CNT_N; ++f)
+            c->slots[threadIdx.x].v[f] = 0ull;
+    if (threadIdx.x == 0) {
+        c->activity = 0ull;
+        c->activated = 0ull;
+        c->fresh = 0ull;
+        c->frontier_verts = 0ull;
+        c->heavy_len = 0u;
+        c->overflow = 0u;
+        c->edges_read = 0ull;
+        c->dests_examined = 0ull;
+        c->reached_verts = 0ull;
+        c->reached_edges = 0ull;
+        c->level = 0u;
+        c->done = 0u;
+    }
+}
+
+// The single root of a BFS or SSSP (caller's id): its device id, its bits, its
+// value, and {0, out-degree} in root_off.
+__global__ void k_init_root(uint64_t orig, const uint32_t* __restrict__ inv, int app, int wkind, void* __restrict__ prop,
+                            uint64_t* __restrict__ cur, uint64_t* __restrict__ visited,
+                            const uint32_t* __restrict__ csri_off, uint32_t* __restrict__ roots,
+                            uint32_t* __restrict__ root_off)
+{
+    if (threadIdx.x != 0 || blockIdx.x != 0)
+        return;
+    const uint32_t r = inv ? inv[orig] : (uint32_t)orig;
+    roots[0] = r;
+    root_off[0] = 0u;
+    root_off[1] = csri_off[r + 1] - csri_off[r];
+    cur[r >> 6] = 1ull << (r & 63u);
+    if (app == WG_APP_BFS) {
+        visited[r >> 6] = 1ull << (r & 63u);
+        ((uint64_t*)prop)[r] = orig;
+    } else if (wkind == WG_WEIGHT_F64)
+        ((uint64_t*)prop)[r] = 0ull;
+    else
+        ((uint32_t*)prop)[r] = 0u;
+}
+
+// Starts an application: its vertex values (prop[0], kept from the last run of
+// the same application on the graph) and the structures built once per graph.
+static int init_common(wg_ctx* ctx, int app, size_t esz, int kind, uint64_t value)
 {
     if (!ctx || !ctx->off)
         return WG_E_STATE;
     WG_HIP(ctx, hipSetDevice(ctx->device));
-    WG_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    wg_free_app_state(ctx);
     int rc;
-    if ((rc = wg_clear_u64(ctx, ctx->bm_cur, ctx->bm_words)) || (rc = wg_clear_u64(ctx, ctx->bm_next, ctx->bm_words)) ||
-        (rc = wg_clear_u64(ctx, ctx->bm_visited, ctx->bm_words)) || (rc = clear_wedge_state(ctx)) ||
-        (rc = wg_reset_counters(ctx, RST_ACTIVITY | RST_FRONTIER | RST_OVERFLOW | RST_WORK)))
+    if ((rc = wg_app_state(ctx, app, ctx->V * esz, 0)))
         return rc;
+    const app_init a = {ctx->bm_cur,      ctx->bm_next, ctx->bm_visited, ctx->bm_words, ctx->wedge,
+                        ctx->wedge_words, ctx->prop[0], ctx->V,          kind,          value, ctx->perm};
+    hipLaunchKernelGGL(k_app_init, dim3(wg_grid(ctx, std::max(ctx->V, ctx->wedge_words), 1024, 8)), dim3(WG_BLOCK), 0,
+                       ctx->stream, a, ctx->ctr);
+    if ((rc = wg_check_launch(ctx)))
+        return rc;
+    ctx->wedge_log2 = -1;
     ctx->app = app;
     ctx->iter = 0;
     ctx->roots_frontier = 0;
@@ -2623,18 +2762,32 @@ static int init_common(wg_ctx* ctx, int app)
         if ((rc = wg_check_launch(ctx)))
             return rc;
     }
-    WG_HIP(ctx, hipMemsetAsync(&ctx->ctr->level, 0, sizeof(unsigned int), ctx->stream));
-    WG_HIP(ctx, hipMemsetAsync(&ctx->ctr->done, 0, sizeof(unsigned int), ctx->stream));
+    return WG_OK;
+}
+
+// Root arrays for n roots, kept while they are large enough.
+static int root_arrays(wg_ctx* ctx, uint32_t n)
+{
+    if (ctx->roots && ctx->roots_cap >= n)
+        return WG_OK;
+    WG_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    (void)hipFree(ctx->roots);
+    (void)hipFree(ctx->root_off);
+    ctx->roots = ctx->root_off = nullptr;
+    ctx->roots_cap = 0;
+    const uint64_t cap = n < 64u ? 64u : n;
+    WG_HIP(ctx, hipMalloc((void**)&ctx->roots, cap * sizeof(uint32_t)));
+    WG_HIP(ctx, hipMalloc((void**)&ctx->root_off, (cap + 1) * sizeof(uint32_t)));
+    ctx->roots_cap = (uint32_t)cap;
     return WG_OK;
 }
 
 // Roots (device ids, distinct): BFS state depth 0 / parent = the root itself
 // (original id), SSSP distance 0; every root is set in bm_cur (BFS frontier;
 // for SSSP the set the first frontier build starts from) and, for BFS, in
-// bm_visited; the activity of the root level (summed out-degree) is counted.
+// bm_visited.
 __global__ void k_init_roots(const uint32_t* __restrict__ roots, uint32_t n, int app, int wkind, void* __restrict__ prop,
-                             const uint32_t* __restrict__ perm, uint64_t* __restrict__ cur, uint64_t* __restrict__ visited,
-                             const uint32_t* __restrict__ od, wg_dev_counters* __restrict__ ctr)
+                             const uint32_t* __restrict__ perm, uint64_t* __restrict__ cur, uint64_t* __restrict__ visited)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n)
@@ -2650,7 +2803,6 @@ __global__ void k_init_roots(const uint32_t* __restrict__ roots, uint32_t n, int
     } else {
         ((uint32_t*)prop)[r] = 0u;
     }
-    atomicAdd(&ctr->slots[0].v[WG_CNT_ACTIVITY], (unsigned long long)od[r]);
 }
 
 static int init_roots(wg_ctx* ctx, int app, const uint64_t* roots, uint32_t n)
@@ -2659,39 +2811,38 @@ static int init_roots(wg_ctx* ctx, int app, const uint64_t* roots, uint32_t n)
         return WG_E_INVAL;
     if (!ctx->off || (app == WG_APP_SSSP && ctx->wkind == WG_WEIGHT_NONE))
         return WG_E_STATE;
-    std::vector<uint32_t> dev(n);
+    std::vector<uint32_t> dev;
     int rc;
-    if ((rc = wg_to_device_ids(ctx, roots, n, dev.data())))
-        return rc;
-    std::sort(dev.begin(), dev.end());
-    dev.erase(std::unique(dev.begin(), dev.end()), dev.end());
-    if ((rc = init_common(ctx, app)))
-        return rc;
-    const size_t esz = (app == WG_APP_BFS || ctx->wkind == WG_WEIGHT_F64) ? 8 : 4;
-    WG_HIP(ctx, hipMalloc(&ctx->prop[0], ctx->V * esz));
-    WG_HIP(ctx, hipMalloc((void**)&ctx->roots, dev.size() * sizeof(uint32_t)));
-    ctx->nroots = (uint32_t)dev.size();
-    ctx->root_dev = dev[0];
-    WG_HIP(ctx, hipMemcpyAsync(ctx->roots, dev.data(), dev.size() * sizeof(uint32_t), hipMemcpyHostToDevice, ctx->stream));
-    if (esz == 8)
-        rc = wg_fill_u64(ctx, (uint64_t*)ctx->prop[0], ctx->V, app == WG_APP_BFS ? ~0ull : (uint64_t)PolSF::INF);
-    else
-        rc = wg_fill_u32(ctx, (uint32_t*)ctx->prop[0], ctx->V, PolSU::INF);
-    if (rc || (rc = wg_reset_counters(ctx, RST_ACTIVITY)))
-        return rc;
-    hipLaunchKernelGGL(k_init_roots, dim3((ctx->nroots + 255) / 256), dim3(256), 0, ctx->stream, ctx->roots, ctx->nroots,
-                       app, ctx->wkind, ctx->prop[0], ctx->perm, ctx->bm_cur, ctx->bm_visited, ctx->od, ctx->ctr);
-    if ((rc = wg_check_launch(ctx)) || (rc = wg_read_counters(ctx)))
-        return rc;
-    ctx->root_activity = ctx->hctr->activity;
-    ctx->roots_frontier = app == WG_APP_BFS;
-    if (app == WG_APP_BFS && ctx->nroots <= WG_PUSH_ROOTS_MAX) { // for the first level's push
-        WG_HIP(ctx, hipMalloc((void**)&ctx->root_off, (ctx->nroots + 1) * sizeof(uint32_t)));
-        hipLaunchKernelGGL(k_root_offsets, dim3(1), dim3(WG_BLOCK), 0, ctx->stream, ctx->roots, ctx->nroots,
-                           ctx->csri_off, ctx->root_off);
-        if ((rc = wg_check_launch(ctx)))
+    if (n == 1 && roots[0] >= ctx->V)
+        return WG_E_RANGE;
+    if (n > 1) {
+        dev.resize(n);
+        if ((rc = wg_to_device_ids(ctx, roots, n, dev.data())))
             return rc;
+        std::sort(dev.begin(), dev.end());
+        dev.erase(std::unique(dev.begin(), dev.end()), dev.end());
+        n = (uint32_t)dev.size();
     }
+    const size_t esz = (app == WG_APP_BFS || ctx->wkind == WG_WEIGHT_F64) ? 8 : 4;
+    if ((rc = init_common(ctx, app, esz, esz == 8 ? INIT_U64 : INIT_U32,
+                          app == WG_APP_BFS ? ~0ull : esz == 8 ? (uint64_t)PolSF::INF : (uint64_t)PolSU::INF)) ||
+        (rc = root_arrays(ctx, n)))
+        return rc;
+    ctx->nroots = n;
+    ctx->roots_frontier = app == WG_APP_BFS;
+    if (dev.empty()) {
+        hipLaunchKernelGGL(k_init_root, dim3(1), dim3(WG_WAVE), 0, ctx->stream, roots[0], ctx->inv, app, ctx->wkind,
+                           ctx->prop[0], ctx->bm_cur, ctx->bm_visited, ctx->csri_off, ctx->roots, ctx->root_off);
+        return wg_check_launch(ctx);
+    }
+    WG_HIP(ctx, hipMemcpyAsync(ctx->roots, dev.data(), n * sizeof(uint32_t), hipMemcpyHostToDevice, ctx->stream));
+    hipLaunchKernelGGL(k_init_roots, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, ctx->roots, n, app, ctx->wkind,
+                       ctx->prop[0], ctx->perm, ctx->bm_cur, ctx->bm_visited);
+    hipLaunchKernelGGL(k_root_offsets, dim3(1), dim3(WG_BLOCK), 0, ctx->stream, ctx->roots, n, ctx->csri_off,
+                       ctx->root_off);
+    if ((rc = wg_check_launch(ctx)))
+        return rc;
+    WG_HIP(ctx, hipStreamSynchronize(ctx->stream)); // dev has been read
     return WG_OK;
 }
 
@@ -2707,16 +2858,7 @@ extern "C" int wg_init_bfs(wg_ctx* ctx, uint64_t root)
 
 extern "C" int wg_init_cc(wg_ctx* ctx)
 {
-    int rc = init_common(ctx, WG_APP_CC);
-    if (rc)
-        return rc;
-    WG_HIP(ctx, hipMalloc(&ctx->prop[0], ctx->V * sizeof(uint32_t)));
-    hipLaunchKernelGGL(k_iota_u32, dim3(wg_grid(ctx, ctx->V, 1024, 8)), dim3(256), 0, ctx->stream, (uint32_t*)ctx->prop[0],
-                       ctx->V, ctx->perm);
-    if ((rc = wg_check_launch(ctx)))
-        return rc;
-    WG_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    return WG_OK;
+    return init_common(ctx, WG_APP_CC, sizeof(uint32_t), INIT_IDS, 0);
 }
 
 extern "C" int wg_init_sssp_roots(wg_ctx* ctx, const uint64_t* roots, uint32_t n)
@@ -3079,7 +3221,6 @@ extern "C" int wg_reached(wg_ctx* ctx, uint64_t* vertices, uint64_t* edges)
 {
     if (!ctx || (ctx->app != WG_APP_BFS && ctx->app != WG_APP_SSSP && ctx->app != WG_APP_CC))
         return WG_E_STATE;
-    WG_HIP(ctx, hipMemsetAsync(&ctx->ctr->reached_verts, 0, 2 * sizeof(unsigned long long), ctx->stream));
     const uint32_t grid = wg_grid(ctx, ctx->V, 1024, 8);
     if (ctx->app == WG_APP_BFS)
         hipLaunchKernelGGL(k_reached_bfs, dim3(grid), dim3(256), 0, ctx->stream, (const uint64_t*)ctx->prop[0], ctx->od,
@@ -3100,7 +3241,7 @@ extern "C" int wg_reached(wg_ctx* ctx, uint64_t* vertices, uint64_t* edges)
         *vertices = ctx->hctr->reached_verts;
     if (edges)
         *edges = ctx->hctr->reached_edges;
-    return WG_OK;
+    return wg_reset_counters(ctx, RST_REACHED); // for the next call
 }
 
 // One iteration of the device-resident loop: the level pull (BFS dense: with
@@ -3239,7 +3380,6 @@ extern "C" int wg_converge(wg_ctx* ctx, const wg_loop_params* p, uint64_t* itera
             WG_HIP(ctx, hipMalloc((void**)&ctx->run_ctl, sizeof(wg_run_ctl)));
             WG_HIP(ctx, hipMalloc((void**)&ctx->run_q, 2 * (size_t)WG_RUN_QCAP * sizeof(uint4)));
         }
-        WG_HIP(ctx, hipMemsetAsync(ctx->run_ctl, 0, sizeof(wg_run_ctl), ctx->stream));
         if (ctx->app != WG_APP_BFS) {
             if (!ctx->run_spare)
                 WG_HIP(ctx, hipMalloc((void**)&ctx->run_spare, ctx->bm_words * sizeof(uint64_t)));
@@ -3249,9 +3389,11 @@ extern "C" int wg_converge(wg_ctx* ctx, const wg_loop_params* p, uint64_t* itera
     }
     const unsigned long long threshold = (ctx->E * (unsigned long long)p->threshold_pct) / 100ull;
     // CC: source/execution_cc.c:95; BFS / SSSP: out-degree of the roots
-    const unsigned long long act0 = ctx->app == WG_APP_CC ? ctx->E : ctx->root_activity;
+    const unsigned long long act0 = ctx->app == WG_APP_CC ? ctx->E : 0ull;
     hipLaunchKernelGGL(k_loop_init, dim3(1), dim3(WG_WAVE), 0, ctx->stream, ctx->ctr, ctx->mlp_set ? ctx->mlp : nullptr,
                        (unsigned int)p->schedule, threshold, blog2, p->max_iterations, act0,
+                       ctx->app == WG_APP_CC ? nullptr : ctx->root_off + ctx->nroots,
+                       ctx->run_wgs[ctx->app & 7] ? ctx->run_ctl : nullptr,
                        ctx->app == WG_APP_CC ? (unsigned long long)ctx->V : (unsigned long long)ctx->nroots,
                        ctx->app == WG_APP_CC ? 1 : 0,
                        ctx->app == WG_APP_CC ? 0ull : (unsigned long long)(ctx->V - ctx->nroots), (unsigned int)ctx->app,
@@ -3261,10 +3403,9 @@ extern "C" int wg_converge(wg_ctx* ctx, const wg_loop_params* p, uint64_t* itera
     // roots' out-edges if that level is frontier-filtered (k_bfs_level), so
     // no blocks are marked for it.
     ctx->push_roots =
-        (ctx->app == WG_APP_BFS && ctx->roots_frontier && ctx->root_off) ? ctx->nroots : 0u;
+        (ctx->app == WG_APP_BFS && ctx->roots_frontier && ctx->nroots <= WG_PUSH_ROOTS_MAX) ? ctx->nroots : 0u;
     ctx->roots_frontier = 0;
     if (ctx->app != WG_APP_CC) { // the roots' blocks, if the first pull is frontier-filtered
-        hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, ctx->stream, ctx->ctr, RST_HEAVY);
         if (!ctx->push_roots) {
             hipLaunchKernelGGL(k_wedge_build, dim3(wg_wedge_build_grid(ctx)), dim3(WG_BLOCK), 0, ctx->stream,
                                ctx->bm_cur, ctx->bm_words, ctx->csri_off, ctx->csri_pos, 0, ctx->wedge, ctx->heavy_list,
@@ -3287,8 +3428,8 @@ extern "C" int wg_converge(wg_ctx* ctx, const wg_loop_params* p, uint64_t* itera
         for (uint32_t i = 0; i < batch; ++i)
             if ((rc = enqueue_iteration(ctx)))
                 return rc;
-        WG_HIP(ctx, hipMemcpyAsync(ctx->hctr, ctx->ctr, WG_CTR_HOST_BYTES, hipMemcpyDeviceToHost, ctx->stream));
-        WG_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        if ((rc = publish(ctx, 0)))
+            return rc;
         if (ctx->hctr->run_err)
             return WG_E_STATE;
         if (ctx->hctr->done)

@@ -110,7 +110,7 @@ int wg_run_pr(wg_ctx* ctx, const wg_run_opts* o, double* ranks, wg_run_stats* st
     wg_run_stats s;
     memset(&s, 0, sizeof(s));
     int rc = wg_init_pr(ctx, o->damping, o->contrib_fp32);
-    if (rc)
+    if (rc || (rc = wg_sync(ctx))) /* the running time does not include the initialisation */
         return rc;
     const double t0 = now_ms();
     for (uint32_t it = 0; it < o->iterations; ++it) {
@@ -158,7 +158,7 @@ static int run_device_loop(wg_ctx* ctx, const wg_run_opts* o, wg_run_stats* st)
     memset(&s, 0, sizeof(s));
     uint64_t it = 0, fit = 0;
     int rc = wg_set_schedule_model(ctx, o->schedule == WG_SCHED_LEARNED ? wg_mlp_params() : NULL, WG_MLP_PARAMS);
-    if (rc)
+    if (rc || (rc = wg_sync(ctx))) /* the running time does not include the initialisation */
         return rc;
     const double t0 = now_ms();
     rc = wg_converge(ctx, &p, &it, &fit);
