@@ -9,15 +9,18 @@
 // member.  One iteration is
 //   1. the edge pull over edge tiles (k_pr_tile / k_pr_span in edge-phase
 //      mode, source/phase_edge_pull_pr.c:28-116): acc[v] for every vertex;
-//   2. k_bm_chunk_sum: the accumulators of each chunk (<= WG_MEMBER_CHUNK
-//      vertices of one member) summed in a fixed order;
-//   3. k_bm_vertex: S of the chunk's member from its chunk sums (fixed order),
-//      then the vertex phase of the chunk's vertices with the member's N.
+//   2. k_bm_vertex: S of the chunk's member from its chunk sums (fixed order),
+//      then the vertex phase of the chunk's vertices (<= WG_MEMBER_CHUNK of one
+//      member) with the member's N, and the chunk's sum for the next iteration.
+// S = sum of a member's accumulators = sum of its ranks, one iteration earlier,
+// over vertices with out-edges, so the vertex phase can sum them for the next
+// iteration: no kernel between the pull and the vertex phase (one launch of four,
+// 5 us of an iteration of 80-100 on 64 graphs of 10.7 million edges in all).
 // Every sum is taken in a fixed order, so runs are bit-reproducible and the
 // captured HIP graph gives the same ranks as plain launches.
 //
 // Small graphs make this launch-bound when run one by one (a few kernels per
-// iteration per graph); as one union, a whole K-iteration run is 1 + 4K
+// iteration per graph); as one union, a whole K-iteration run is 1 + 3K
 // kernels, captured once into a HIP graph and replayed as one launch.  The
 // tile shape (edges per lane) and the tile kernel's workgroups per CU are
 // picked by timing every candidate (wg_batch_autotune).
@@ -54,10 +57,9 @@ struct wg_members {
     uint32_t* member_chunk = nullptr; // n + 1: member g holds chunks [member_chunk[g], member_chunk[g + 1])
     shape_tiles tiles[k_n_ipt];
     double* tile_part = nullptr;  // heavy-tile partial sums (largest tiling)
-    double* blk_part = nullptr;   // per-block sums of the edge pull (not used for S)
-    double* chunk_part = nullptr; // per-chunk sums of the accumulators
+    double* chunk_part = nullptr; // two arrays of nchunks: per-chunk sums of ranks, this and the next iteration's
     double* acc = nullptr;        // V accumulators
-    double* scratch = nullptr;    // [0]: unused S input, [1]: total of the accumulators
+    double* scratch = nullptr;    // the edge pull's S input (unused in edge-phase mode)
     void* c[2] = {nullptr, nullptr}; // contributions
     int c_fp32 = -1;              // precision c[] was allocated for
     int cur = -1;                 // buffer holding the last run's contributions
@@ -107,7 +109,6 @@ void wg_free_members(wg_ctx* ctx)
         free_dev_ptr(t.heavy_t);
     }
     free_dev_ptr(m->tile_part);
-    free_dev_ptr(m->blk_part);
     free_dev_ptr(m->chunk_part);
     free_dev_ptr(m->acc);
     free_dev_ptr(m->scratch);
@@ -142,28 +143,20 @@ template <typename T>
 __global__ __launch_bounds__(WG_BLOCK) void k_bm_init(const uint32_t* __restrict__ od, T* __restrict__ c,
                                                       const uint32_t* __restrict__ chunk_v,
                                                       const uint32_t* __restrict__ chunk_m,
-                                                      const uint32_t* __restrict__ first, uint32_t nchunks)
-{
-    for (uint32_t ch = blockIdx.x; ch < nchunks; ch += gridDim.x) {
-        const uint32_t g = chunk_m[ch];
-        const double N = (double)(first[g + 1] - first[g]);
-        for (uint32_t v = chunk_v[ch] + threadIdx.x; v < chunk_v[ch + 1]; v += WG_BLOCK) {
-            const uint32_t o = od[v];
-            c[v] = (T)((1.0 / N) / (o ? (double)o : N));
-        }
-    }
-}
-
-// Sum of the accumulators of each chunk, thread-strided then in wave order.
-__global__ __launch_bounds__(WG_BLOCK) void k_bm_chunk_sum(const double* __restrict__ acc,
-                                                           const uint32_t* __restrict__ chunk_v, uint32_t nchunks,
-                                                           double* __restrict__ chunk_part)
+                                                      const uint32_t* __restrict__ first, uint32_t nchunks,
+                                                      double* __restrict__ chunk_part)
 {
     __shared__ double s_red[WG_WPB];
     for (uint32_t ch = blockIdx.x; ch < nchunks; ch += gridDim.x) {
+        const uint32_t g = chunk_m[ch];
+        const double N = (double)(first[g + 1] - first[g]);
         double s = 0.0;
-        for (uint32_t v = chunk_v[ch] + threadIdx.x; v < chunk_v[ch + 1]; v += WG_BLOCK)
-            s += acc[v];
+        for (uint32_t v = chunk_v[ch] + threadIdx.x; v < chunk_v[ch + 1]; v += WG_BLOCK) {
+            const uint32_t o = od[v];
+            c[v] = (T)((1.0 / N) / (o ? (double)o : N));
+            if (o)
+                s += 1.0 / N;
+        }
         s = block_sum_det(s, s_red);
         if (threadIdx.x == 0)
             chunk_part[ch] = s;
@@ -171,14 +164,16 @@ __global__ __launch_bounds__(WG_BLOCK) void k_bm_chunk_sum(const double* __restr
 }
 
 // source/phase_vertex_pr.c:26-77 for the vertices of each chunk, with N and S
-// of the chunk's member.
+// of the chunk's member; the chunk's ranks with out-edges summed thread-strided,
+// then in wave order.
 template <typename T>
 __global__ __launch_bounds__(WG_BLOCK) void k_bm_vertex(const double* __restrict__ acc, const uint32_t* __restrict__ od,
                                                         T* __restrict__ cout, const uint32_t* __restrict__ chunk_v,
                                                         const uint32_t* __restrict__ chunk_m,
                                                         const uint32_t* __restrict__ member_chunk,
                                                         const uint32_t* __restrict__ first, uint32_t nchunks,
-                                                        const double* __restrict__ chunk_part, double damping)
+                                                        const double* __restrict__ chunk_part,
+                                                        double* __restrict__ chunk_next, double damping)
 {
     __shared__ double s_red[WG_WPB];
     for (uint32_t ch = blockIdx.x; ch < nchunks; ch += gridDim.x) {
@@ -188,13 +183,19 @@ __global__ __launch_bounds__(WG_BLOCK) void k_bm_vertex(const double* __restrict
         const double N = (double)(first[g + 1] - first[g]);
         const double corr = (1.0 - S) / N;
         const double omd_n = (1.0 - damping) / N;
+        double s = 0.0;
         for (uint32_t v = chunk_v[ch] + threadIdx.x; v < chunk_v[ch + 1]; v += WG_BLOCK) {
             const uint32_t odv = od[v];
             const double t1 = acc[v] + corr;
             const double t2 = t1 * damping;
             const double rank = t2 + omd_n;
             cout[v] = (T)(rank / (odv ? (double)odv : N));
+            if (odv)
+                s += rank;
         }
+        s = block_sum_det(s, s_red);
+        if (threadIdx.x == 0)
+            chunk_next[ch] = s;
         __syncthreads(); // s_red is reused by the next chunk
     }
 }
@@ -284,13 +285,11 @@ static int build_members(wg_ctx* ctx, wg_members* m, const uint64_t* first, uint
             (rc = upload_vec(ctx, &t.heavy_v, hv)) || (rc = upload_vec(ctx, &t.heavy_t, ht)))
             return rc;
     }
-    const size_t nblk = (size_t)ctx->num_cu * 16 + WG_NXCD + (size_t)ctx->num_cu * 4 + 16;
     WG_HIP(ctx, hipMalloc((void**)&m->tile_part, (max_tiles + 1) * sizeof(double)));
-    WG_HIP(ctx, hipMalloc((void**)&m->blk_part, nblk * sizeof(double)));
-    WG_HIP(ctx, hipMalloc((void**)&m->chunk_part, (m->nchunks + 1) * sizeof(double)));
+    WG_HIP(ctx, hipMalloc((void**)&m->chunk_part, 2 * (size_t)m->nchunks * sizeof(double)));
     WG_HIP(ctx, hipMalloc((void**)&m->acc, (ctx->V ? ctx->V : 1) * sizeof(double)));
-    WG_HIP(ctx, hipMalloc((void**)&m->scratch, 2 * sizeof(double)));
-    WG_HIP(ctx, hipMemset(m->scratch, 0, 2 * sizeof(double)));
+    WG_HIP(ctx, hipMalloc((void**)&m->scratch, sizeof(double)));
+    WG_HIP(ctx, hipMemset(m->scratch, 0, sizeof(double)));
     return WG_OK;
 }
 
@@ -342,8 +341,7 @@ static bool same_shape(const wg_batch_shape& a, const wg_batch_shape& b)
     return a.edges_per_lane == b.edges_per_lane && a.blocks_per_cu == b.blocks_per_cu && a.xcd_split == b.xcd_split;
 }
 
-// Queues the whole run: init, then `iters` times edge pull, chunk sums and
-// vertex phase.  Only kernel launches (no copies, fills or waits), so the same
+// Queues the whole run: init, then `iters` times edge pull and vertex phase.  Only kernel launches (no copies, fills or waits), so the same
 // sequence is captured into the HIP graph.
 template <typename T, int IPT>
 static int queue_run(wg_ctx* ctx, wg_members* m, const shape_tiles& t, uint32_t bpc, uint32_t xcd, uint32_t iters,
@@ -358,20 +356,20 @@ static int queue_run(wg_ctx* ctx, wg_members* m, const shape_tiles& t, uint32_t 
     const uint32_t sgrid = wg_grid(ctx, t.nheavy, 4, 4);
     T* c[2] = {(T*)m->c[0], (T*)m->c[1]};
     hipLaunchKernelGGL(k_bm_init<T>, dim3(cgrid), dim3(WG_BLOCK), 0, ctx->stream, ctx->od, c[0], m->chunk_v, m->chunk_m,
-                       m->d_first, m->nchunks);
+                       m->d_first, m->nchunks, m->chunk_part);
     for (uint32_t it = 0; it < iters; ++it) {
         const T* cin = c[it & 1];
         T* cout = c[(it & 1) ^ 1];
         hipLaunchKernelGGL((k_pr_tile<T, 1, IPT>), dim3(grid), dim3(WG_BLOCK), 0, ctx->stream, ctx->off, ctx->src, cin,
                            (T*)nullptr, m->acc, ctx->od, t.tile_v, t.tile_e, t.ntiles, m->scratch, damping, 1.0,
-                           m->tile_part, m->blk_part, split);
+                           m->tile_part, (double*)nullptr, split);
         hipLaunchKernelGGL((k_pr_span<T, 1, IPT>), dim3(sgrid), dim3(WG_BLOCK), 0, ctx->stream, ctx->off, t.heavy_v,
                            t.heavy_t, t.nheavy, m->tile_part, (T*)nullptr, m->acc, ctx->od, m->scratch, damping, 1.0,
-                           m->blk_part, grid, m->scratch + 1, &ctx->ctr->ticket);
-        hipLaunchKernelGGL(k_bm_chunk_sum, dim3(cgrid), dim3(WG_BLOCK), 0, ctx->stream, m->acc, m->chunk_v, m->nchunks,
-                           m->chunk_part);
+                           (double*)nullptr, 0u, (double*)nullptr, &ctx->ctr->ticket);
         hipLaunchKernelGGL(k_bm_vertex<T>, dim3(cgrid), dim3(WG_BLOCK), 0, ctx->stream, m->acc, ctx->od, cout,
-                           m->chunk_v, m->chunk_m, m->member_chunk, m->d_first, m->nchunks, m->chunk_part, damping);
+                           m->chunk_v, m->chunk_m, m->member_chunk, m->d_first, m->nchunks,
+                           m->chunk_part + (it & 1) * (size_t)m->nchunks,
+                           m->chunk_part + ((it & 1) ^ 1) * (size_t)m->nchunks, damping);
     }
     return wg_check_launch(ctx);
 }

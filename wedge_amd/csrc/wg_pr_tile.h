@@ -256,6 +256,8 @@ __global__ __launch_bounds__(WPB * WG_WAVE) void k_pr_tile(const uint32_t* __res
         }
         wg_wave_sync(); // the next tile reuses this wavefront's LDS
     }
+    if (!blk_part) // the caller does not use the sum
+        return;
     s_part = block_sum_det<WPB>(s_part, s_red);
     if (threadIdx.x == 0)
         blk_part[blockIdx.x] = s_part;
@@ -314,6 +316,8 @@ __global__ __launch_bounds__(WG_BLOCK) void k_pr_span(const uint32_t* __restrict
             }
         }
     }
+    if (!S_out) // the caller does not use the sum
+        return;
     s_part = block_sum_det(s_part, s_red);
     if (threadIdx.x == 0) {
         blk_part[main_blocks + blockIdx.x] = s_part;
