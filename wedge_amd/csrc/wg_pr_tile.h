@@ -43,10 +43,15 @@ static __device__ __forceinline__ double block_sum_det(double v, double* s_red)
     return r;
 }
 
+// x as a value the compiler knows nothing about.  Gathers that are each in a
+// branch of their own start from it: from a constant, what is done with their
+// results (the conversion to FP64, an addition) moves into the branches, and the
+// wavefront waits for one gather before it issues the next.
 template <typename T>
-static __device__ __forceinline__ double load_contrib(const T* __restrict__ p, uint32_t i)
+static __device__ __forceinline__ T opaque_value(T x)
 {
-    return (double)p[i];
+    asm volatile("" : "+v"(x));
+    return x;
 }
 
 // MODE 0: fused iteration (contrib_out + partial S of ranks)
@@ -97,10 +102,10 @@ __global__ __launch_bounds__(WPB * WG_WAVE) void k_pr_tile(const uint32_t* __res
             s_hub[i] = cin[i];
         __syncthreads();
     }
-    auto gather = [&](uint32_t sj) -> double {
+    auto gather = [&](uint32_t sj) -> T {
         if (HUB && sj < nhub)
-            return (double)s_hub[sj];
-        return load_contrib(cin, sj);
+            return s_hub[sj];
+        return cin[sj];
     };
 
     const int wave = threadIdx.x / WG_WAVE;
@@ -134,11 +139,17 @@ __global__ __launch_bounds__(WPB * WG_WAVE) void k_pr_tile(const uint32_t* __res
             s_idx[j] = (a + j < e1) ? __builtin_nontemporal_load(&src[a + j]) : 0u;
         if (tv & WG_HEAVY_BIT) {
             // heavy tile: one destination, partial sum in a fixed order
+            T x[IPT];
+#pragma unroll
+            for (int j = 0; j < IPT; ++j) {
+                x[j] = opaque_value(T(0));
+                if (a + j < e1)
+                    x[j] = gather(s_idx[j]);
+            }
             double s = 0.0;
 #pragma unroll
             for (int j = 0; j < IPT; ++j)
-                if (a + j < e1)
-                    s += gather(s_idx[j]);
+                s += (double)x[j];
             s = wg_wave_sum(s);
             if (lane == 0)
                 tile_part[t] = s;
@@ -159,10 +170,10 @@ __global__ __launch_bounds__(WPB * WG_WAVE) void k_pr_tile(const uint32_t* __res
                 odw[k] = (i < nv) ? od[v0 + i] : 0u;
             }
         }
-        double g[IPT];
+        T g[IPT];
 #pragma unroll
         for (int j = 0; j < IPT; ++j) {
-            g[j] = 0.0;
+            g[j] = opaque_value(T(0));
             if (a + j < e1)
                 g[j] = gather(s_idx[j]);
         }
@@ -194,7 +205,7 @@ __global__ __launch_bounds__(WPB * WG_WAVE) void k_pr_tile(const uint32_t* __res
             for (int j = 0; j < IPT; ++j) {
                 const uint32_t e = a + j;
                 if (e < e1) {
-                    run += g[j];
+                    run += (double)g[j];
                     if (e + 1 == dend) {
                         if (first && cont)
                             fp = run;
