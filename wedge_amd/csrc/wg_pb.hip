@@ -1056,11 +1056,16 @@ __device__ __forceinline__ uint32_t pb_slice_of(uint32_t i, uint32_t n)
 // loaded them, so the destinations, the offsets and then the partials are
 // two rounds of loads.  A chunk with more blocks (rare) loads its block
 // number, chunk_block[c], then the blocks' offsets, boff[].  R chunks per wavefront are
-// in flight at a time: the pull waits on this chain of loads, so more is
-// better as far as registers allow (the PageRank pull at s27: R = 6, 8, 10,
-// 12 took 3.66, 3.60, 3.57, 3.53 ms; 12 for FP64 PageRank partials, 8 for
-// FP32 ones (12 took their pull from 3.27 to 4.45 ms) and for the minimum,
-// 4 for the 64-source BFS, whose epilogue keeps more registers).
+// in flight at a time: the pull waits on this chain of loads.  8 for the
+// PageRank partials and the minimum (R = 8, 12, 16 took the FP64 PageRank
+// pull of R-MAT graphs of scale 22, 24, 25 74, 286, 550 us; 75, 300, 576; 78,
+// 297, 574), 4 for the 64-source BFS, whose epilogue keeps more registers.
+// No load is in a branch: chunks past the slice's end repeat its last one,
+// lanes outside the slice load from a valid place, and only their additions
+// are left out.  (With each load in a branch of its own there was a wait after
+// a group's first one and twice the instructions: the FP64 pull at scales 22
+// and 25 took 77 and 565 us against 74 and 550, the FP32 one 66 and 482
+// against 61 and 432.)
 template <int R, typename X, class ADD>
 __device__ __forceinline__ void pb_pull_range(const X* __restrict__ part, const uint16_t* __restrict__ pdst,
                                               const uint32_t* __restrict__ chunk_block,
@@ -1071,42 +1076,38 @@ __device__ __forceinline__ void pb_pull_range(const X* __restrict__ part, const 
         return;
     const int lane = wg_lane();
     const unsigned long long upto = lane == 63 ? ~0ull : (2ull << lane) - 1ull; // lanes 0..lane
-    const uint32_t wave = threadIdx.x / WG_WAVE;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WG_WAVE); // chunk numbers are scalars
     const uint32_t c1 = ((b1 - 1u) >> 6) + 1u;
     const uint32_t* __restrict__ cbo = chunk_block + ((npairs + 63u) >> 6) + 1u;
     for (uint32_t c = (b0 >> 6) + wave; c < c1; c += WG_PB_WAVES * R) {
-        uint32_t o[R], pd[R], bo[R];
+        uint32_t pd[R], bo[R];
         X x[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            const uint32_t cc = c + (uint32_t)r * WG_PB_WAVES; // uniform
-            o[r] = cc * 64u + (uint32_t)lane;
-            pd[r] = 0u;
-            bo[r] = 0u;
-            if (cc < c1) {
-                if (o[r] < npairs)
-                    pd[r] = pdst[o[r]];
-                if ((uint32_t)lane < WG_PB_CHUNK_OFFS)
-                    bo[r] = cbo[(uint64_t)cc * WG_PB_CHUNK_OFFS + (uint32_t)lane];
-            }
+            const uint32_t cr = c + (uint32_t)r * WG_PB_WAVES, cc = cr < c1 ? cr : c1 - 1u;
+            const uint32_t o = cc * 64u + (uint32_t)lane;
+            pd[r] = pdst[o < npairs ? o : npairs - 1u];
+            bo[r] = cbo[(uint64_t)cc * WG_PB_CHUNK_OFFS + ((uint32_t)lane & (WG_PB_CHUNK_OFFS - 1u))];
         }
         unsigned slow = 0u; // uniform: chunks with more blocks than kept offsets, done below
 #pragma unroll
         for (int r = 0; r < R; ++r) {
+            const uint32_t cr = c + (uint32_t)r * WG_PB_WAVES, o = cr * 64u + (uint32_t)lane;
             // blocks started after the chunk's first position: up to this one, and in all
-            const unsigned long long starts = wg_ballot(lane > 0 && (pd[r] & WG_PB_BFLAG));
+            const unsigned long long starts = wg_ballot(lane > 0 && (pd[r] & WG_PB_BFLAG) && o < npairs);
             const uint32_t k = (uint32_t)__popcll(starts & upto);
-            if ((uint32_t)__popcll(starts) >= WG_PB_CHUNK_OFFS)
+            if (cr < c1 && (uint32_t)__popcll(starts) >= WG_PB_CHUNK_OFFS)
                 slow |= 1u << r;
             const uint32_t off = (uint32_t)__shfl((int)bo[r], (int)k, WG_WAVE);
-            x[r] = X(0);
-            if (!((slow >> r) & 1u) && o[r] >= b0 && o[r] < b1)
-                x[r] = __builtin_nontemporal_load(&part[o[r] - off]);
+            const bool mine = cr < c1 && !((slow >> r) & 1u) && o >= b0 && o < b1;
+            x[r] = __builtin_nontemporal_load(&part[mine ? o - off : 0u]);
         }
 #pragma unroll
-        for (int r = 0; r < R; ++r)
-            if (!((slow >> r) & 1u) && o[r] >= b0 && o[r] < b1)
+        for (int r = 0; r < R; ++r) {
+            const uint32_t cr = c + (uint32_t)r * WG_PB_WAVES, o = cr * 64u + (uint32_t)lane;
+            if (cr < c1 && !((slow >> r) & 1u) && o >= b0 && o < b1)
                 add(pd[r] & WG_PB_DMASK, x[r]);
+        }
         while (slow) { // the block number, then every block offset the chunk needs
             const uint32_t r = (uint32_t)__builtin_ctz(slow);
             slow &= slow - 1u;
@@ -1200,8 +1201,8 @@ __global__ __launch_bounds__(WG_PB_THREADS) void k_pb_pull(
         for (uint32_t i = threadIdx.x; i < nv; i += WG_PB_THREADS)
             s_acc[i] = 0.0;
         __syncthreads();
-        pb_pull_range<sizeof(T) == 8 ? 12 : 8>(part, pdst, chunk_block, boff, nblocks, npairs, sl.y, sl.z,
-                                               [&](uint32_t d, T x) { atomicAdd(&s_acc[d], (double)x); });
+        pb_pull_range<8>(part, pdst, chunk_block, boff, nblocks, npairs, sl.y, sl.z,
+                         [&](uint32_t d, T x) { atomicAdd(&s_acc[d], (double)x); });
         __syncthreads();
         if (sl.w != WG_PB_NOSLOT &&
             !pb_join_slices(s_acc, nv, b, sl.w, bin_slot, slot_acc, bin_ticket, (uint32_t)WD, &s_flag,
