@@ -2,7 +2,8 @@
 pull bins of 4K, 8K and 16K vertices of the binned layout, the 128- and
 512-edge tiles of the 64-source SSSP with and without marked destinations
 (hub lists cut into chunks), and one to eight wavefronts per tile of the
-personalised PageRank, BFS levels in one workgroup.  Against the oracle: exact for BFS, CC and SSSP, 1e-10
+personalised PageRank, BFS levels and SSSP rounds in one workgroup, and results
+stored to page-locked memory by the kernel or copied.  Against the oracle: exact for BFS, CC and SSSP, 1e-10
 L1 for FP64 PageRank (sums of FP64 values in another order), 2e-7 L1 for
 FP32-stored contributions (one rounding of 6e-8 per contribution)."""
 from __future__ import annotations
@@ -217,3 +218,53 @@ def test_sssp_rounds_in_one_workgroup(graph, kind):
                 c.load(gw)
         finally:
             c.close()
+
+
+# page-locked memory: at an allocation's start, inside one, ending with one, at
+# no multiple of the element size (copied), and over 32 MiB (copied); the
+# elements around the result keep their value
+@pytest.mark.parametrize("V", [1, 65, 70001, (1 << 22) + 3])
+@pytest.mark.parametrize("relabel", [False, True])
+def test_results_in_page_locked_memory(V, relabel):
+    import ctypes
+    import torch
+
+    rng = np.random.default_rng(V)
+    n = min(2 * V, 200000)
+    g = W.from_edges(V, rng.integers(0, V, n), rng.integers(0, V, n), rng.integers(1, 9, n).astype(np.uint32))
+    c = W.Context(0, relabel=relabel)
+    lib, h = c._lib, c.handle
+
+    def check(read, want):
+        want = np.ascontiguousarray(want)
+        for before, after in ((0, 64), (64, 0), (want.itemsize, want.itemsize), (want.itemsize // 2 + 1, 64)):
+            mem = torch.full((before + want.nbytes + after,), 0x5A, dtype=torch.uint8).pin_memory()
+            assert read(ctypes.c_void_p(mem.data_ptr() + before)) == 0
+            b = mem.numpy()
+            assert b[before:before + want.nbytes].tobytes() == want.tobytes(), (before, after)
+            assert (b[:before] == 0x5A).all() and (b[before + want.nbytes:] == 0x5A).all()
+
+    def as_(t, f, *a):
+        return lambda p: f(h, *a, ctypes.cast(p, ctypes.POINTER(t)))
+
+    try:
+        c.load(g)
+        c.init_bfs(0)
+        c.converge(W.SCHED_FRONTIER)
+        check(as_(ctypes.c_uint64, lib.wg_read_bfs), c.read_bfs())
+        c.init_sssp(0)
+        c.converge(W.SCHED_FRONTIER)
+        check(lambda p: lib.wg_read_sssp(h, p), c.read_sssp())
+        ranks, _ = c.run_pr(iterations=2)
+        check(as_(ctypes.c_double, lib.wg_read_ranks), ranks)
+        if V > 1 << 20:
+            return
+        roots = np.array([0, V - 1], np.uint64)
+        c.msbfs(roots)
+        check(as_(ctypes.c_uint32, lib.wg_read_msbfs, 1), c.read_msbfs(1))
+        c.mssssp(roots)
+        check(lambda p: lib.wg_read_mssssp(h, 1, p), c.read_mssssp(1))
+        c.ppr(roots, 2, 0.85)
+        check(as_(ctypes.c_double, lib.wg_read_ppr, 1), c.read_ppr(1))
+    finally:
+        c.close()

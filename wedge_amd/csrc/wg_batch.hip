@@ -534,7 +534,7 @@ extern "C" int wg_read_msbfs(wg_ctx* ctx, uint32_t source, uint32_t* host_depths
     if (source >= ctx->ms_n)
         return WG_E_RANGE;
     void* stage = nullptr;
-    int rc = wg_stage(ctx, ctx->V * sizeof(uint32_t), &stage);
+    int rc = wg_result_dst(ctx, host_depths, ctx->V, sizeof(uint32_t), &stage);
     if (rc)
         return rc;
     hipLaunchKernelGGL(k_ms_column, dim3(wg_grid(ctx, ctx->V, 1024, 8)), dim3(256), 0, ctx->stream,
@@ -966,7 +966,7 @@ extern "C" int wg_read_mssssp(wg_ctx* ctx, uint32_t source, void* host_dist)
         return WG_E_RANGE;
     const size_t esz = ctx->wkind == WG_WEIGHT_F64 ? 8 : 4;
     void* stage = nullptr;
-    int rc = wg_stage(ctx, ctx->V * esz, &stage);
+    int rc = wg_result_dst(ctx, host_dist, ctx->V, esz, &stage);
     if (rc)
         return rc;
     const uint32_t grid = wg_grid(ctx, ctx->V, 1024, 8);

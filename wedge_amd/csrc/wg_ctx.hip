@@ -379,9 +379,45 @@ int wg_stage(wg_ctx* ctx, size_t bytes, void** out)
     return WG_OK;
 }
 
+// Whether a kernel may store `bytes` of elements of esz bytes at host: page-locked
+// memory of this device at its own address, all of it inside the allocation.
+static bool host_mapped(wg_ctx* ctx, void* host, size_t bytes, size_t esz)
+{
+    hipPointerAttribute_t at;
+    void* base = nullptr;
+    size_t size = 0;
+    const bool known = hipPointerGetAttributes(&at, host) == hipSuccess && at.type == hipMemoryTypeHost &&
+                       at.device == ctx->device && at.devicePointer == host &&
+                       hipPointerGetAttribute(&base, HIP_POINTER_ATTRIBUTE_RANGE_START_ADDR, host) == hipSuccess &&
+                       hipPointerGetAttribute(&size, HIP_POINTER_ATTRIBUTE_RANGE_SIZE, host) == hipSuccess;
+    if (!known) {
+        (void)hipGetLastError(); // an address the runtime does not know is no error here
+        return false;
+    }
+    const uintptr_t h = (uintptr_t)host, b = (uintptr_t)base;
+    return h % esz == 0 && h >= b && bytes <= size && h - b <= size - bytes;
+}
+
+// Where a kernel that stores n results in the caller's order puts them.  Up to
+// 32 MiB of page-locked memory takes its stores themselves, which leaves out a pass
+// and a launch (the copy is a kernel that stores over the same link); anything else
+// gets the stage and a copy.  Staged and direct, us: 2^16, 2^18, 2^20, 2^22, 2^24
+// ranks 31/22, 59/50, 176/170, 646/645, 2539/2556 (the copy's wider stores win once
+// the link is all that counts); a 64-source depth column of 2^18 vertices 42/32.
+#define WG_DIRECT_MAX ((size_t)32 << 20)
+int wg_result_dst(wg_ctx* ctx, void* host, uint64_t n, size_t esz, void** out)
+{
+    if (n <= WG_DIRECT_MAX / esz && host_mapped(ctx, host, (size_t)n * esz, esz)) {
+        *out = host;
+        return WG_OK;
+    }
+    return wg_stage(ctx, (size_t)n * esz, out);
+}
+
 int wg_copy_out(wg_ctx* ctx, const void* dev, void* host, size_t bytes)
 {
-    WG_HIP(ctx, hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, ctx->stream));
+    if (dev != host)
+        WG_HIP(ctx, hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, ctx->stream));
     WG_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return WG_OK;
 }
@@ -391,7 +427,7 @@ int wg_read_vertex_array(wg_ctx* ctx, const void* dev, void* host, size_t esz)
     if (!ctx->inv)
         return wg_copy_out(ctx, dev, host, ctx->V * esz);
     void* stage = nullptr;
-    int rc = wg_stage(ctx, ctx->V * esz, &stage);
+    int rc = wg_result_dst(ctx, host, ctx->V, esz, &stage);
     if (rc)
         return rc;
     const uint32_t grid = wg_grid(ctx, ctx->V, 1024, 8);

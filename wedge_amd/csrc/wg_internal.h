@@ -368,7 +368,9 @@ int wg_to_device_ids(wg_ctx* ctx, const uint64_t* orig, uint32_t n, uint32_t* ou
 int wg_read_vertex_array(wg_ctx* ctx, const void* dev, void* host, size_t elem_size);
 // a kept device array of at least `bytes` for results on their way to the host
 int wg_stage(wg_ctx* ctx, size_t bytes, void** out);
-// device to host, waited for
+// where a kernel stores n results of esz bytes bound for host: host itself or the stage
+int wg_result_dst(wg_ctx* ctx, void* host, uint64_t n, size_t esz, void** out);
+// device to host (nothing to copy if dev is host: wg_result_dst), waited for
 int wg_copy_out(wg_ctx* ctx, const void* dev, void* host, size_t bytes);
 // edge tiles of at most tile_edges edges (and WG_TILE_VERTS destinations)
 void wg_build_tiles(const uint32_t* off, uint64_t V, uint32_t tile_edges, std::vector<uint32_t>& tv,

@@ -413,7 +413,7 @@ extern "C" int wg_read_ppr(wg_ctx* ctx, uint32_t seed, double* host_ranks)
     if (seed >= ctx->ms_n)
         return WG_E_RANGE;
     void* stage = nullptr;
-    int rc = wg_stage(ctx, ctx->V * sizeof(double), &stage);
+    int rc = wg_result_dst(ctx, host_ranks, ctx->V, sizeof(double), &stage);
     if (rc)
         return rc;
     hipLaunchKernelGGL(k_ppr_column, dim3(wg_grid(ctx, ctx->V, 1024, 8)), dim3(256), 0, ctx->stream,

@@ -420,7 +420,7 @@ extern "C" int wg_read_ranks(wg_ctx* ctx, double* host_ranks)
     if (!ctx || ctx->app != WG_APP_PR || !host_ranks)
         return WG_E_STATE;
     void* stage = nullptr;
-    int rc = wg_stage(ctx, ctx->V * sizeof(double), &stage);
+    int rc = wg_result_dst(ctx, host_ranks, ctx->V, sizeof(double), &stage);
     if (rc)
         return rc;
     const double N = (double)ctx->V;
