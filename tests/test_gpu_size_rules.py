@@ -227,7 +227,6 @@ def test_sssp_rounds_in_one_workgroup(graph, kind):
 @pytest.mark.parametrize("relabel", [False, True])
 def test_results_in_page_locked_memory(V, relabel):
     import ctypes
-    import torch
 
     rng = np.random.default_rng(V)
     n = min(2 * V, 200000)
@@ -238,11 +237,17 @@ def test_results_in_page_locked_memory(V, relabel):
     def check(read, want):
         want = np.ascontiguousarray(want)
         for before, after in ((0, 64), (64, 0), (want.itemsize, want.itemsize), (want.itemsize // 2 + 1, 64)):
-            mem = torch.full((before + want.nbytes + after,), 0x5A, dtype=torch.uint8).pin_memory()
-            assert read(ctypes.c_void_p(mem.data_ptr() + before)) == 0
-            b = mem.numpy()
-            assert b[before:before + want.nbytes].tobytes() == want.tobytes(), (before, after)
-            assert (b[:before] == 0x5A).all() and (b[before + want.nbytes:] == 0x5A).all()
+            size = before + want.nbytes + after
+            mem = ctypes.c_void_p()
+            assert lib.hipHostMalloc(ctypes.byref(mem), ctypes.c_size_t(size), ctypes.c_uint(0)) == 0
+            try:
+                b = np.ctypeslib.as_array(ctypes.cast(mem, ctypes.POINTER(ctypes.c_uint8)), (size,))
+                b[:] = 0x5A
+                assert read(ctypes.c_void_p(mem.value + before)) == 0
+                assert b[before:before + want.nbytes].tobytes() == want.tobytes(), (before, after)
+                assert (b[:before] == 0x5A).all() and (b[before + want.nbytes:] == 0x5A).all()
+            finally:
+                assert lib.hipHostFree(mem) == 0
 
     def as_(t, f, *a):
         return lambda p: f(h, *a, ctypes.cast(p, ctypes.POINTER(t)))

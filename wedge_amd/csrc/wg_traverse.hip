@@ -2586,17 +2586,28 @@ static int clear_wedge_state(wg_ctx* ctx)
     return rc;
 }
 
+// A device array that a traversal can do without: null if there is no room.
+static void* optional_array(size_t bytes)
+{
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess)
+        return p;
+    (void)hipGetLastError();
+    return nullptr;
+}
+
 // Vertex records, far lists and the mean weight for the SSSP rounds of one
-// workgroup (once per graph; 64 bytes per vertex and 8 MiB).
+// workgroup (once per graph; 64 bytes per vertex and 8 MiB).  Without room for
+// them the pulls take every iteration.
 static int build_solo_sssp(wg_ctx* ctx)
 {
     double *sum = nullptr, total = 0.0;
     WG_HIP(ctx, hipMalloc((void**)&sum, sizeof(double)));
-    uint4* rec = nullptr;
-    if (!ctx->solo_far && hipMalloc((void**)&ctx->solo_far, 2ull * SOLO_FAR * sizeof(uint32_t)) != hipSuccess)
-        ctx->solo_far = nullptr;
-    hipError_t e = ctx->solo_far ? hipMalloc((void**)&rec, ctx->V * 4 * sizeof(uint4)) : hipErrorOutOfMemory;
-    if (e == hipSuccess) {
+    if (!ctx->solo_far)
+        ctx->solo_far = (uint32_t*)optional_array(2ull * SOLO_FAR * sizeof(uint32_t));
+    uint4* rec = ctx->solo_far ? (uint4*)optional_array(ctx->V * 4 * sizeof(uint4)) : nullptr;
+    hipError_t e = hipSuccess;
+    if (rec) {
         const dim3 gv(wg_grid(ctx, ctx->V, 256, 8)), ge(wg_grid(ctx, ctx->E, 4096, 4)), blk(WG_BLOCK);
         const uint64_t one = 0;
         (void)hipMemcpyAsync(sum, &one, sizeof(double), hipMemcpyHostToDevice, ctx->stream);
@@ -2622,6 +2633,8 @@ static int build_solo_sssp(wg_ctx* ctx)
         return WG_E_HIP;
     }
     ctx->solo_wrec = rec;
+    if (!rec)
+        return WG_OK;
     const double mean = total / (double)ctx->E;
     ctx->solo_delta = mean > 0.0 && mean < 1e300 ? 4.0 * mean : 1.0;
     return WG_OK;
@@ -2754,11 +2767,13 @@ static int init_common(wg_ctx* ctx, int app, size_t esz, int kind, uint64_t valu
         ctx->E <= ctx->V * SOLO_MEAN_DEGREE && (rc = build_solo_sssp(ctx)))
         return rc;
     // vertex records for the levels of one workgroup, on graphs with few
-    // out-edges per vertex (once per graph; 32 bytes per vertex)
+    // out-edges per vertex (once per graph; 32 bytes per vertex; without room
+    // for them those levels take the other kernels)
     if (app == WG_APP_BFS && !ctx->solo_rec && ctx->E <= ctx->V * SOLO_MEAN_DEGREE) {
-        WG_HIP(ctx, hipMalloc((void**)&ctx->solo_rec, ctx->V * 2 * sizeof(uint4)));
-        hipLaunchKernelGGL(k_solo_rec, dim3(wg_grid(ctx, ctx->V, 256, 8)), dim3(256), 0, ctx->stream, ctx->csri_off,
-                           ctx->csr_dst, ctx->V, ctx->solo_rec);
+        ctx->solo_rec = (uint4*)optional_array(ctx->V * 2 * sizeof(uint4));
+        if (ctx->solo_rec)
+            hipLaunchKernelGGL(k_solo_rec, dim3(wg_grid(ctx, ctx->V, 256, 8)), dim3(256), 0, ctx->stream, ctx->csri_off,
+                               ctx->csr_dst, ctx->V, ctx->solo_rec);
         if ((rc = wg_check_launch(ctx)))
             return rc;
     }
