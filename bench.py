@@ -187,8 +187,11 @@ def schedule_pair(ctx, g, root, reps, wbytes, orc=None):
         for sched in ("plain", "learned"):
             r, st, work, fused = run_best(ctx, app, root, reps, schedule=sched)
             res[sched] = (r, st)
+            # SSSP rounds of one workgroup (at most 4 edges per vertex) queue
+            # their vertices too: no bitmap per iteration
+            queued = st["iterations"] if app == "sssp" and g.num_edges <= 4 * g.num_vertices else fused
             out[f"{app}_{sched}"] = traversal_entry(app, g.num_vertices, st, work, 0 if app == "bfs" else wbytes,
-                                                    ctx.validate(), fused)
+                                                    ctx.validate(), queued)
             out[f"{app}_{sched}"]["fused_levels"] = fused
         out[f"{app}_learned_vs_plain"] = round(res["plain"][1]["running_ms"] / res["learned"][1]["running_ms"], 3)
         out[f"{app}_identical"] = bool(np.array_equal(res["plain"][0], res["learned"][0]))
