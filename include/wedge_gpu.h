@@ -247,7 +247,8 @@ typedef struct wg_loop_params {
     int schedule;
     uint32_t threshold_pct;  /* plain rule: dense iff activity > E * pct / 100 */
     int block_log2;          /* Wedge granularity of the plain rule */
-    uint32_t max_iterations; /* 0 = until convergence */
+    uint32_t max_iterations; /* 0 = until convergence; k: at most k pulls, after which a BFS or SSSP
+                                has taken every path of k edges from its roots into account */
 } wg_loop_params;
 int wg_converge(wg_ctx* ctx, const wg_loop_params* params, uint64_t* iterations, uint64_t* frontier_iterations);
 /* *on = 1 if the initialised CC / SSSP's dense pulls run on the binned layout
@@ -270,9 +271,11 @@ int wg_dense_pull_binned(const wg_ctx* ctx, int* on);
  * fewer iterations).  Default: BFS with 32 workgroups, CC and SSSP off.
  * On graphs with at most 4 edges per vertex, levels that suit one workgroup run
  * inside the decision kernel: BFS levels of up to 2048 vertices (counted as
- * fused; with workgroups >= 2), and, unless SSSP is in apps, SSSP rounds that
- * take the activated vertices nearest first (distances unchanged, each round an
- * iteration and a frontier iteration). */
+ * fused; with workgroups >= 2), and SSSP rounds that take the activated vertices
+ * nearest first (distances unchanged, each round an iteration and a frontier
+ * iteration, so there are several times as many).  The SSSP rounds are not taken
+ * by a loop with max_iterations, nor once this function was called with SSSP in
+ * apps, whatever the workgroups. */
 int wg_set_fused_levels(wg_ctx* ctx, uint32_t workgroups, uint32_t apps);
 /* Iterations of the last wg_converge that ran fused (included in its
  * iteration counts). */

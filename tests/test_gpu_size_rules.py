@@ -220,6 +220,47 @@ def test_sssp_rounds_in_one_workgroup(graph, kind):
             c.close()
 
 
+def _hop_distances(g, w, root, k):
+    """Shortest distances over paths of at most k edges (unreached: infinite)."""
+    d = np.full(g.num_vertices, np.inf)
+    d[root] = 0.0
+    dst = g.destinations()
+    for _ in range(k):
+        new = d.copy()
+        np.minimum.at(new, dst, d[g.sources] + w)
+        d = new
+    return d
+
+
+# at most 4 out-edges per vertex, where a loop without a cap takes nearest-first
+# rounds; integer weights below 2^32 and their sums are exact in FP64
+@pytest.mark.parametrize("graph", ["grid", "fan"])
+@pytest.mark.parametrize("cap", [1, 3, 24])
+def test_sssp_after_capped_pulls(graph, cap):
+    g = W.grid(61, 83, seed=4) if graph == "grid" else _broom(300)
+    root = g.max_outdegree_vertex() if graph == "grid" else 0
+    for w in _weighted(g, "random", 6):
+        bound = _hop_distances(g, w.astype(np.float64), root, cap)
+        gw = W.Graph(g.offsets, g.sources, w)
+        best = oracle.Oracle.of(gw, 8).sssp(root)[0]
+        c = W.Context(0)
+        try:
+            c.load(gw)
+            for schedule in (W.SCHED_FRONTIER, W.SCHED_PLAIN, W.SCHED_DENSE):
+                c.init_sssp(root)
+                assert c.converge(schedule, max_iterations=cap)[0] <= cap
+                got = c.read_sssp()
+                if w.dtype == np.uint32:
+                    best_f = np.where(best == np.uint64(2**64 - 1), np.inf, best.astype(np.float64))
+                    got = np.where(got == np.uint32(0xFFFFFFFF), np.inf, got.astype(np.float64))
+                else:
+                    best_f = best
+                assert (got <= bound).all(), (w.dtype, schedule)
+                assert (got >= best_f).all(), (w.dtype, schedule)
+        finally:
+            c.close()
+
+
 # page-locked memory: at an allocation's start, inside one, ending with one, at
 # no multiple of the element size (copied), and over 32 MiB (copied); the
 # elements around the result keep their value

@@ -188,6 +188,7 @@ struct wg_ctx {
     uint4* solo_wrec;         // SSSP: the same with weights (built by the first SSSP init)
     uint32_t* solo_far;       // SSSP: far lists of the rounds of one workgroup
     double solo_delta;        // and their first step between cutoffs
+    bool solo_sssp;           // the running wg_converge takes such rounds
     uint32_t* bfs_heavy_v;
     uint32_t* bfs_heavy_e;    // chunk start edge (chunk end = min(start + WG_BFS_HEAVY, off[v+1]))
     uint32_t n_out_pos;       // vertices with out-degree > 0

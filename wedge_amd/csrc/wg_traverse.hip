@@ -2226,7 +2226,6 @@ __device__ void sssp_solo(sssp_lds<typename P::T>& L, const uint32_t* __restrict
         return;
     run_state st;
     st.g = read_cfg(ctr);
-    st.max_iters = ctr->max_iters;
     st.iters = ctr->iters;
     st.fiters = ctr->fiters;
     st.unvisited = ctr->unvisited;
@@ -2445,7 +2444,7 @@ __device__ void sssp_solo(sssp_lds<typename P::T>& L, const uint32_t* __restrict
         }
         cur = nxt;
         __syncthreads();
-        if (full || nf > SOLO_PENDING || rounds >= SOLO_ROUNDS || (st.max_iters && st.iters >= st.max_iters))
+        if (full || nf > SOLO_PENDING || rounds >= SOLO_ROUNDS)
             break;
     }
     // what waits goes back to next, counted as the pulls count it (a vertex that
@@ -2468,7 +2467,7 @@ __device__ void sssp_solo(sssp_lds<typename P::T>& L, const uint32_t* __restrict
     __syncthreads();
     const unsigned long long A = L.act, F = L.fresh;
     st.unvisited = st.unvisited >= F ? st.unvisited - F : 0ull;
-    stop = stop || (A == 0ull && !full) || (st.max_iters && st.iters >= st.max_iters);
+    stop = stop || (A == 0ull && !full);
     int mode = 0, blog2 = st.g.plain_blog2;
     if (!stop && tid < WG_WAVE)
         loop_choose_wave(st.g, mlp, A, n + nf, st.iters, st.unvisited, &mode, &blog2);
@@ -3309,7 +3308,7 @@ static int enqueue_iteration(wg_ctx* ctx)
         hipLaunchKernelGGL(WG_CW(ctx, k_decide_bfs), dim3(1), dim3(SOLO_T), 0, ctx->stream, ctx->ctr, mlp, ctx->run_ctl,
                            ctx->csri_off, ctx->csr_dst, ctx->solo_rec, ctx->bm_next, ctx->bm_visited, packed,
                            ctx->bm_words, ctx->perm);
-    } else if (ctx->app == WG_APP_SSSP && ctx->solo_wrec && !((ctx->run_set >> WG_APP_SSSP) & 1u) && !wg_pb_min_on(ctx)) {
+    } else if (ctx->solo_sssp) {
 #define WG_DECIDE_SSSP(P, T)                                                                                           \
     hipLaunchKernelGGL(WG_CW(ctx, k_decide_sssp, P), dim3(1), dim3(SOLO_T), 0, ctx->stream, ctx->ctr, mlp,             \
                        ctx->csri_off, ctx->csri_pos, ctx->dst, ctx->w, ctx->solo_wrec, (T*)ctx->prop[0], ctx->bm_next, \
@@ -3420,6 +3419,11 @@ extern "C" int wg_converge(wg_ctx* ctx, const wg_loop_params* p, uint64_t* itera
     ctx->push_roots =
         (ctx->app == WG_APP_BFS && ctx->roots_frontier && ctx->nroots <= WG_PUSH_ROOTS_MAX) ? ctx->nroots : 0u;
     ctx->roots_frontier = 0;
+    // A round of one workgroup relaxes the nearest vertices only, so a loop that
+    // stops after k iterations takes the pulls: after k of them every distance is at
+    // most that of the best path of k edges.
+    ctx->solo_sssp = ctx->app == WG_APP_SSSP && ctx->solo_wrec && !p->max_iterations &&
+                     !((ctx->run_set >> WG_APP_SSSP) & 1u) && !wg_pb_min_on(ctx);
     if (ctx->app != WG_APP_CC) { // the roots' blocks, if the first pull is frontier-filtered
         if (!ctx->push_roots) {
             hipLaunchKernelGGL(k_wedge_build, dim3(wg_wedge_build_grid(ctx)), dim3(WG_BLOCK), 0, ctx->stream,
