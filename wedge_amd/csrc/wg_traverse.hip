@@ -1003,11 +1003,16 @@ __global__ void k_loop_init(wg_dev_counters* c, const float* __restrict__ mlp, u
 }
 
 // End of a pull (one wavefront): fold the counts, account the iteration,
-// stop at zero activity, choose the next schedule.
-__device__ void decide_wave(wg_dev_counters* c, const float* __restrict__ mlp)
+// stop at zero activity, choose the next schedule.  Returns (to every lane)
+// whether the next level is frontier-filtered with at most max_nact vertices and
+// max_act out-edges.  Inlined by force: as a function of its own (several kernels
+// call it) it gets generic pointers, and an iteration of a loop of launches takes
+// 1-2 us longer (CC on a 300x401 grid, learned schedule: 17.9 -> 18.8 ms).
+__device__ __forceinline__ bool decide_wave(wg_dev_counters* c, const float* __restrict__ mlp,
+                                            unsigned long long max_nact = 0ull, unsigned long long max_act = 0ull)
 {
     if (c->done)
-        return;
+        return false;
     const unsigned long long act0 = c->activity, nact0 = c->activated, fresh0 = c->fresh;
     const unsigned int iters = c->iters + 1u, fiters = c->fiters + (c->mode == WG_MODE_FRONTIER ? 1u : 0u);
     const unsigned int max_iters = c->max_iters;
@@ -1022,8 +1027,9 @@ __device__ void decide_wave(wg_dev_counters* c, const float* __restrict__ mlp)
     int mode = 0, blog2 = g.plain_blog2;
     if (!stop)
         loop_choose_wave(g, mlp, act, nact, iters, unvisited, &mode, &blog2);
+    const bool within = !stop && mode == WG_MODE_FRONTIER && nact <= max_nact && act <= max_act;
     if (threadIdx.x != 0)
-        return;
+        return within;
     c->iters = iters;
     c->fiters = fiters;
     c->activity = 0ull;
@@ -1036,10 +1042,11 @@ __device__ void decide_wave(wg_dev_counters* c, const float* __restrict__ mlp)
     c->unvisited = unvisited;
     if (stop) {
         c->done = 1u;
-        return;
+        return false;
     }
     c->mode = (unsigned int)mode;
     c->blog2 = blog2;
+    return within;
 }
 
 // Also clears the counts of the fused-level run that may follow (rc, if any).
@@ -1845,15 +1852,14 @@ __global__ void k_solo_rec(const uint32_t* __restrict__ csri_off, const uint32_t
 }
 
 // BFS levels of one workgroup (all its SOLO_T threads), in the state that
-// decide_wave left; as k_bfs_run, which see for the rules.
+// decide_wave left, the first within SOLO_NACT and SOLO_ACT; as k_bfs_run, which
+// see for the rules.
 template <bool CW>
 __device__ void bfs_solo(solo_lds& L, const uint32_t* __restrict__ csri_off, const uint32_t* __restrict__ csr_dst,
                          const uint4* __restrict__ rec, uint64_t* __restrict__ next, uint64_t* __restrict__ visited,
                          uint64_t* __restrict__ packed, uint64_t nwords, const uint32_t* __restrict__ perm,
                          wg_dev_counters* __restrict__ ctr, const float* __restrict__ mlp)
 {
-    if (ctr->done || ctr->mode != WG_MODE_FRONTIER || ctr->last_activity > SOLO_ACT || ctr->last_activated > SOLO_NACT)
-        return;
     run_state st;
     st.g = read_cfg(ctr);
     st.max_iters = ctr->max_iters;
@@ -2068,8 +2074,12 @@ __global__ __launch_bounds__(SOLO_T) void k_decide_bfs(wg_dev_counters* __restri
                                                        uint64_t nwords, const uint32_t* __restrict__ perm)
 {
     __shared__ solo_lds L;
-    if (threadIdx.x < WG_WAVE)
-        decide_wave(c, mlp);
+    __shared__ bool s_enter; // through LDS: the control block is a memory round trip away
+    if (threadIdx.x < WG_WAVE) {
+        const bool enter = decide_wave(c, mlp, SOLO_NACT, SOLO_ACT);
+        if (threadIdx.x == 0)
+            s_enter = enter;
+    }
     if (threadIdx.x < 3) {
         rc->tail[threadIdx.x].v = 0ull;
         rc->act[threadIdx.x].v = 0ull;
@@ -2077,7 +2087,8 @@ __global__ __launch_bounds__(SOLO_T) void k_decide_bfs(wg_dev_counters* __restri
         rc->fresh[threadIdx.x].v = 0ull;
     }
     __syncthreads(); // the control block as the first wavefront left it
-    bfs_solo<CW>(L, csri_off, csr_dst, rec, next, visited, packed, nwords, perm, c, mlp);
+    if (s_enter)
+        bfs_solo<CW>(L, csri_off, csr_dst, rec, next, visited, packed, nwords, perm, c, mlp);
 }
 
 // ---- SSSP in one workgroup ----------------------------------------------------------
@@ -2222,8 +2233,6 @@ __device__ void sssp_solo(sssp_lds<typename P::T>& L, const uint32_t* __restrict
 {
     typedef typename P::T T;
     typedef solo_pol<P> S;
-    if (ctr->done || ctr->mode != WG_MODE_FRONTIER || ctr->last_activity > SOLO_SACT || ctr->last_activated > SOLO_SNACT)
-        return;
     run_state st;
     st.g = read_cfg(ctr);
     st.iters = ctr->iters;
@@ -2498,9 +2507,15 @@ __global__ __launch_bounds__(SOLO_T) void k_decide_sssp(wg_dev_counters* __restr
                                                         unsigned int* __restrict__ ovf)
 {
     __shared__ sssp_lds<typename P::T> L;
-    if (threadIdx.x < WG_WAVE)
-        decide_wave(c, mlp);
+    __shared__ bool s_enter;
+    if (threadIdx.x < WG_WAVE) {
+        const bool enter = decide_wave(c, mlp, SOLO_SNACT, SOLO_SACT);
+        if (threadIdx.x == 0)
+            s_enter = enter;
+    }
     __syncthreads(); // the control block as the first wavefront left it
+    if (!s_enter)
+        return;
     sssp_solo<CW, P>(L, csri_off, csri_pos, dst, (const typename solo_pol<P>::W*)w, rec, prop, next, nwords, far, delta, c,
                      ovf, mlp);
 }
