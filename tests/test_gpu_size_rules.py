@@ -220,6 +220,81 @@ def test_sssp_rounds_in_one_workgroup(graph, kind):
             c.close()
 
 
+def _hubs(degrees):
+    """Vertices with the given out-degrees one after another, two levels apart:
+    each leads to leaves of its own, the first of them to the next vertex."""
+    src, dst, n = [], [], 1
+    hub = 0
+    for d in degrees:
+        src.append(np.full(d, hub))
+        dst.append(np.arange(n, n + d))
+        src.append(np.array([n]))
+        dst.append(np.array([n + d]))
+        hub = n + d
+        n += d + 1
+    return W.from_edges(n, np.concatenate(src), np.concatenate(dst))
+
+
+def _many_lists(mids, degree, leaves):
+    """A root to `mids` vertices, each with `degree` random ones of `leaves`."""
+    rng = np.random.default_rng(9)
+    src = np.concatenate([np.zeros(mids, np.int64), np.repeat(np.arange(1, mids + 1), degree)])
+    dst = np.concatenate([np.arange(1, mids + 1), mids + 1 + rng.integers(0, leaves, mids * degree)])
+    return W.from_edges(mids + 1 + leaves, src, dst, dedup=True)
+
+
+# out-lists longer than a vertex's record: up to one chunk of 256 out-edges, one
+# more, several rounds of the 16 wavefronts, and for SSSP the longest that one
+# workgroup takes (65536) and one more
+@pytest.mark.parametrize("relabel", [False, True])
+def test_bfs_long_lists_in_one_workgroup(relabel):
+    g = _hubs([1, 7, 8, 9, 255, 256, 257, 511, 512, 513, 3000, 12287, 12288, 12289, 20])
+    _, depth, _ = oracle.Oracle.of(g, 4).bfs(0)
+    c = W.Context(0, relabel=relabel)
+    try:
+        c.load(g)
+        for schedule in (W.SCHED_FRONTIER, W.SCHED_PLAIN):
+            got = []
+            for wgs in (0, 32):
+                c.set_fused_levels(wgs)
+                c.init_bfs(0)
+                got.append((c.converge(schedule), c.read_bfs()))
+            assert got[0][0] == got[1][0], schedule
+            assert np.array_equal(got[0][1], got[1][1]), schedule
+            assert np.array_equal(W.bfs_depth(got[1][1]), depth), schedule
+    finally:
+        c.close()
+
+
+# many: 3000 vertices at one distance (equal weights), a chunk each, where a
+# round holds 2048
+@pytest.mark.parametrize("graph", ["hubs", "many"])
+def test_sssp_long_lists_in_one_workgroup(graph):
+    g = _hubs([1, 5, 6, 7, 8, 255, 256, 257, 513, 4097, 65536, 65537, 20]) if graph == "hubs" else \
+        _many_lists(3000, 9, 20000)
+    assert g.num_edges <= 4 * g.num_vertices
+    for kind in ("equal", "random"):
+        for w in _weighted(g, kind, 11):
+            gw = W.Graph(g.offsets, g.sources, w)
+            want = oracle.Oracle.of(gw, 8).sssp(0)[0]
+            if w.dtype == np.uint32:
+                want = np.where(want == np.uint64(2**64 - 1), np.uint64(0xFFFFFFFF), want).astype(np.uint32)
+            c = W.Context(0)
+            try:
+                c.load(gw)
+                its = []
+                for rounds in (True, False):
+                    if not rounds:
+                        c.set_fused_levels(0, (W.APP_SSSP,))
+                    c.init_sssp(0)
+                    its.append(c.converge(W.SCHED_FRONTIER)[0])
+                    assert np.array_equal(c.read_sssp(), want), (kind, w.dtype, rounds)
+                if graph == "hubs" and kind == "random":  # nearest first takes more, smaller rounds
+                    assert its[0] > its[1], its
+            finally:
+                c.close()
+
+
 def _hop_distances(g, w, root, k):
     """Shortest distances over paths of at most k edges (unreached: infinite)."""
     d = np.full(g.num_vertices, np.inf)

@@ -1194,7 +1194,9 @@ __global__ __launch_bounds__(WG_BLOCK) void k_level_advance(uint64_t* __restrict
 #define SOLO_Q SOLO_ACT    // queue entries: a level appends at most one per out-edge
 #define SOLO_MEAN_DEGREE 4u // records and such levels up to this many out-edges per vertex
 #define SOLO_REC 7u        // destinations in a vertex's record
-#define SOLO_NBIG (SOLO_ACT / (SOLO_REC + 1u))
+#define SOLO_LANE_EDGES 4u   // out-edges of a long list that a lane has in flight
+#define SOLO_CHUNK (SOLO_LANE_EDGES * WG_WAVE)
+#define SOLO_NBIG (SOLO_ACT / (SOLO_REC + 1u)) // chunks: ceil(d / SOLO_CHUNK) <= d / (SOLO_REC + 1) for d > SOLO_REC
 
 // x as a value the compiler knows nothing about, in its register now.  For
 // several loads or atomics in flight, each in a branch of its own: their
@@ -1827,10 +1829,39 @@ __device__ __forceinline__ void solo_append(uint32_t* q, uint32_t* tail, uint32_
             q[base + pre[j]] = v[j];
 }
 
+// A chunk of an out-list longer than a record: up to SOLO_CHUNK out-edges, taken
+// by one wavefront.  Cut into these, a hub's list is spread over the workgroup's
+// wavefronts and each has four edges per lane in flight.  Walked by one wavefront,
+// an edge per lane, lists of 12000 out-edges made an SSSP slower than the pulls are
+// (80 such vertices one after another, learned schedule: pulls 16.8 ms, these
+// rounds 27.6, with chunks 10.4).
+struct solo_chunk {
+    uint32_t id; // BFS: the vertex in the caller's numbering; SSSP: the vertex
+    uint32_t first, count; // out-edge positions
+};
+
+__device__ __forceinline__ uint32_t solo_chunks(uint32_t degree)
+{
+    return degree / SOLO_CHUNK + (degree % SOLO_CHUNK ? 1u : 0u);
+}
+
+// Lists the chunks of out-edges [first, first + degree) at big[at], ..., those
+// below cap.
+__device__ __forceinline__ void solo_list(solo_chunk* big, uint32_t cap, uint32_t at, uint32_t id, uint32_t first,
+                                          uint32_t degree)
+{
+    for (uint32_t o = 0; o < degree && at < cap; o += SOLO_CHUNK, ++at) {
+        big[at].id = id;
+        big[at].first = first + o;
+        big[at].count = degree - o < SOLO_CHUNK ? degree - o : SOLO_CHUNK;
+    }
+}
+
 struct solo_lds {
     uint32_t q[2][SOLO_Q];
     uint32_t tail[2];
-    uint32_t nbig, big[SOLO_NBIG]; // vertices of the level with more out-edges than a record holds
+    uint32_t nbig; // chunks of the level's vertices with more out-edges than a record holds
+    solo_chunk big[SOLO_NBIG];
     uint32_t act[2];               // out-edges of the level's vertices
     int dec[2];
     float mlp[WG_MLP_OFF_END];     // the schedule model, under the learned schedule
@@ -1942,10 +1973,9 @@ __device__ void bfs_solo(solo_lds& L, const uint32_t* __restrict__ csri_off, con
                 work.dests += deg[k];
                 if (perm)
                     val = depth | (unsigned long long)perm[u[k]];
-                if (deg[k] > SOLO_REC) { // left to a wavefront
-                    const uint32_t b = atomicAdd(&L.nbig, 1u);
-                    if (b < SOLO_NBIG)
-                        L.big[b] = u[k];
+                if (deg[k] > SOLO_REC) { // left to the wavefronts
+                    solo_list(L.big, SOLO_NBIG, atomicAdd(&L.nbig, solo_chunks(deg[k])), (uint32_t)val, csri_off[u[k]],
+                              deg[k]);
                     deg[k] = 0u;
                 }
             }
@@ -1980,18 +2010,37 @@ __device__ void bfs_solo(solo_lds& L, const uint32_t* __restrict__ csri_off, con
         __syncthreads();
         if (const uint32_t nbig = L.nbig < SOLO_NBIG ? L.nbig : SOLO_NBIG) { // the same in the whole workgroup
             for (uint32_t b = tid / WG_WAVE; b < nbig; b += SOLO_WAVES) {
-                const uint32_t x = L.big[b], e = csri_off[x + 1];
-                const unsigned long long val = depth | (unsigned long long)(perm ? perm[x] : x);
-                for (uint32_t c = csri_off[x]; c < e; c += WG_WAVE) {
-                    uint32_t v[1] = {0u};
-                    bool nw[1] = {false};
-                    if (c + (uint32_t)lane < e) {
-                        v[0] = csr_dst[c + (uint32_t)lane];
-                        nw[0] = !((solo_load(&visited[v[0] >> 6]) >> (v[0] & 63u)) & 1ull) &&
-                                atomicMin((unsigned long long*)&packed[v[0]], val) == ~0ull;
-                    }
-                    solo_append<1>(qn, tn, SOLO_Q, v, nw);
+                const solo_chunk x = L.big[b];
+                const unsigned long long val = opaque(depth | (unsigned long long)x.id);
+                uint32_t v[SOLO_LANE_EDGES];
+                unsigned long long old[SOLO_LANE_EDGES];
+                bool nw[SOLO_LANE_EDGES];
+#pragma unroll
+                for (uint32_t j = 0; j < SOLO_LANE_EDGES; ++j) {
+                    const uint32_t o = j * WG_WAVE + (uint32_t)lane;
+                    v[j] = opaque_t(0u);
+                    if (o < x.count)
+                        v[j] = csr_dst[x.first + o];
                 }
+#pragma unroll
+                for (uint32_t j = 0; j < SOLO_LANE_EDGES; ++j) {
+                    old[j] = opaque(~0ull);
+                    if (j * WG_WAVE + (uint32_t)lane < x.count)
+                        old[j] = solo_load(&visited[v[j] >> 6]);
+                }
+#pragma unroll
+                for (uint32_t j = 0; j < SOLO_LANE_EDGES; ++j)
+                    nw[j] = !((old[j] >> (v[j] & 63u)) & 1ull);
+#pragma unroll
+                for (uint32_t j = 0; j < SOLO_LANE_EDGES; ++j) {
+                    old[j] = opaque(0ull);
+                    if (nw[j])
+                        old[j] = atomicMin((unsigned long long*)&packed[v[j]], val);
+                }
+#pragma unroll
+                for (uint32_t j = 0; j < SOLO_LANE_EDGES; ++j)
+                    nw[j] = old[j] == ~0ull;
+                solo_append<SOLO_LANE_EDGES>(qn, tn, SOLO_Q, v, nw);
             }
             __syncthreads();
         }
@@ -2108,7 +2157,7 @@ __global__ __launch_bounds__(SOLO_T) void k_decide_bfs(wg_dev_counters* __restri
 #define SOLO_NEAR 16384u     // near queue entries
 #define SOLO_PENDING 32768u  // far list entries (about) at which the workgroup hands back
 #define SOLO_FAR (1u << 20)  // capacity of each of the two far lists
-#define SOLO_SBIG 2048u
+#define SOLO_SBIG 2048u      // chunks of longer out-lists in a round
 #define SOLO_SNACT 16384u    // entered with at most so many activated vertices
 #define SOLO_SACT 65536u     // and out-edges
 #define SOLO_ROUNDS 16384u   // rounds per launch
@@ -2194,7 +2243,9 @@ template <typename T>
 struct sssp_lds {
     uint32_t q[2][SOLO_NEAR];
     uint32_t tail[2], ftail[2];
-    uint32_t nbig, big[SOLO_SBIG];
+    uint32_t nbig;
+    solo_chunk big[SOLO_SBIG];
+    uint32_t back;                 // vertices went back to next unrelaxed
     unsigned long long act, fresh; // at the end: out-edges of the waiting vertices, vertices first reached
     T least;                       // smallest distance left on the far list
 };
@@ -2247,6 +2298,7 @@ __device__ void sssp_solo(sssp_lds<typename P::T>& L, const uint32_t* __restrict
     }
     if (tid == 0) {
         L.nbig = 0u;
+        L.back = 0u;
         L.act = 0ull;
         L.fresh = 0ull;
         L.least = P::INF;
@@ -2376,12 +2428,16 @@ __device__ void sssp_solo(sssp_lds<typename P::T>& L, const uint32_t* __restrict
                 }
                 deg = x[0];
                 edges += deg;
-                if (deg > S::REC) { // left to a wavefront
-                    const uint32_t b = atomicAdd(&L.nbig, 1u);
-                    if (b < SOLO_SBIG)
-                        L.big[b] = u;
-                    else // no room: its own thread would be too slow, back to next
+                if (deg > S::REC) { // left to the wavefronts
+                    const uint32_t nch = solo_chunks(deg);
+                    // a list that one workgroup should not walk, or no room for all
+                    // its chunks (those there is room for are relaxed): back to next
+                    const uint32_t at = deg > SOLO_SACT ? SOLO_SBIG : atomicAdd(&L.nbig, nch);
+                    solo_list(L.big, SOLO_SBIG, at, u, csri_off[u], deg);
+                    if (at + nch > SOLO_SBIG) {
                         atomicOr((unsigned long long*)&next[u >> 6], 1ull << (u & 63u));
+                        L.back = 1u;
+                    }
                     deg = 0u;
                 }
             }
@@ -2414,25 +2470,45 @@ __device__ void sssp_solo(sssp_lds<typename P::T>& L, const uint32_t* __restrict
         __syncthreads();
         if (const uint32_t nb = L.nbig < SOLO_SBIG ? L.nbig : SOLO_SBIG) { // the same in the whole workgroup
             for (uint32_t b = tid / WG_WAVE; b < nb; b += SOLO_WAVES) {
-                const uint32_t u = L.big[b], e = csri_off[u + 1];
-                const T du = solo_load_t(&prop[u]);
-                for (uint32_t c = csri_off[u]; c < e; c += WG_WAVE) {
-                    uint32_t v[1] = {0u};
-                    T m[1] = {P::INF};
-                    bool up[1] = {false};
-                    if (c + (uint32_t)lane < e) {
-                        const uint32_t p = csri_pos[c + (uint32_t)lane];
-                        v[0] = dst[p];
-                        m[0] = S::add(du, w[p], ovf);
-                        if (m[0] < P::INF) {
-                            work.dests += 1ull;
-                            const T old = atomic_min_t<T>(&prop[v[0]], m[0]);
-                            up[0] = old > m[0];
-                            fresh += up[0] && old == P::INF ? 1ull : 0ull;
-                        }
-                    }
-                    sssp_put<1, T>(L, nxt, far[fi], fi, v, m, up, cutoff, next);
+                const solo_chunk x = L.big[b];
+                const T du = solo_load_t(&prop[x.id]);
+                uint32_t p[SOLO_LANE_EDGES], v[SOLO_LANE_EDGES];
+                typename S::W we[SOLO_LANE_EDGES];
+                T m[SOLO_LANE_EDGES], old[SOLO_LANE_EDGES];
+                bool up[SOLO_LANE_EDGES];
+#pragma unroll
+                for (uint32_t j = 0; j < SOLO_LANE_EDGES; ++j) {
+                    const uint32_t o = j * WG_WAVE + (uint32_t)lane;
+                    p[j] = opaque_t(0u);
+                    if (o < x.count)
+                        p[j] = csri_pos[x.first + o];
                 }
+#pragma unroll
+                for (uint32_t j = 0; j < SOLO_LANE_EDGES; ++j) {
+                    v[j] = opaque_t(0u);
+                    we[j] = opaque_t((typename S::W)0);
+                    if (j * WG_WAVE + (uint32_t)lane < x.count) {
+                        v[j] = dst[p[j]];
+                        we[j] = w[p[j]];
+                    }
+                }
+#pragma unroll
+                for (uint32_t j = 0; j < SOLO_LANE_EDGES; ++j)
+                    m[j] = j * WG_WAVE + (uint32_t)lane < x.count ? S::add(du, we[j], ovf) : P::INF;
+#pragma unroll
+                for (uint32_t j = 0; j < SOLO_LANE_EDGES; ++j) {
+                    old[j] = opaque_t(T(0));
+                    if (m[j] < P::INF) {
+                        work.dests += 1ull;
+                        old[j] = atomic_min_t<T>(&prop[v[j]], m[j]);
+                    }
+                }
+#pragma unroll
+                for (uint32_t j = 0; j < SOLO_LANE_EDGES; ++j) {
+                    up[j] = old[j] > m[j];
+                    fresh += up[j] && old[j] == P::INF ? 1ull : 0ull;
+                }
+                sssp_put<SOLO_LANE_EDGES, T>(L, nxt, far[fi], fi, v, m, up, cutoff, next);
             }
             __syncthreads();
         }
@@ -2442,7 +2518,7 @@ __device__ void sssp_solo(sssp_lds<typename P::T>& L, const uint32_t* __restrict
         rounds += 1u;
         st.iters += 1u;
         st.fiters += 1u;
-        full = L.tail[nxt] > SOLO_NEAR || L.ftail[fi] > SOLO_FAR || L.nbig > SOLO_SBIG;
+        full = L.tail[nxt] > SOLO_NEAR || L.ftail[fi] > SOLO_FAR || L.back;
         n = L.tail[nxt];
         n = n < SOLO_NEAR ? n : SOLO_NEAR;
         const uint32_t nf = L.ftail[fi];
