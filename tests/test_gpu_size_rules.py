@@ -266,6 +266,37 @@ def test_bfs_long_lists_in_one_workgroup(relabel):
         c.close()
 
 
+def test_bfs_small_levels_between_wide_ones():
+    """Fans of 3000 (more than one workgroup takes) with chains between them, short
+    of what a fused run waits for before it hands levels back, just that, and
+    several times as long: the run and the workgroup take turns."""
+    src, dst, n, at = [], [], 1, 0
+    for length in (1, 3, 7, 8, 9, 16, 17, 70, 8, 9, 40, 1):
+        src.append(np.full(3000, at))
+        dst.append(np.arange(n, n + 3000))
+        chain = np.concatenate([[n], np.arange(n + 3000, n + 3000 + length)])
+        src.append(chain[:-1])
+        dst.append(chain[1:])
+        n += 3000 + length
+        at = n - 1
+    g = W.from_edges(n, np.concatenate(src), np.concatenate(dst))
+    _, depth, _ = oracle.Oracle.of(g, 4).bfs(0)
+    c = W.Context(0)
+    try:
+        c.load(g)
+        got = []
+        for wgs in (0, 32, 2):
+            c.set_fused_levels(wgs)
+            c.init_bfs(0)
+            got.append((c.converge(W.SCHED_FRONTIER), c.read_bfs()))
+        for it, packed in got:
+            assert it == got[0][0]
+            assert np.array_equal(packed, got[0][1])
+            assert np.array_equal(W.bfs_depth(packed), depth)
+    finally:
+        c.close()
+
+
 # many: 3000 vertices at one distance (equal weights), a chunk each, where a
 # round holds 2048
 @pytest.mark.parametrize("graph", ["hubs", "many"])

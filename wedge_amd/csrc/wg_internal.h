@@ -136,6 +136,7 @@ struct wg_run_ctl {
     wg_run_line act[3];
     wg_run_line nact[3];
     wg_run_line fresh[3];
+    wg_run_line backs;   // BFS: times a run handed small levels back to the decision kernel
 };
 
 struct wg_prof {

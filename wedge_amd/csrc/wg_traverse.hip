@@ -1192,6 +1192,12 @@ __global__ __launch_bounds__(WG_BLOCK) void k_level_advance(uint64_t* __restrict
 #define SOLO_PER (SOLO_NACT / SOLO_T)
 #define SOLO_ACT 12288u
 #define SOLO_Q SOLO_ACT    // queue entries: a level appends at most one per out-edge
+// A run hands back after SOLO_AFTER small levels in a row, twice as many each
+// time until the workgroup ran SOLO_PAYS levels at a stretch (after every small
+// level: BFS over 400 vertices of 3000 out-edges, each two levels from the last,
+// 85 ms against 13.1 without a hand-back and 13.1 this way).
+#define SOLO_AFTER 8u
+#define SOLO_PAYS 64u
 #define SOLO_MEAN_DEGREE 4u // records and such levels up to this many out-edges per vertex
 #define SOLO_REC 7u        // destinations in a vertex's record
 #define SOLO_LANE_EDGES 4u   // out-edges of a long list that a lane has in flight
@@ -1364,6 +1370,7 @@ __device__ __forceinline__ void run_append(uint4* __restrict__ q, unsigned int* 
 struct run_state {
     loop_cfg g;
     unsigned int max_iters, level0, iters, fiters;
+    unsigned int small_levels, solo_after; // BFS: levels in a row that suit one workgroup, and at how many it gets them
     unsigned long long unvisited;
 };
 
@@ -1379,6 +1386,8 @@ __device__ __forceinline__ bool run_gate(const wg_dev_counters* ctr, run_state& 
     st.level0 = ctr->level;
     st.iters = ctr->iters;
     st.fiters = ctr->fiters;
+    st.small_levels = 0u;
+    st.solo_after = 0xffffffffu;
     st.unvisited = ctr->unvisited;
     return true;
 }
@@ -1475,7 +1484,7 @@ __device__ void run_entry(const uint64_t* __restrict__ act, uint64_t nwords, con
 __device__ __forceinline__ bool run_level_end(wg_run_ctl* __restrict__ rc, wg_dev_counters* __restrict__ ctr,
                                               unsigned int r, unsigned long long act, unsigned long long nact,
                                               unsigned long long fresh, run_state& st, const float* s_mlp, bool learned,
-                                              bool solo, bool* ok)
+                                              bool* ok)
 {
     const unsigned int rn = (r + 1u) % 3u, rz = (r + 2u) % 3u;
     __shared__ int s_dec[2];
@@ -1523,14 +1532,19 @@ __device__ __forceinline__ bool run_level_end(wg_run_ctl* __restrict__ rc, wg_de
     const int mode = stop ? 0 : s_dec[0];
     const int blog2 = stop ? st.g.plain_blog2 : s_dec[1];
     __syncthreads();
-    // a level that one workgroup does faster goes back to the decision kernel
-    // (if that takes levels; half of what it takes, so that a level near the line
-    // does not come straight back)
-    const bool small = solo && N <= SOLO_NACT / 2u && A <= SOLO_ACT / 2u;
+    // levels that one workgroup does faster (half of what it takes, so that a
+    // level near the line does not come straight back) go back to the decision
+    // kernel, if there were several in a row: the way there is a launch sequence,
+    // 100 us and more, and one workgroup saves a few us a level
+    const bool small = N <= SOLO_NACT / 2u && A <= SOLO_ACT / 2u;
+    st.small_levels = small ? st.small_levels + 1u : 0u;
+    const bool back = st.small_levels >= st.solo_after;
     const bool cont =
         !stop && mode == WG_MODE_FRONTIER && A <= WG_RUN_ACT_PER_WG * gridDim.x &&
-        N <= WG_RUN_NACT_PER_WG * gridDim.x && T <= WG_RUN_QCAP && !small;
+        N <= WG_RUN_NACT_PER_WG * gridDim.x && T <= WG_RUN_QCAP && !back;
     if (!cont && blockIdx.x == 0 && threadIdx.x == 0) {
+        if (back)
+            rc->backs.v += 1ull;
         ctr->iters = st.iters;
         ctr->fiters = st.fiters;
         ctr->last_activity = A;
@@ -1567,6 +1581,10 @@ __global__ __launch_bounds__(WG_BLOCK) void k_bfs_run(const uint32_t* __restrict
     run_state st;
     if (!run_gate(ctr, st))
         return;
+    if (solo) { // the same in every workgroup: it changes after the run's last barrier
+        const unsigned long long b = rc->backs.v;
+        st.solo_after = SOLO_AFTER << (b < 20ull ? (unsigned int)b : 20u);
+    }
     __shared__ float s_mlp[WG_MLP_OFF_END];
     const bool learned = run_stage_model(mlp, st, s_mlp);
     run_entry(next, nwords, csri_off, qa, rc);
@@ -1637,7 +1655,7 @@ __global__ __launch_bounds__(WG_BLOCK) void k_bfs_run(const uint32_t* __restrict
         add_work(work, ctr);
         work = work_tally<CW>();
         // a BFS activation is always a first visit
-        if (!run_level_end(rc, ctr, r, act, nact, nact, st, s_mlp, learned, solo, &ok))
+        if (!run_level_end(rc, ctr, r, act, nact, nact, st, s_mlp, learned, &ok))
             return;
         uint4* t = qc;
         qc = qn;
@@ -1735,7 +1753,7 @@ __global__ __launch_bounds__(WG_BLOCK) void k_min_run(const uint32_t* __restrict
         bool ok = true;
         add_work(work, ctr);
         work = work_tally<CW>();
-        if (!run_level_end(rc, ctr, r, act, nact, fresh, st, s_mlp, learned, false, &ok)) {
+        if (!run_level_end(rc, ctr, r, act, nact, fresh, st, s_mlp, learned, &ok)) {
             if (ok && (r & 1u) == 0u) // the last activations are in spare
                 for (uint64_t wd = (uint64_t)blockIdx.x * WG_BLOCK + threadIdx.x; wd < nwords;
                      wd += (uint64_t)gridDim.x * WG_BLOCK) {
@@ -1889,7 +1907,7 @@ template <bool CW>
 __device__ void bfs_solo(solo_lds& L, const uint32_t* __restrict__ csri_off, const uint32_t* __restrict__ csr_dst,
                          const uint4* __restrict__ rec, uint64_t* __restrict__ next, uint64_t* __restrict__ visited,
                          uint64_t* __restrict__ packed, uint64_t nwords, const uint32_t* __restrict__ perm,
-                         wg_dev_counters* __restrict__ ctr, const float* __restrict__ mlp)
+                         wg_run_ctl* __restrict__ rc, wg_dev_counters* __restrict__ ctr, const float* __restrict__ mlp)
 {
     run_state st;
     st.g = read_cfg(ctr);
@@ -2100,6 +2118,8 @@ __device__ void bfs_solo(solo_lds& L, const uint32_t* __restrict__ csri_off, con
             ctr->unvisited = st.unvisited;
             ctr->level = st.level0 + r + 1u;
             ctr->run_levels += r + 1u;
+            if (r + 1u >= SOLO_PAYS)
+                rc->backs.v = 0ull;
             if (stop) {
                 ctr->done = 1u;
             } else {
@@ -2137,7 +2157,7 @@ __global__ __launch_bounds__(SOLO_T) void k_decide_bfs(wg_dev_counters* __restri
     }
     __syncthreads(); // the control block as the first wavefront left it
     if (s_enter)
-        bfs_solo<CW>(L, csri_off, csr_dst, rec, next, visited, packed, nwords, perm, c, mlp);
+        bfs_solo<CW>(L, csri_off, csr_dst, rec, next, visited, packed, nwords, perm, rc, c, mlp);
 }
 
 // ---- SSSP in one workgroup ----------------------------------------------------------
