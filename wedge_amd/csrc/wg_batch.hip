@@ -362,7 +362,7 @@ __global__ void k_ms_column(const uint16_t* __restrict__ depth, const unsigned l
 
 static int ms_alloc(wg_ctx* ctx, size_t bytes, void** p)
 {
-    WG_HIP(ctx, hipMalloc(p, bytes ? bytes : 8));
+    WG_HIP(ctx, wg_dev_malloc(ctx, p, bytes ? bytes : 8));
     return WG_OK;
 }
 

@@ -270,8 +270,8 @@ static int run_checks(wg_ctx* ctx, int app, const void* vals, const uint32_t* dr
     uint64_t* ok = nullptr;
     uint64_t* rootbm = nullptr;
     unsigned long long* bad = nullptr;
-    if (hipMalloc((void**)&ok, words * 8) != hipSuccess || hipMalloc((void**)&rootbm, words * 8) != hipSuccess ||
-        hipMalloc((void**)&bad, sizeof(unsigned long long)) != hipSuccess) {
+    if (wg_dev_malloc(ctx, (void**)&ok, words * 8) != hipSuccess || wg_dev_malloc(ctx, (void**)&rootbm, words * 8) != hipSuccess ||
+        wg_dev_malloc(ctx, (void**)&bad, sizeof(unsigned long long)) != hipSuccess) {
         (void)hipFree(ok);
         (void)hipFree(rootbm);
         return WG_E_NOMEM;
@@ -367,8 +367,8 @@ extern "C" int wg_validate_values(wg_ctx* ctx, int app, const uint64_t* roots, u
     const uint64_t V = ctx->V;
     void *raw = nullptr, *dev = nullptr;
     uint32_t* droots = nullptr;
-    if (hipMalloc(&raw, V * esz) != hipSuccess || hipMalloc(&dev, V * esz) != hipSuccess ||
-        hipMalloc((void**)&droots, (nroots ? nroots : 1) * sizeof(uint32_t)) != hipSuccess) {
+    if (wg_dev_malloc(ctx, &raw, V * esz) != hipSuccess || wg_dev_malloc(ctx, &dev, V * esz) != hipSuccess ||
+        wg_dev_malloc(ctx, (void**)&droots, (nroots ? nroots : 1) * sizeof(uint32_t)) != hipSuccess) {
         (void)hipFree(raw);
         (void)hipFree(dev);
         return WG_E_NOMEM;

@@ -347,7 +347,7 @@ int wg_to_device_ids(wg_ctx* ctx, const uint64_t* orig, uint32_t n, uint32_t* ou
             (void)hipFree(ctx->idmap);
         ctx->idmap = nullptr;
         ctx->idmap_bytes = 0;
-        WG_HIP(ctx, hipMalloc(&ctx->idmap, need));
+        WG_HIP(ctx, wg_dev_malloc(ctx, &ctx->idmap, need));
         ctx->idmap_bytes = need;
     }
     uint64_t* din = (uint64_t*)ctx->idmap;
@@ -372,7 +372,7 @@ int wg_stage(wg_ctx* ctx, size_t bytes, void** out)
             (void)hipFree(ctx->stage);
         ctx->stage = nullptr;
         ctx->stage_bytes = 0;
-        WG_HIP(ctx, hipMalloc(&ctx->stage, bytes));
+        WG_HIP(ctx, wg_dev_malloc(ctx, &ctx->stage, bytes));
         ctx->stage_bytes = bytes;
     }
     *out = ctx->stage;
@@ -517,6 +517,27 @@ static void free_dev(void** p)
     }
 }
 
+hipError_t wg_dev_malloc(wg_ctx* ctx, void** p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && (ctx->solo_rec || ctx->solo_wrec || ctx->solo_far || ctx->stage)) {
+        (void)hipStreamSynchronize(ctx->stream);
+        // not built again for this graph: the next initialisation would take the room back
+        ctx->solo_none |= (ctx->solo_rec ? 1u << WG_APP_BFS : 0u) | (ctx->solo_wrec ? 1u << WG_APP_SSSP : 0u);
+        free_dev((void**)&ctx->solo_rec);
+        free_dev((void**)&ctx->solo_wrec);
+        free_dev((void**)&ctx->solo_far);
+        free_dev(&ctx->stage);
+        ctx->stage_bytes = 0;
+        e = hipMalloc(p, bytes);
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError(); // reported here: not by the next launch's check too
+        *p = nullptr;
+    }
+    return e;
+}
+
 int wg_free_app_state(wg_ctx* ctx)
 {
     free_dev(&ctx->prop[0]);
@@ -542,9 +563,9 @@ int wg_app_state(wg_ctx* ctx, int app, size_t bytes, int both)
         return WG_OK;
     WG_HIP(ctx, hipStreamSynchronize(ctx->stream));
     wg_free_app_state(ctx);
-    WG_HIP(ctx, hipMalloc(&ctx->prop[0], bytes));
+    WG_HIP(ctx, wg_dev_malloc(ctx, &ctx->prop[0], bytes));
     if (both)
-        WG_HIP(ctx, hipMalloc(&ctx->prop[1], bytes));
+        WG_HIP(ctx, wg_dev_malloc(ctx, &ctx->prop[1], bytes));
     ctx->prop_bytes = bytes;
     return WG_OK;
 }
@@ -591,6 +612,7 @@ static void free_graph(wg_ctx* ctx)
     free_dev((void**)&ctx->solo_rec);
     free_dev((void**)&ctx->solo_wrec);
     free_dev((void**)&ctx->solo_far);
+    ctx->solo_none = 0;
     free_dev((void**)&ctx->perm);
     free_dev((void**)&ctx->inv);
     free_dev(&ctx->stage);
@@ -641,7 +663,7 @@ extern "C" int wg_measure_copy(wg_ctx* ctx, uint64_t bytes, double* gb_per_s)
     hipEvent_t ev[2] = {nullptr, nullptr};
     int rc = WG_OK;
     float best = 0.0f;
-    if (hipMalloc(&a, n * 16) != hipSuccess || hipMalloc(&b, n * 16) != hipSuccess) {
+    if (wg_dev_malloc(ctx, &a, n * 16) != hipSuccess || wg_dev_malloc(ctx, &b, n * 16) != hipSuccess) {
         (void)hipFree(a);
         return WG_E_NOMEM;
     }
@@ -734,7 +756,7 @@ static void build_tiles(const uint32_t* off, uint64_t V, std::vector<uint32_t>& 
 template <typename T>
 static int upload(wg_ctx* ctx, T** dptr, const T* host, uint64_t n)
 {
-    WG_HIP(ctx, hipMalloc((void**)dptr, (n ? n : 1) * sizeof(T)));
+    WG_HIP(ctx, wg_dev_malloc(ctx, (void**)dptr, (n ? n : 1) * sizeof(T)));
     if (n && host)
         WG_HIP(ctx, hipMemcpy(*dptr, host, n * sizeof(T), hipMemcpyHostToDevice));
     return WG_OK;

@@ -190,6 +190,7 @@ struct wg_ctx {
     uint32_t* solo_far;       // SSSP: far lists of the rounds of one workgroup
     double solo_delta;        // and their first step between cutoffs
     bool solo_sssp;           // the running wg_converge takes such rounds
+    unsigned int solo_none;   // bit per application: no memory for its records on this graph
     uint32_t* bfs_heavy_v;
     uint32_t* bfs_heavy_e;    // chunk start edge (chunk end = min(start + WG_BFS_HEAVY, off[v+1]))
     uint32_t n_out_pos;       // vertices with out-degree > 0
@@ -354,6 +355,10 @@ uint32_t wg_frontier_grid(const wg_ctx* ctx);
 uint32_t wg_wedge_build_grid(const wg_ctx* ctx);
 uint32_t wg_advance_grid(const wg_ctx* ctx);
 int wg_pr_reset(wg_ctx* ctx);
+// hipMalloc for a context with a graph: where there is no room, the memory that
+// the context can do without (the vertex records of the one-workgroup levels, the
+// results' stage) is given up first
+hipError_t wg_dev_malloc(wg_ctx* ctx, void** p, size_t bytes);
 int wg_free_app_state(wg_ctx* ctx);
 // prop[0] (and prop[1] if `both`) of `bytes` for the application, kept if it is
 // the one whose state the context holds; else everything is released first

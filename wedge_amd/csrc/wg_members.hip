@@ -222,7 +222,7 @@ __global__ __launch_bounds__(WG_BLOCK) void k_bm_ranks(const uint32_t* __restric
 template <typename T>
 static int upload_vec(wg_ctx* ctx, T** d, const std::vector<T>& h)
 {
-    WG_HIP(ctx, hipMalloc((void**)d, (h.empty() ? 1 : h.size()) * sizeof(T)));
+    WG_HIP(ctx, wg_dev_malloc(ctx, (void**)d, (h.empty() ? 1 : h.size()) * sizeof(T)));
     if (!h.empty())
         WG_HIP(ctx, hipMemcpy(*d, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice));
     return WG_OK;
@@ -252,7 +252,7 @@ static int build_members(wg_ctx* ctx, wg_members* m, const uint64_t* first, uint
 
     // edges must stay inside their member
     unsigned int* bad = nullptr;
-    WG_HIP(ctx, hipMalloc((void**)&bad, sizeof(unsigned int)));
+    WG_HIP(ctx, wg_dev_malloc(ctx, (void**)&bad, sizeof(unsigned int)));
     unsigned int hbad = 0;
     hipError_t e0 = hipMemsetAsync(bad, 0, sizeof(unsigned int), ctx->stream);
     if (ctx->E && e0 == hipSuccess)
@@ -285,10 +285,10 @@ static int build_members(wg_ctx* ctx, wg_members* m, const uint64_t* first, uint
             (rc = upload_vec(ctx, &t.heavy_v, hv)) || (rc = upload_vec(ctx, &t.heavy_t, ht)))
             return rc;
     }
-    WG_HIP(ctx, hipMalloc((void**)&m->tile_part, (max_tiles + 1) * sizeof(double)));
-    WG_HIP(ctx, hipMalloc((void**)&m->chunk_part, 2 * (size_t)m->nchunks * sizeof(double)));
-    WG_HIP(ctx, hipMalloc((void**)&m->acc, (ctx->V ? ctx->V : 1) * sizeof(double)));
-    WG_HIP(ctx, hipMalloc((void**)&m->scratch, sizeof(double)));
+    WG_HIP(ctx, wg_dev_malloc(ctx, (void**)&m->tile_part, (max_tiles + 1) * sizeof(double)));
+    WG_HIP(ctx, wg_dev_malloc(ctx, (void**)&m->chunk_part, 2 * (size_t)m->nchunks * sizeof(double)));
+    WG_HIP(ctx, wg_dev_malloc(ctx, (void**)&m->acc, (ctx->V ? ctx->V : 1) * sizeof(double)));
+    WG_HIP(ctx, wg_dev_malloc(ctx, (void**)&m->scratch, sizeof(double)));
     WG_HIP(ctx, hipMemset(m->scratch, 0, sizeof(double)));
     return WG_OK;
 }
@@ -408,8 +408,8 @@ static int ensure_buffers(wg_ctx* ctx, wg_members* m, int fp32)
     m->cur = -1;
     const size_t esz = fp32 ? sizeof(float) : sizeof(double);
     const size_t n = ctx->V ? ctx->V : 1;
-    WG_HIP(ctx, hipMalloc(&m->c[0], n * esz));
-    WG_HIP(ctx, hipMalloc(&m->c[1], n * esz));
+    WG_HIP(ctx, wg_dev_malloc(ctx, &m->c[0], n * esz));
+    WG_HIP(ctx, wg_dev_malloc(ctx, &m->c[1], n * esz));
     m->c_fp32 = fp32;
     return WG_OK;
 }

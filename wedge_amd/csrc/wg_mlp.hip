@@ -40,7 +40,7 @@ extern "C" int wg_set_schedule_model(wg_ctx* ctx, const float* params, uint64_t 
         return WG_E_INVAL;
     WG_HIP(ctx, hipSetDevice(ctx->device));
     if (!ctx->mlp)
-        WG_HIP(ctx, hipMalloc((void**)&ctx->mlp, WG_MLP_PARAMS * sizeof(float)));
+        WG_HIP(ctx, wg_dev_malloc(ctx, (void**)&ctx->mlp, WG_MLP_PARAMS * sizeof(float)));
     WG_HIP(ctx, hipMemcpyAsync(ctx->mlp, params, WG_MLP_PARAMS * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
     WG_HIP(ctx, hipStreamSynchronize(ctx->stream));
     ctx->mlp_set = 1;
@@ -82,11 +82,11 @@ extern "C" int wg_mlp_infer(wg_ctx* ctx, int app, const float* features, const f
         for (uint64_t s = 0; s < n; ++s)
             if (plain[s] < -1 || plain[s] >= WG_MLP_ACTIONS)
                 return WG_E_RANGE;
-    if ((base && hipMalloc((void**)&dB, n * WG_MLP_ACTIONS * sizeof(float)) != hipSuccess) ||
-        (plain && hipMalloc((void**)&dPl, n * sizeof(int32_t)) != hipSuccess) ||
-        hipMalloc((void**)&dX, n * WG_MLP_IN * sizeof(float)) != hipSuccess ||
-        hipMalloc((void**)&dY, n * WG_MLP_ACTIONS * sizeof(float)) != hipSuccess ||
-        hipMalloc((void**)&dA, n * sizeof(int32_t)) != hipSuccess) {
+    if ((base && wg_dev_malloc(ctx, (void**)&dB, n * WG_MLP_ACTIONS * sizeof(float)) != hipSuccess) ||
+        (plain && wg_dev_malloc(ctx, (void**)&dPl, n * sizeof(int32_t)) != hipSuccess) ||
+        wg_dev_malloc(ctx, (void**)&dX, n * WG_MLP_IN * sizeof(float)) != hipSuccess ||
+        wg_dev_malloc(ctx, (void**)&dY, n * WG_MLP_ACTIONS * sizeof(float)) != hipSuccess ||
+        wg_dev_malloc(ctx, (void**)&dA, n * sizeof(int32_t)) != hipSuccess) {
         rc = WG_E_NOMEM;
         goto done;
     }
@@ -259,7 +259,7 @@ extern "C" int wg_mlp_train(wg_ctx* ctx, const float* features, const int32_t* a
     std::vector<void*> owned;
     auto dalloc = [&](size_t bytes) -> void* {
         void* p = nullptr;
-        if (hipMalloc(&p, bytes ? bytes : 4) != hipSuccess)
+        if (wg_dev_malloc(ctx, &p, bytes ? bytes : 4) != hipSuccess)
             return nullptr;
         owned.push_back(p);
         return p;

@@ -318,7 +318,7 @@ __global__ void k_pb_place(const uint16_t* __restrict__ pdst_w, uint32_t npairs,
 template <typename T>
 static int pb_upload(wg_ctx* ctx, T** d, const std::vector<T>& h)
 {
-    PB_TRY(hipMalloc((void**)d, (h.empty() ? 1 : h.size()) * sizeof(T)));
+    PB_TRY(wg_dev_malloc(ctx, (void**)d, (h.empty() ? 1 : h.size()) * sizeof(T)));
     if (!h.empty())
         PB_TRY(hipMemcpyAsync(*d, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice, ctx->stream));
     return WG_OK;
@@ -388,16 +388,16 @@ static int pb_build(wg_ctx* ctx, wg_pb* pb, int ws_log, int wd_log)
     std::vector<uint64_t> ws(S + 1, 0);
     const uint32_t g = wg_grid(ctx, E ? E : 1, 1024, 8);
     if (E) {
-        PB_TRY(hipMalloc(&key0.p, E * 2));
-        PB_TRY(hipMalloc(&key1.p, E * 2));
-        PB_TRY(hipMalloc(&idx0.p, E * 4));
-        PB_TRY(hipMalloc(&perm.p, E * 4));
+        PB_TRY(wg_dev_malloc(ctx, &key0.p, E * 2));
+        PB_TRY(wg_dev_malloc(ctx, &key1.p, E * 2));
+        PB_TRY(wg_dev_malloc(ctx, &idx0.p, E * 4));
+        PB_TRY(wg_dev_malloc(ctx, &perm.p, E * 4));
         hipLaunchKernelGGL(k_pb_keys, dim3(g), dim3(256), 0, st, ctx->src, E, ws_log, (uint16_t*)key0.p,
                            (uint32_t*)idx0.p);
         size_t tb = 0;
         PB_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, (const uint16_t*)key0.p, (uint16_t*)key1.p,
                                                   (const uint32_t*)idx0.p, (uint32_t*)perm.p, (uint64_t)E, 0, bits, st));
-        PB_TRY(hipMalloc(&tmp.p, tb ? tb : 1));
+        PB_TRY(wg_dev_malloc(ctx, &tmp.p, tb ? tb : 1));
         PB_TRY(hipcub::DeviceRadixSort::SortPairs(tmp.p, tb, (const uint16_t*)key0.p, (uint16_t*)key1.p,
                                                   (const uint32_t*)idx0.p, (uint32_t*)perm.p, (uint64_t)E, 0, bits, st));
         (void)hipFree(tmp.p);
@@ -406,7 +406,7 @@ static int pb_build(wg_ctx* ctx, wg_pb* pb, int ws_log, int wd_log)
         idx0.p = nullptr;
         (void)hipFree(key0.p);
         key0.p = nullptr;
-        PB_TRY(hipMalloc(&wsd.p, (S + 1) * sizeof(uint64_t)));
+        PB_TRY(wg_dev_malloc(ctx, &wsd.p, (S + 1) * sizeof(uint64_t)));
         hipLaunchKernelGGL(k_pb_window_starts, dim3((S + 256) / 256), dim3(256), 0, st, (const uint16_t*)key1.p, E, S,
                            (uint64_t*)wsd.p);
         PB_TRY(hipGetLastError());
@@ -452,7 +452,7 @@ static int pb_build(wg_ctx* ctx, wg_pb* pb, int ws_log, int wd_log)
     if (nq) {
         if ((rc = pb_upload(ctx, (uint32_t**)&twin.p, tile_win)) || (rc = pb_upload(ctx, (uint64_t**)&pqd.p, pq)))
             return rc;
-        PB_TRY(hipMalloc((void**)&pb->code, nq * sizeof(uint16_t)));
+        PB_TRY(wg_dev_malloc(ctx, (void**)&pb->code, nq * sizeof(uint16_t)));
         const uint32_t gq = wg_grid(ctx, nq, 1024, 8);
         hipLaunchKernelGGL(k_pb_codes, dim3(gq), dim3(256), 0, st, nq, (const uint32_t*)twin.p, (const uint64_t*)wsd.p,
                            (const uint64_t*)pqd.p, (const uint32_t*)perm.p, ctx->src, ctx->dst,
@@ -460,23 +460,23 @@ static int pb_build(wg_ctx* ctx, wg_pb* pb, int ws_log, int wd_log)
         PB_TRY(hipGetLastError());
         if (ctx->w && ctx->wkind != WG_WEIGHT_NONE) { // weights in code order, for the binned SSSP pull
             if (ctx->wkind == WG_WEIGHT_F64) {
-                PB_TRY(hipMalloc(&pb->wq, nq * sizeof(double)));
+                PB_TRY(wg_dev_malloc(ctx, &pb->wq, nq * sizeof(double)));
                 hipLaunchKernelGGL(k_pb_weights<double>, dim3(gq), dim3(256), 0, st, nq, (const uint32_t*)twin.p,
                                    (const uint64_t*)wsd.p, (const uint64_t*)pqd.p, (const uint32_t*)perm.p,
                                    (const double*)ctx->w, (double*)pb->wq);
             } else {
-                PB_TRY(hipMalloc(&pb->wq, nq * sizeof(uint32_t)));
+                PB_TRY(wg_dev_malloc(ctx, &pb->wq, nq * sizeof(uint32_t)));
                 hipLaunchKernelGGL(k_pb_weights<uint32_t>, dim3(gq), dim3(256), 0, st, nq, (const uint32_t*)twin.p,
                                    (const uint64_t*)wsd.p, (const uint64_t*)pqd.p, (const uint32_t*)perm.p,
                                    (const uint32_t*)ctx->w, (uint32_t*)pb->wq);
             }
             PB_TRY(hipGetLastError());
         }
-        PB_TRY(hipMalloc(&pidx.p, nq * sizeof(uint32_t)));
+        PB_TRY(wg_dev_malloc(ctx, &pidx.p, nq * sizeof(uint32_t)));
         hipcub::TransformInputIterator<uint32_t, pb_end_flag, const uint16_t*> flags(pb->code, pb_end_flag());
         size_t tb = 0;
         PB_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, tb, flags, (uint32_t*)pidx.p, (uint64_t)nq, st));
-        PB_TRY(hipMalloc(&tmp.p, tb ? tb : 1));
+        PB_TRY(wg_dev_malloc(ctx, &tmp.p, tb ? tb : 1));
         PB_TRY(hipcub::DeviceScan::ExclusiveSum(tmp.p, tb, flags, (uint32_t*)pidx.p, (uint64_t)nq, st));
         uint32_t last_idx = 0;
         uint16_t last_code = 0;
@@ -488,15 +488,15 @@ static int pb_build(wg_ctx* ctx, wg_pb* pb, int ws_log, int wd_log)
         npairs = last_idx + ((last_code & WG_PB_END) ? 1u : 0u);
     }
     pb->npairs = npairs;
-    PB_TRY(hipMalloc((void**)&pb->tile_pbase, ((uint64_t)pb->ntiles + 1) * sizeof(uint32_t)));
-    PB_TRY(hipMalloc((void**)&pb->pdst, (npairs ? npairs : 1) * sizeof(uint16_t)));
-    PB_TRY(hipMalloc((void**)&pb->part, (npairs ? npairs : 1) * sizeof(double)));
+    PB_TRY(wg_dev_malloc(ctx, (void**)&pb->tile_pbase, ((uint64_t)pb->ntiles + 1) * sizeof(uint32_t)));
+    PB_TRY(wg_dev_malloc(ctx, (void**)&pb->pdst, (npairs ? npairs : 1) * sizeof(uint16_t)));
+    PB_TRY(wg_dev_malloc(ctx, (void**)&pb->part, (npairs ? npairs : 1) * sizeof(double)));
     std::vector<uint32_t> bstart, bkey;
     if (nq) {
         hipLaunchKernelGGL(k_pb_tile_base, dim3(pb->ntiles / 256 + 1), dim3(256), 0, st, (const uint32_t*)pidx.p,
                            pb->ntiles, npairs, pb->tile_pbase);
-        PB_TRY(hipMalloc(&pkey.p, (npairs ? npairs : 1) * sizeof(uint32_t)));
-        PB_TRY(hipMalloc(&pdst_w.p, (npairs ? npairs : 1) * sizeof(uint16_t)));
+        PB_TRY(wg_dev_malloc(ctx, &pkey.p, (npairs ? npairs : 1) * sizeof(uint32_t)));
+        PB_TRY(wg_dev_malloc(ctx, &pdst_w.p, (npairs ? npairs : 1) * sizeof(uint16_t)));
         const uint32_t gq = wg_grid(ctx, nq, 1024, 8);
         hipLaunchKernelGGL(k_pb_pairs, dim3(gq), dim3(256), 0, st, nq, pb->code, (const uint32_t*)pidx.p,
                            (const uint32_t*)twin.p, (const uint64_t*)wsd.p, (const uint64_t*)pqd.p,
@@ -506,9 +506,9 @@ static int pb_build(wg_ctx* ctx, wg_pb* pb, int ws_log, int wd_log)
         perm.p = nullptr;
 
         // 4. blocks: runs of equal (window, bin) among the pairs
-        PB_TRY(hipMalloc(&bflag.p, npairs));
-        PB_TRY(hipMalloc(&bst.p, (uint64_t)npairs * 4));
-        PB_TRY(hipMalloc(&nsel.p, sizeof(uint64_t)));
+        PB_TRY(wg_dev_malloc(ctx, &bflag.p, npairs));
+        PB_TRY(wg_dev_malloc(ctx, &bst.p, (uint64_t)npairs * 4));
+        PB_TRY(wg_dev_malloc(ctx, &nsel.p, sizeof(uint64_t)));
         hipLaunchKernelGGL(k_pb_block_flags, dim3(wg_grid(ctx, npairs, 1024, 8)), dim3(256), 0, st,
                            (const uint32_t*)pkey.p, (uint64_t)npairs, (uint8_t*)bflag.p);
         PB_TRY(hipGetLastError());
@@ -518,7 +518,7 @@ static int pb_build(wg_ctx* ctx, wg_pb* pb, int ws_log, int wd_log)
         size_t tb = 0;
         PB_TRY(hipcub::DeviceSelect::Flagged(nullptr, tb, pos, (const uint8_t*)bflag.p, (uint32_t*)bst.p,
                                              (uint64_t*)nsel.p, (int64_t)npairs, st));
-        PB_TRY(hipMalloc(&tmp.p, tb ? tb : 1));
+        PB_TRY(wg_dev_malloc(ctx, &tmp.p, tb ? tb : 1));
         PB_TRY(hipcub::DeviceSelect::Flagged(tmp.p, tb, pos, (const uint8_t*)bflag.p, (uint32_t*)bst.p,
                                              (uint64_t*)nsel.p, (int64_t)npairs, st));
         uint64_t nb = 0;
@@ -526,7 +526,7 @@ static int pb_build(wg_ctx* ctx, wg_pb* pb, int ws_log, int wd_log)
         PB_TRY(hipStreamSynchronize(st));
         (void)hipFree(tmp.p);
         tmp.p = nullptr;
-        PB_TRY(hipMalloc(&bk.p, (nb ? nb : 1) * 4));
+        PB_TRY(wg_dev_malloc(ctx, &bk.p, (nb ? nb : 1) * 4));
         hipLaunchKernelGGL(k_pb_block_keys, dim3((uint32_t)(nb / 256 + 1)), dim3(256), 0, st, (const uint32_t*)bst.p,
                            (uint32_t)nb, (const uint32_t*)pkey.p, (uint32_t*)bk.p);
         PB_TRY(hipGetLastError());
@@ -614,10 +614,10 @@ static int pb_build(wg_ctx* ctx, wg_pb* pb, int ws_log, int wd_log)
                            (const uint16_t*)pdst_w.p, npairs, (const uint32_t*)bst.p, (uint32_t)nb,
                            (const uint32_t*)woffd.p, pb->pdst);
     PB_TRY(hipGetLastError());
-    PB_TRY(hipMalloc((void**)&pb->slot_acc, ((uint64_t)(nslots ? nslots : 1) << wd_log) * sizeof(double)));
-    PB_TRY(hipMalloc((void**)&pb->bin_ticket, B * sizeof(unsigned int)));
+    PB_TRY(wg_dev_malloc(ctx, (void**)&pb->slot_acc, ((uint64_t)(nslots ? nslots : 1) << wd_log) * sizeof(double)));
+    PB_TRY(wg_dev_malloc(ctx, (void**)&pb->bin_ticket, B * sizeof(unsigned int)));
     PB_TRY(hipMemsetAsync(pb->bin_ticket, 0, B * sizeof(unsigned int), st));
-    PB_TRY(hipMalloc((void**)&pb->bin_part, B * sizeof(double)));
+    PB_TRY(wg_dev_malloc(ctx, (void**)&pb->bin_part, B * sizeof(double)));
     PB_TRY(hipStreamSynchronize(st));
     return WG_OK;
 }

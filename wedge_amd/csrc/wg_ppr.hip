@@ -350,9 +350,9 @@ extern "C" int wg_ppr(wg_ctx* ctx, const uint64_t* seeds, uint32_t nseeds, uint3
         R = ctx->prop[0];
     } else {
         wg_free_app_state(ctx);
-        if (hipMalloc(&C0, V * PPR_LANES * sizeof(float)) != hipSuccess ||
-            hipMalloc(&C1, V * PPR_LANES * sizeof(float)) != hipSuccess ||
-            hipMalloc(&R, V * PPR_LANES * sizeof(double)) != hipSuccess || hipMalloc(&aux, aux_bytes) != hipSuccess) {
+        if (wg_dev_malloc(ctx, &C0, V * PPR_LANES * sizeof(float)) != hipSuccess ||
+            wg_dev_malloc(ctx, &C1, V * PPR_LANES * sizeof(float)) != hipSuccess ||
+            wg_dev_malloc(ctx, &R, V * PPR_LANES * sizeof(double)) != hipSuccess || wg_dev_malloc(ctx, &aux, aux_bytes) != hipSuccess) {
             (void)hipFree(C0);
             (void)hipFree(C1);
             (void)hipFree(R);

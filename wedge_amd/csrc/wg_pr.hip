@@ -381,7 +381,7 @@ extern "C" int wg_edge_pull_pr(wg_ctx* ctx, double* total_rank)
     if (!ctx || ctx->app != WG_APP_PR)
         return WG_E_STATE;
     if (!ctx->acc)
-        WG_HIP(ctx, hipMalloc((void**)&ctx->acc, ctx->V * sizeof(double)));
+        WG_HIP(ctx, wg_dev_malloc(ctx, (void**)&ctx->acc, ctx->V * sizeof(double)));
     int rc = ctx->pr_fp32 ? pr_launch<float>(ctx, 1) : pr_launch<double>(ctx, 1);
     if (rc)
         return rc;

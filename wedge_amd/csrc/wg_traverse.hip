@@ -2722,13 +2722,12 @@ static void* optional_array(size_t bytes)
 // them the pulls take every iteration.
 static int build_solo_sssp(wg_ctx* ctx)
 {
-    double *sum = nullptr, total = 0.0;
-    WG_HIP(ctx, hipMalloc((void**)&sum, sizeof(double)));
-    if (!ctx->solo_far)
-        ctx->solo_far = (uint32_t*)optional_array(2ull * SOLO_FAR * sizeof(uint32_t));
+    double total = 0.0;
+    ctx->solo_far = (uint32_t*)optional_array(2ull * SOLO_FAR * sizeof(uint32_t));
     uint4* rec = ctx->solo_far ? (uint4*)optional_array(ctx->V * 4 * sizeof(uint4)) : nullptr;
+    double* sum = rec ? (double*)optional_array(sizeof(double)) : nullptr;
     hipError_t e = hipSuccess;
-    if (rec) {
+    if (sum) {
         const dim3 gv(wg_grid(ctx, ctx->V, 256, 8)), ge(wg_grid(ctx, ctx->E, 4096, 4)), blk(WG_BLOCK);
         const uint64_t one = 0;
         (void)hipMemcpyAsync(sum, &one, sizeof(double), hipMemcpyHostToDevice, ctx->stream);
@@ -2747,15 +2746,20 @@ static int build_solo_sssp(wg_ctx* ctx)
         const hipError_t e2 = hipStreamSynchronize(ctx->stream);
         e = e == hipSuccess ? e2 : e;
     }
+    if (!sum || e != hipSuccess) {
+        (void)hipFree(rec);
+        (void)hipFree(ctx->solo_far);
+        ctx->solo_far = nullptr;
+        ctx->solo_none |= 1u << WG_APP_SSSP;
+    }
     (void)hipFree(sum);
     if (e != hipSuccess) {
-        (void)hipFree(rec);
         ctx->last_hip_error = (int)e;
         return WG_E_HIP;
     }
-    ctx->solo_wrec = rec;
-    if (!rec)
+    if (!sum)
         return WG_OK;
+    ctx->solo_wrec = rec;
     const double mean = total / (double)ctx->E;
     ctx->solo_delta = mean > 0.0 && mean < 1e300 ? 4.0 * mean : 1.0;
     return WG_OK;
@@ -2868,7 +2872,7 @@ static int init_common(wg_ctx* ctx, int app, size_t esz, int kind, uint64_t valu
         return rc;
     // the smallest in-neighbours the dense BFS levels test first (once per graph)
     if (app == WG_APP_BFS && !ctx->first_src) {
-        WG_HIP(ctx, hipMalloc((void**)&ctx->first_src, (ctx->V ? ctx->V : 1) * sizeof(uint32_t)));
+        WG_HIP(ctx, wg_dev_malloc(ctx, (void**)&ctx->first_src, (ctx->V ? ctx->V : 1) * sizeof(uint32_t)));
         hipLaunchKernelGGL(k_first_src, dim3(wg_grid(ctx, ctx->V, 256, 8)), dim3(256), 0, ctx->stream, ctx->off, ctx->src,
                            ctx->V, ctx->first_src);
         if ((rc = wg_check_launch(ctx)))
@@ -2877,22 +2881,25 @@ static int init_common(wg_ctx* ctx, int app, size_t esz, int kind, uint64_t valu
     // the out-edges' destinations in out-edge order, for the first level's
     // push and the fused levels (once per graph)
     if (app == WG_APP_BFS && !ctx->csr_dst) {
-        WG_HIP(ctx, hipMalloc((void**)&ctx->csr_dst, (ctx->E ? ctx->E : 1) * sizeof(uint32_t)));
+        WG_HIP(ctx, wg_dev_malloc(ctx, (void**)&ctx->csr_dst, (ctx->E ? ctx->E : 1) * sizeof(uint32_t)));
         if (ctx->E)
             hipLaunchKernelGGL(k_csr_dst, dim3(wg_grid(ctx, ctx->E, 1024, 8)), dim3(256), 0, ctx->stream, ctx->csri_pos,
                                ctx->dst, ctx->E, ctx->csr_dst);
         if ((rc = wg_check_launch(ctx)))
             return rc;
     }
-    if (app == WG_APP_SSSP && !ctx->solo_wrec && !wg_pb_min_on(ctx) && ctx->E &&
+    if (app == WG_APP_SSSP && !ctx->solo_wrec && !((ctx->solo_none >> app) & 1u) && !wg_pb_min_on(ctx) && ctx->E &&
         ctx->E <= ctx->V * SOLO_MEAN_DEGREE && (rc = build_solo_sssp(ctx)))
         return rc;
     // vertex records for the levels of one workgroup, on graphs with few
     // out-edges per vertex (once per graph; 32 bytes per vertex; without room
     // for them those levels take the other kernels)
-    if (app == WG_APP_BFS && !ctx->solo_rec && ctx->E <= ctx->V * SOLO_MEAN_DEGREE) {
+    if (app == WG_APP_BFS && !ctx->solo_rec && !((ctx->solo_none >> app) & 1u) &&
+        ctx->E <= ctx->V * SOLO_MEAN_DEGREE) {
         ctx->solo_rec = (uint4*)optional_array(ctx->V * 2 * sizeof(uint4));
-        if (ctx->solo_rec)
+        if (!ctx->solo_rec)
+            ctx->solo_none |= 1u << WG_APP_BFS;
+        else
             hipLaunchKernelGGL(k_solo_rec, dim3(wg_grid(ctx, ctx->V, 256, 8)), dim3(256), 0, ctx->stream, ctx->csri_off,
                                ctx->csr_dst, ctx->V, ctx->solo_rec);
         if ((rc = wg_check_launch(ctx)))
@@ -2912,8 +2919,8 @@ static int root_arrays(wg_ctx* ctx, uint32_t n)
     ctx->roots = ctx->root_off = nullptr;
     ctx->roots_cap = 0;
     const uint64_t cap = n < 64u ? 64u : n;
-    WG_HIP(ctx, hipMalloc((void**)&ctx->roots, cap * sizeof(uint32_t)));
-    WG_HIP(ctx, hipMalloc((void**)&ctx->root_off, (cap + 1) * sizeof(uint32_t)));
+    WG_HIP(ctx, wg_dev_malloc(ctx, (void**)&ctx->roots, cap * sizeof(uint32_t)));
+    WG_HIP(ctx, wg_dev_malloc(ctx, (void**)&ctx->root_off, (cap + 1) * sizeof(uint32_t)));
     ctx->roots_cap = (uint32_t)cap;
     return WG_OK;
 }
@@ -2941,6 +2948,34 @@ __global__ void k_init_roots(const uint32_t* __restrict__ roots, uint32_t n, int
     }
 }
 
+// The state of a traversal from n roots: the caller's id of the only one, or their
+// device ids, distinct.
+static int start_roots(wg_ctx* ctx, int app, uint64_t root, const std::vector<uint32_t>& dev, uint32_t n)
+{
+    const size_t esz = (app == WG_APP_BFS || ctx->wkind == WG_WEIGHT_F64) ? 8 : 4;
+    int rc;
+    if ((rc = init_common(ctx, app, esz, esz == 8 ? INIT_U64 : INIT_U32,
+                          app == WG_APP_BFS ? ~0ull : esz == 8 ? (uint64_t)PolSF::INF : (uint64_t)PolSU::INF)) ||
+        (rc = root_arrays(ctx, n)))
+        return rc;
+    ctx->nroots = n;
+    ctx->roots_frontier = app == WG_APP_BFS;
+    if (dev.empty()) {
+        hipLaunchKernelGGL(k_init_root, dim3(1), dim3(WG_WAVE), 0, ctx->stream, root, ctx->inv, app, ctx->wkind,
+                           ctx->prop[0], ctx->bm_cur, ctx->bm_visited, ctx->csri_off, ctx->roots, ctx->root_off);
+        return wg_check_launch(ctx);
+    }
+    WG_HIP(ctx, hipMemcpyAsync(ctx->roots, dev.data(), n * sizeof(uint32_t), hipMemcpyHostToDevice, ctx->stream));
+    hipLaunchKernelGGL(k_init_roots, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, ctx->roots, n, app, ctx->wkind,
+                       ctx->prop[0], ctx->perm, ctx->bm_cur, ctx->bm_visited);
+    hipLaunchKernelGGL(k_root_offsets, dim3(1), dim3(WG_BLOCK), 0, ctx->stream, ctx->roots, n, ctx->csri_off,
+                       ctx->root_off);
+    if ((rc = wg_check_launch(ctx)))
+        return rc;
+    WG_HIP(ctx, hipStreamSynchronize(ctx->stream)); // dev has been read
+    return WG_OK;
+}
+
 static int init_roots(wg_ctx* ctx, int app, const uint64_t* roots, uint32_t n)
 {
     if (!ctx || !roots || n == 0)
@@ -2959,27 +2994,10 @@ static int init_roots(wg_ctx* ctx, int app, const uint64_t* roots, uint32_t n)
         dev.erase(std::unique(dev.begin(), dev.end()), dev.end());
         n = (uint32_t)dev.size();
     }
-    const size_t esz = (app == WG_APP_BFS || ctx->wkind == WG_WEIGHT_F64) ? 8 : 4;
-    if ((rc = init_common(ctx, app, esz, esz == 8 ? INIT_U64 : INIT_U32,
-                          app == WG_APP_BFS ? ~0ull : esz == 8 ? (uint64_t)PolSF::INF : (uint64_t)PolSU::INF)) ||
-        (rc = root_arrays(ctx, n)))
-        return rc;
-    ctx->nroots = n;
-    ctx->roots_frontier = app == WG_APP_BFS;
-    if (dev.empty()) {
-        hipLaunchKernelGGL(k_init_root, dim3(1), dim3(WG_WAVE), 0, ctx->stream, roots[0], ctx->inv, app, ctx->wkind,
-                           ctx->prop[0], ctx->bm_cur, ctx->bm_visited, ctx->csri_off, ctx->roots, ctx->root_off);
-        return wg_check_launch(ctx);
-    }
-    WG_HIP(ctx, hipMemcpyAsync(ctx->roots, dev.data(), n * sizeof(uint32_t), hipMemcpyHostToDevice, ctx->stream));
-    hipLaunchKernelGGL(k_init_roots, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, ctx->roots, n, app, ctx->wkind,
-                       ctx->prop[0], ctx->perm, ctx->bm_cur, ctx->bm_visited);
-    hipLaunchKernelGGL(k_root_offsets, dim3(1), dim3(WG_BLOCK), 0, ctx->stream, ctx->roots, n, ctx->csri_off,
-                       ctx->root_off);
-    if ((rc = wg_check_launch(ctx)))
-        return rc;
-    WG_HIP(ctx, hipStreamSynchronize(ctx->stream)); // dev has been read
-    return WG_OK;
+    rc = start_roots(ctx, app, roots[0], dev, n);
+    if (rc) // a state without its roots serves no loop
+        wg_free_app_state(ctx);
+    return rc;
 }
 
 extern "C" int wg_init_bfs_roots(wg_ctx* ctx, const uint64_t* roots, uint32_t n)
@@ -2994,7 +3012,12 @@ extern "C" int wg_init_bfs(wg_ctx* ctx, uint64_t root)
 
 extern "C" int wg_init_cc(wg_ctx* ctx)
 {
-    return init_common(ctx, WG_APP_CC, sizeof(uint32_t), INIT_IDS, 0);
+    if (!ctx || !ctx->off)
+        return WG_E_STATE;
+    const int rc = init_common(ctx, WG_APP_CC, sizeof(uint32_t), INIT_IDS, 0);
+    if (rc)
+        wg_free_app_state(ctx);
+    return rc;
 }
 
 extern "C" int wg_init_sssp_roots(wg_ctx* ctx, const uint64_t* roots, uint32_t n)
@@ -3512,13 +3535,13 @@ extern "C" int wg_converge(wg_ctx* ctx, const wg_loop_params* p, uint64_t* itera
     if (wg_pb_min_on(ctx) && (rc = wg_pb_min_prepare(ctx))) // dense iterations on the binned layout
         return rc;
     if (ctx->run_wgs[ctx->app & 7]) {
-        if (!ctx->run_q) {
-            WG_HIP(ctx, hipMalloc((void**)&ctx->run_ctl, sizeof(wg_run_ctl)));
-            WG_HIP(ctx, hipMalloc((void**)&ctx->run_q, 2 * (size_t)WG_RUN_QCAP * sizeof(uint4)));
-        }
+        if (!ctx->run_ctl)
+            WG_HIP(ctx, wg_dev_malloc(ctx, (void**)&ctx->run_ctl, sizeof(wg_run_ctl)));
+        if (!ctx->run_q)
+            WG_HIP(ctx, wg_dev_malloc(ctx, (void**)&ctx->run_q, 2 * (size_t)WG_RUN_QCAP * sizeof(uint4)));
         if (ctx->app != WG_APP_BFS) {
             if (!ctx->run_spare)
-                WG_HIP(ctx, hipMalloc((void**)&ctx->run_spare, ctx->bm_words * sizeof(uint64_t)));
+                WG_HIP(ctx, wg_dev_malloc(ctx, (void**)&ctx->run_spare, ctx->bm_words * sizeof(uint64_t)));
             if ((rc = wg_clear_u64(ctx, ctx->run_spare, ctx->bm_words)))
                 return rc;
         }
