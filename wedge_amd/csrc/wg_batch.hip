@@ -20,6 +20,7 @@
 // built from the vertices with any new source (source/wedge.c:63-155).  The
 // schedule per level is the plain rule on the summed out-degree of those
 // vertices.  Each source's depths equal those of a single-source BFS.
+#include "wg_span.h"
 #include "wg_frontier.h"
 
 #include <algorithm>
@@ -680,11 +681,10 @@ __global__ __launch_bounds__(WG_BLOCK) void k_mss_touch_heavy(const uint32_t* __
     const uint32_t nwaves = gridDim.x * WG_WPB;
     for (uint32_t i = blockIdx.x * WG_WPB + threadIdx.x / WG_WAVE; i < n; i += nwaves) {
         const uint32_t u = heavy[2 * i], s = heavy[2 * i + 1];
-        const uint32_t end = csri_off[u + 1];
-        const uint32_t e = (s + WG_MSS_CHUNK < end) ? s + WG_MSS_CHUNK : end;
+        const uint32_t len = wg_step(s, csri_off[u + 1], WG_MSS_CHUNK);
 #pragma unroll 4
-        for (uint32_t p = s + (uint32_t)wg_lane(); p < e; p += WG_WAVE) {
-            const uint32_t v = dst[csri_pos[p]];
+        for (uint32_t k = (uint32_t)wg_lane(); k < len; k += WG_WAVE) {
+            const uint32_t v = dst[csri_pos[s + k]];
             const unsigned long long m = 1ull << (v & 63);
             if (!(touched[v >> 6] & m))
                 atomicOr(&touched[v >> 6], m);
@@ -780,10 +780,11 @@ __global__ __launch_bounds__(WG_BLOCK) void k_mss_relax(const uint32_t* __restri
         const uint32_t e0 = tile_e[ti], e1 = tile_e[ti + 1];
         uint32_t cur = 0xffffffffu; // destination being summed up (uniform), none yet
         T m = P::INF, old = P::INF;
-        for (uint32_t p = e0; p < e1; p += WG_WAVE) {
+        for (uint32_t p = e0, len; (len = wg_step(p, e1, WG_WAVE)) != 0u; p += len) {
             const uint32_t q = p + (uint32_t)lane;
-            const uint32_t u = q < e1 ? src[q] : 0u;
-            const bool a = q < e1 && test_bit64(active, u);
+            const bool in = (uint32_t)lane < len;
+            const uint32_t u = in ? src[q] : 0u;
+            const bool a = in && test_bit64(active, u);
             const uint32_t v = (a && !heavy) ? dst[q] : v0;
             unsigned long long left = wg_ballot(a);
             if (!left)

@@ -73,11 +73,12 @@ __device__ __forceinline__ void ppr_add(ppr_sum& a, ppr_f4 r)
         a.x[j] += (double)r[j];
 }
 
-// In-edges p, p + step, ... < e into a, in that order: this lane's four seeds.
-__device__ __forceinline__ void ppr_gather(uint32_t p, uint32_t e, uint32_t step, const uint32_t* __restrict__ src,
+// In-edges p, p + step, ... of the n from src on (n is a tile's edges at most, so
+// no sum here wraps) into a, in that order: this lane's four seeds.
+__device__ __forceinline__ void ppr_gather(uint32_t p, uint32_t n, uint32_t step, const uint32_t* __restrict__ src,
                                            const ppr_f4* __restrict__ C, uint32_t l, ppr_sum& a)
 {
-    for (; p + (PPR_FLIGHT - 1) * step < e; p += PPR_FLIGHT * step) {
+    for (; p + (PPR_FLIGHT - 1) * step < n; p += PPR_FLIGHT * step) {
         uint32_t u[PPR_FLIGHT];
         ppr_f4 r[PPR_FLIGHT];
 #pragma unroll
@@ -95,16 +96,16 @@ __device__ __forceinline__ void ppr_gather(uint32_t p, uint32_t e, uint32_t step
     ppr_f4 r[PPR_FLIGHT - 1];
 #pragma unroll
     for (int k = 0; k < PPR_FLIGHT - 1; ++k)
-        u[k] = p + k * step < e ? src[p + k * step] : 0u;
+        u[k] = p + k * step < n ? src[p + k * step] : 0u;
 #pragma unroll
     for (int k = 0; k < PPR_FLIGHT - 1; ++k) {
         r[k] = ppr_f4{0.0f, 0.0f, 0.0f, 0.0f};
-        if (p + k * step < e)
+        if (p + k * step < n)
             r[k] = C[(uint64_t)u[k] * (PPR_LANES / 4) + l];
     }
 #pragma unroll
     for (int k = 0; k < PPR_FLIGHT - 1; ++k)
-        if (p + k * step < e)
+        if (p + k * step < n)
             ppr_add(a, r[k]);
 }
 
@@ -177,7 +178,7 @@ __global__ __launch_bounds__(WG_BLOCK) void k_ppr_tile(const uint32_t* __restric
             if (sub)
                 continue;
             ppr_sum a = {};
-            ppr_gather(e0 + grp, e1, PPR_GROUPS, src, C, l, a);
+            ppr_gather(grp, e1 - e0, PPR_GROUPS, src + e0, C, l, a);
             ppr_join(a);
             if (grp == 0)
 #pragma unroll
@@ -190,7 +191,8 @@ __global__ __launch_bounds__(WG_BLOCK) void k_ppr_tile(const uint32_t* __restric
             const uint32_t v = v0 + i;
             ppr_sum a = {};
             const uint32_t o = od[v];
-            ppr_gather(off[v], off[v + 1], 1u, src, C, l, a);
+            const uint32_t b = off[v];
+            ppr_gather(0u, off[v + 1] - b, 1u, src + b, C, l, a);
             ppr_vertex(v, o, a, seed, dang, damping, l, Cn, R, dsum);
         }
     }
