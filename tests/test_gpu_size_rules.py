@@ -367,6 +367,44 @@ def test_sssp_after_capped_pulls(graph, cap):
             c.close()
 
 
+# up to 4096 roots have offsets for a push of their out-edges, more only a total
+@pytest.mark.parametrize("n", [2, 4095, 4096, 4097, 9001])
+def test_many_roots(n):
+    g = _sparse(20011, 70000, 12, weights="int")
+    roots = np.random.default_rng(n).choice(20011, n, replace=False).astype(np.uint64)
+    total = int(g.outdegrees()[roots.astype(np.int64)].sum())
+    dst = g.destinations()
+
+    def fixpoint(d, w):
+        while True:
+            new = d.copy()
+            np.minimum.at(new, dst, d[g.sources] + w)
+            if np.array_equal(new, d):
+                return d
+            d = new
+
+    start = np.full(g.num_vertices, np.inf)
+    start[roots.astype(np.int64)] = 0.0
+    c = W.Context(0)
+    try:
+        c.load(g)
+        for init, read, w in ((c.init_bfs_roots, lambda: W.bfs_depth(c.read_bfs()), 1.0),
+                              (c.init_sssp_roots, c.read_sssp, g.weights.astype(np.float64))):
+            want = fixpoint(start, w)
+            for schedule in (W.SCHED_PLAIN, W.SCHED_FRONTIER):
+                init(roots)
+                c.converge(schedule)
+                got = read()
+                assert np.array_equal(np.where(got == np.uint32(0xFFFFFFFF), np.inf, got.astype(np.float64)), want)
+            # the roots' out-degrees choose the first pull
+            pct = total * 100 // g.num_edges
+            for threshold, frontier in ((pct, g.num_edges * pct // 100 >= total), (pct + 1, True)):
+                init(roots)
+                assert c.converge(W.SCHED_PLAIN, threshold_pct=threshold, max_iterations=1) == (1, int(frontier))
+    finally:
+        c.close()
+
+
 # page-locked memory: at an allocation's start, inside one, ending with one, at
 # no multiple of the element size (copied), and over 32 MiB (copied); the
 # elements around the result keep their value

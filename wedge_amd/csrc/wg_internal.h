@@ -247,7 +247,8 @@ struct wg_ctx {
     wg_dev_counters* hctr_dev; // the mirror's device address (null if it has none)
     uint32_t* roots;          // BFS / SSSP roots in device numbering, distinct
     uint32_t* root_off;       // exclusive prefix of the roots' out-degrees (nroots + 1 entries): for the first
-                              // level's push, and the activity a traversal starts with
+                              // level's push, and the activity a traversal starts with; from more than
+                              // WG_PUSH_ROOTS_MAX roots only that activity, in [0]
     uint32_t nroots;
     uint32_t roots_cap;       // roots the two arrays have room for
     int roots_frontier;       // the BFS frontier is still the roots (no pull or advance since the init)

@@ -2920,22 +2920,35 @@ static int root_arrays(wg_ctx* ctx, uint32_t n)
     ctx->roots_cap = 0;
     const uint64_t cap = n < 64u ? 64u : n;
     WG_HIP(ctx, wg_dev_malloc(ctx, (void**)&ctx->roots, cap * sizeof(uint32_t)));
-    WG_HIP(ctx, wg_dev_malloc(ctx, (void**)&ctx->root_off, (cap + 1) * sizeof(uint32_t)));
+    const uint64_t noff = cap < WG_PUSH_ROOTS_MAX ? cap : WG_PUSH_ROOTS_MAX;
+    WG_HIP(ctx, wg_dev_malloc(ctx, (void**)&ctx->root_off, (noff + 1) * sizeof(uint32_t)));
     ctx->roots_cap = (uint32_t)cap;
     return WG_OK;
+}
+
+// Where the roots' total out-degree is: behind their offsets, if they have any.
+static uint32_t* root_total(const wg_ctx* ctx)
+{
+    return ctx->root_off + (ctx->nroots <= WG_PUSH_ROOTS_MAX ? ctx->nroots : 0u);
 }
 
 // Roots (device ids, distinct): BFS state depth 0 / parent = the root itself
 // (original id), SSSP distance 0; every root is set in bm_cur (BFS frontier;
 // for SSSP the set the first frontier build starts from) and, for BFS, in
-// bm_visited.
+// bm_visited.  total, if given (zero before), gets the roots' out-degrees.
 __global__ void k_init_roots(const uint32_t* __restrict__ roots, uint32_t n, int app, int wkind, void* __restrict__ prop,
-                             const uint32_t* __restrict__ perm, uint64_t* __restrict__ cur, uint64_t* __restrict__ visited)
+                             const uint32_t* __restrict__ perm, uint64_t* __restrict__ cur, uint64_t* __restrict__ visited,
+                             const uint32_t* __restrict__ od, uint32_t* __restrict__ total)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t r = i < n ? roots[i] : 0u;
+    if (total) {
+        const uint32_t d = wg_wave_sum(i < n ? od[r] : 0u);
+        if (wg_lane() == 0 && d)
+            atomicAdd(total, d);
+    }
     if (i >= n)
         return;
-    const uint32_t r = roots[i];
     const unsigned long long bit = 1ull << (r & 63);
     atomicOr((unsigned long long*)&cur[r >> 6], bit);
     if (app == WG_APP_BFS) {
@@ -2966,10 +2979,18 @@ static int start_roots(wg_ctx* ctx, int app, uint64_t root, const std::vector<ui
         return wg_check_launch(ctx);
     }
     WG_HIP(ctx, hipMemcpyAsync(ctx->roots, dev.data(), n * sizeof(uint32_t), hipMemcpyHostToDevice, ctx->stream));
+    // The offsets are for a push of the first level (at most WG_PUSH_ROOTS_MAX
+    // roots); from more roots only their total is used, and one workgroup adding up
+    // 2 million of them takes 14 ms.
+    const bool offsets = n <= WG_PUSH_ROOTS_MAX;
+    if (!offsets)
+        WG_HIP(ctx, hipMemsetAsync(root_total(ctx), 0, sizeof(uint32_t), ctx->stream));
     hipLaunchKernelGGL(k_init_roots, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, ctx->roots, n, app, ctx->wkind,
-                       ctx->prop[0], ctx->perm, ctx->bm_cur, ctx->bm_visited);
-    hipLaunchKernelGGL(k_root_offsets, dim3(1), dim3(WG_BLOCK), 0, ctx->stream, ctx->roots, n, ctx->csri_off,
-                       ctx->root_off);
+                       ctx->prop[0], ctx->perm, ctx->bm_cur, ctx->bm_visited, ctx->od,
+                       offsets ? (uint32_t*)nullptr : root_total(ctx));
+    if (offsets)
+        hipLaunchKernelGGL(k_root_offsets, dim3(1), dim3(WG_BLOCK), 0, ctx->stream, ctx->roots, n, ctx->csri_off,
+                           ctx->root_off);
     if ((rc = wg_check_launch(ctx)))
         return rc;
     WG_HIP(ctx, hipStreamSynchronize(ctx->stream)); // dev has been read
@@ -3551,7 +3572,7 @@ extern "C" int wg_converge(wg_ctx* ctx, const wg_loop_params* p, uint64_t* itera
     const unsigned long long act0 = ctx->app == WG_APP_CC ? ctx->E : 0ull;
     hipLaunchKernelGGL(k_loop_init, dim3(1), dim3(WG_WAVE), 0, ctx->stream, ctx->ctr, ctx->mlp_set ? ctx->mlp : nullptr,
                        (unsigned int)p->schedule, threshold, blog2, p->max_iterations, act0,
-                       ctx->app == WG_APP_CC ? nullptr : ctx->root_off + ctx->nroots,
+                       ctx->app == WG_APP_CC ? nullptr : root_total(ctx),
                        ctx->run_wgs[ctx->app & 7] ? ctx->run_ctl : nullptr,
                        ctx->app == WG_APP_CC ? (unsigned long long)ctx->V : (unsigned long long)ctx->nroots,
                        ctx->app == WG_APP_CC ? 1 : 0,
