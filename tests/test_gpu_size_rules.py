@@ -1,11 +1,14 @@
 """The branches that a graph's size selects, each at a size that takes it:
-pull bins of 4K, 8K and 16K vertices of the binned layout, the 128- and
-512-edge tiles of the 64-source SSSP with and without marked destinations
-(hub lists cut into chunks), and one to eight wavefronts per tile of the
-personalised PageRank, BFS levels and SSSP rounds in one workgroup, and results
-stored to page-locked memory by the kernel or copied.  Against the oracle: exact for BFS, CC and SSSP, 1e-10
-L1 for FP64 PageRank (sums of FP64 values in another order), 2e-7 L1 for
-FP32-stored contributions (one rounding of 6e-8 per contribution)."""
+pull bins of 4K, 8K and 16K vertices of the binned layout, the 128-edge tiles of
+the 64-source SSSP with and without marked destinations (hub lists cut into
+chunks; the 512-edge tiles of larger graphs are tests/test_gpu_configs.py's 64
+sources on rmat-s24), one to eight wavefronts per tile of the personalised
+PageRank, BFS levels and SSSP rounds in one workgroup (long out-lists cut into
+chunks, levels handed back and forth, the pulls of a capped SSSP), traversals
+from few and many roots, and results stored to page-locked memory by the kernel
+or copied.  Against the oracle: exact for BFS, CC and SSSP, 1e-10 L1 for FP64
+PageRank (sums of FP64 values in another order), 2e-7 L1 for FP32-stored
+contributions (one rounding of 6e-8 per contribution)."""
 from __future__ import annotations
 
 import numpy as np

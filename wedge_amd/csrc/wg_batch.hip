@@ -634,9 +634,12 @@ __global__ void k_mss_roots(const uint32_t* __restrict__ roots, uint32_t n, type
 // Lanes take vertices with few out-edges; longer lists are left to
 // k_mss_touch_heavy as chunks of WG_MSS_CHUNK out-edges, so that a hub's list
 // is spread over many wavefronts (one wavefront walking it alone took 420 us
-// of a 1.0 ms round on rmat-s18).  At most E/32 + E/WG_MSS_CHUNK chunks are
-// listed, which heavy_list holds; heavy_cap bounds the writes regardless.
+// of a 1.0 ms round on rmat-s18).  A listed vertex has at least 33 out-edges and
+// ceil(d / 1024) <= d / 33 chunks, so at most E / 33 chunks are listed; heavy_list
+// holds more than E / 32.  The bound matters (a chunk that is not listed leaves
+// destinations unmarked); the comparison with heavy_cap only keeps the writes inside.
 #define WG_MSS_CHUNK 1024u
+static_assert(WG_MSS_CHUNK > WG_WEDGE_LANE_MAX && WG_WEDGE_LANE_MAX >= 32u, "the bound on the listed chunks");
 __global__ __launch_bounds__(WG_BLOCK) void k_mss_touch(const uint64_t* __restrict__ active, uint64_t nwords,
                                                          const uint32_t* __restrict__ csri_off,
                                                          const uint32_t* __restrict__ csri_pos,

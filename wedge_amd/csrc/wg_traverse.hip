@@ -1198,7 +1198,15 @@ __global__ __launch_bounds__(WG_BLOCK) void k_level_advance(uint64_t* __restrict
 // 85 ms against 13.1 without a hand-back and 13.1 this way).
 #define SOLO_AFTER 8u
 #define SOLO_PAYS 64u
-#define SOLO_MEAN_DEGREE 4u // records and such levels up to this many out-edges per vertex
+// Records and such levels up to this many out-edges per vertex: road networks have
+// 2 to 3.  Other graphs of so few gain less (init and converge, ms, without and with
+// these levels and rounds; SSSP plain schedule, learned, BFS plain; R-MAT scale 18 x 3:
+// 6.6 / 5.6, 1.08 / 0.93, - ; scale 22 x 4: 5.5 / 5.1, 2.9 / 2.9, 0.96 / 0.80; uniformly
+// random, 2M x 4: 7.3 / 7.0, 2.6 / 2.1, 3.3 / 3.3).  Slower by 2-5 %: levels of one
+// hub and of its thousands of neighbours in turn, under the learned schedule (29.9
+// against 28.9 ms), where the decision's larger workgroup starts for nothing.  The
+// first BFS of a graph pays 0.1 to 0.3 ms for the records' allocation.
+#define SOLO_MEAN_DEGREE 4u
 #define SOLO_REC 7u        // destinations in a vertex's record
 #define SOLO_LANE_EDGES 4u   // out-edges of a long list that a lane has in flight
 #define SOLO_CHUNK (SOLO_LANE_EDGES * WG_WAVE)
@@ -2170,7 +2178,8 @@ __global__ __launch_bounds__(SOLO_T) void k_decide_bfs(wg_dev_counters* __restri
 // list (global) the others; a round relaxes the near queue's out-edges, and when
 // no near vertex is left the cutoff moves past the nearest far one.  A vertex
 // whose distance falls is put on one of the two every time, so the fixpoint is
-// that of the pulls.  The step between cutoffs follows the size of the rounds
+// that of the pulls (the near-far method of Davidson, Baxter, Garland and Owens,
+// IPDPS 2014, with both queues in one workgroup).  The step between cutoffs follows the size of the rounds
 // (about a vertex per thread: wide enough to fill the workgroup, no wider, since
 // vertices relaxed too early are relaxed again).  SOLO_PENDING waiting vertices
 // are work for the whole device: the loop's pulls go on from there.
